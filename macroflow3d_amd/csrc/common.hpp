@@ -107,10 +107,6 @@ __host__ __device__ inline long neighbour_coef(int nx, int ny, int nz, const BcT
     return n;
 }
 
-__host__ __device__ inline bool interior_cell(int nx, int ny, int nz, int i, int j, int k) {
-    return i > 0 && i < nx - 1 && j > 0 && j < ny - 1 && k > 0 && k < nz - 1;
-}
-
 // ---------------------------------------------------------------------------
 // Device-resident iteration state of the Krylov solvers. Scalars never leave
 // the device inside the iteration; the host reads this struct only at its

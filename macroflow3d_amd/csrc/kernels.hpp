@@ -8,11 +8,9 @@ namespace kern {
 
 // ---- stencil (stencil.hip) -------------------------------------------------
 int gsrb(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, double* x,
-         const double* b, const double* K, int iters, bool zero_init);
+         const double* b, const double* K, int iters);
 int residual(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, const double* x,
              const double* b, const double* K, double* r);
-int residual_restrict(hipStream_t s, const mf3d_grid& fine, const BcTypes& bc, bool pin,
-                      const double* x, const double* b, const double* K, double* b_coarse);
 // first-stage block count of the fused reductions: one partial per kReduceCells
 // consecutive cells (8 per thread of a 256-thread block)
 unsigned reduce_blocks(size_t n);

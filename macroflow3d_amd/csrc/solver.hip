@@ -1986,8 +1986,7 @@ int mf3d_gsrb_smooth_3d(mf3d_stream stream, const mf3d_grid* grid, double* x, co
     MF3D_CHECK_LEN(n, cells(*grid), "x/b/K");
     if (num_iters < 0) return fail(MF3D_ERR_INVALID_ARGUMENT, "num_iters < 0");
     clear_stale_error();
-    return kern::gsrb(as_stream(stream), *grid, bc_types(*bc), pin != 0, x, b, K, num_iters,
-                      false);
+    return kern::gsrb(as_stream(stream), *grid, bc_types(*bc), pin != 0, x, b, K, num_iters);
 }
 
 int mf3d_compute_residual_3d(mf3d_stream stream, const mf3d_grid* grid, const double* x,

@@ -7,6 +7,9 @@
 // These kernels serve every level and every boundary mix of the
 // reference-semantics entry points (mf3d_gsrb_smooth_3d, ...).
 
+#include <algorithm>
+
+#include "hface.hpp"
 #include "kernels.hpp"
 
 namespace mf3d {
@@ -18,240 +21,192 @@ inline unsigned grid_for(size_t n, int block = kBlock) {
     return (unsigned)((n + block - 1) / block);
 }
 
-// GSRB value of one cell: (sum K_f x_nb - b dx^2) / sum K_f.
-// Interior: gsrb_interior_kernel (src/multigrid/smoothers/gsrb_3d.cu:29-73).
-// Boundary: gsrb_{face,edge,vertex}_kernel (gsrb_3d.cu:76-366), pin doubles
-// the diagonal of cell 0 (gsrb_3d.cu:360-362).
-template <bool ZERO>
-__device__ inline double gsrb_value(int nx, int ny, int nz, const BcTypes& bc, bool pin,
-                                    const double* __restrict__ x, const double* __restrict__ b,
-                                    const double* __restrict__ K, int i, int j, int k, long idx,
-                                    double dx2) {
-    const double KC = K[idx];
-    if (interior_cell(nx, ny, nz, i, j, k)) {
-        const long Nx = nx, st = (long)nx * ny;
-        const double iKC = 1.0 / KC;
-        const double K_xp = 2.0 / (iKC + 1.0 / K[idx + 1]);
-        const double K_xm = 2.0 / (iKC + 1.0 / K[idx - 1]);
-        const double K_yp = 2.0 / (iKC + 1.0 / K[idx + Nx]);
-        const double K_ym = 2.0 / (iKC + 1.0 / K[idx - Nx]);
-        const double K_zp = 2.0 / (iKC + 1.0 / K[idx + st]);
-        const double K_zm = 2.0 / (iKC + 1.0 / K[idx - st]);
-        double result = 0.0;
-        if (!ZERO) {
-            result = x[idx + 1] * K_xp;
-            result += x[idx - 1] * K_xm;
-            result += x[idx + Nx] * K_yp;
-            result += x[idx - Nx] * K_ym;
-            result += x[idx + st] * K_zp;
-            result += x[idx - st] * K_zm;
+// ---- smoother, residual and operator straight from K ---------------------------
+// Bound: at the sizes these entry points see (levels of a few million cells,
+// resident in the Infinity Cache) the instructions, not the bytes: a cell needs
+// seven reciprocals of K, six of face sums and, in the smoother, a division.
+// So a thread owns an x-adjacent cell pair (2m, 2m + 1) of one row and marches
+// up in z with x, K and 1/K of its pair at planes k - 1, k, k + 1 in registers:
+// a plane costs one pair load of each (the z+ neighbour, the next plane's own
+// values and the z- ones of the plane after), the two y rows and the values
+// either side of the pair. Boundaries are addressed without branches (a missing
+// neighbour reads an in-bounds stand-in and its face is selected), because
+// nearly every wave holds a boundary cell of some row and would run both sides
+// of a branch. Reciprocals are the hardware estimate and two Newton steps, with
+// the hardware's fix-up for 0 and infinity (a cell of K = 0 closes its faces).
+// 198 x 150 x 122 on MI355X, one thread per cell -> this: GSRB colour 49.6 ->
+// 24.8 us, residual 52.6 -> 26.0 us, operator 54.2 -> 25.4 us.
+
+// 1 / s
+__device__ __forceinline__ double recip(double s) {
+    return __builtin_amdgcn_div_fixup(rcp_nr(s), s, 1.0);
+}
+// n / s: the quotient of the refined reciprocal, corrected by its remainder
+__device__ __forceinline__ double quot(double n, double s) {
+    const double r = rcp_nr(s);
+    const double q = n * r;
+    return __builtin_amdgcn_div_fixup(fma(fma(-q, s, n), r, q), s, n);
+}
+// face between a cell (1/K = ia; K2 = 2 K) and a side whose cell has 1/K = ib:
+// the harmonic mean 2 / (1/K_a + 1/K_b), 2 K on a Dirichlet face, 0 without
+__device__ __forceinline__ double kface(const Side& s, double ia, double ib, double K2) {
+    return s.nb ? 2.0 * recip(ia + ib) : (s.face ? K2 : 0.0);
+}
+
+struct ColumnGeo {
+    int nx, ny, nz;
+    int np;     // pairs per row: ceil(nx / 2)
+    int tiles;  // workgroups per plane
+    int kz;     // planes per workgroup
+    long nblocks;
+};
+
+struct Pair {
+    double v[2];
+};
+// cells i, i + 1 of a row: one 16-byte load when VEC (nx even, 16-byte aligned
+// arrays), else two loads (the second cell may lie past an odd row: d = 0)
+template <bool VEC>
+__device__ __forceinline__ Pair ldpair(const double* __restrict__ p, long o, int d) {
+    typedef double __attribute__((ext_vector_type(2))) dbl2;
+    Pair r;
+    if (VEC) {
+        const dbl2 t = *reinterpret_cast<const dbl2*>(p + o);
+        r.v[0] = t.x, r.v[1] = t.y;
+    } else {
+        r.v[0] = p[o], r.v[1] = p[o + d];
+    }
+    return r;
+}
+
+// COL_GSRB: one colour of a GSRB iteration in place in x (gsrb_3d.cu:29-366:
+// (sum K_f x_nb - b dx^2) / sum K_f, the pin doubling the diagonal of cell 0).
+// Only the other colour's values and the thread's own cells are read, so the
+// order of the threads does not matter.
+// COL_RES: out = b - A x (residual_3d.cu:30-376; the pin adds the diagonal
+// times x_C at cell 0). COL_APPLY: out = A x (varcoeff_laplacian.cu:38-239; the
+// pin's diagonal counts in-domain neighbours only, :110-119, :232-234).
+enum { COL_GSRB = 0, COL_RES = 1, COL_APPLY = 2 };
+template <int KIND, bool VEC>
+__global__ void __launch_bounds__(kBlock)
+    column_kernel(ColumnGeo G, double dx2, double inv_dx2, BcTypes bc, int pin, const double* x,
+                  const double* b, const double* __restrict__ K, double* out, int colour) {
+    const long blk = xcd_block(G.nblocks);
+    if (blk < 0) return;
+    const int chunk = (int)(blk / G.tiles);
+    const long tp = (blk - (long)chunk * G.tiles) * kBlock + threadIdx.x;
+    if (tp >= (long)G.np * G.ny) return;
+    const int nx = G.nx, ny = G.ny, nz = G.nz;
+    const int j = (int)(tp / G.np);
+    const int i = 2 * (int)(tp - (long)j * G.np);
+    const bool two = i + 1 < nx;  // the pair's second cell exists
+    const int d1 = two ? 1 : 0;
+    const long sz = (long)nx * ny;
+    const int k0 = chunk * G.kz, k1 = min(nz, k0 + G.kz);
+    const Side N = side(j < ny - 1, nx, bc.t[3], -(long)(ny - 1) * nx);
+    const Side S = side(j > 0, -(long)nx, bc.t[2], (long)(ny - 1) * nx);
+    const Side W = side(i > 0, -1, bc.t[0], nx - 1);              // of cell i
+    const Side E = side(i + 2 < nx, 1, bc.t[1], -(long)(nx - 1)); // of the last cell, at i + d1
+    const Side In = side(true, 0, 0, 0);
+    long o = (long)k0 * sz + (long)j * nx + i;
+    const Side D0 = side(k0 > 0, -sz, bc.t[4], (long)(nz - 1) * sz);
+    Pair Kc = ldpair<VEC>(K, o, d1), xc = ldpair<VEC>(x, o, d1);
+    Pair Kd = ldpair<VEC>(K, o + D0.off, d1), xd = ldpair<VEC>(x, o + D0.off, d1);
+    Pair ic, id;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) ic.v[e] = recip(Kc.v[e]), id.v[e] = recip(Kd.v[e]);
+    for (int k = k0; k < k1; ++k, o += sz) {
+        const Side U = side(k < nz - 1, sz, bc.t[5], -(long)(nz - 1) * sz);
+        const Side D = k == k0 ? D0 : In;
+        const Pair Ku = ldpair<VEC>(K, o + U.off, d1), xu = ldpair<VEC>(x, o + U.off, d1);
+        Pair iu;
+        if (KIND == COL_GSRB) {
+            // the pair's cell of this colour: i + e, its x neighbours the pair's
+            // other cell and the one beyond the pair on its own side
+            const int e = (j + k + colour) & 1;
+            const long oe = o + (e ? d1 : 0);
+            const bool live = e == 0 || two;
+            const Side Xp = e ? E : side(two, 1, bc.t[1], -(long)(nx - 1));
+            const Side Xm = e ? In : W;
+            const double Kn = K[oe + N.off], Ks = K[oe + S.off];
+            const double xn = x[oe + N.off], xs = x[oe + S.off];
+            const long os = oe + (e ? E.off : W.off);  // beyond the pair
+            const double Ko = K[os], xo = x[os];
+            // (with an odd row's single last cell, x+ lies across the boundary)
+            const long op = oe + Xp.off;
+            const double Kp1 = two ? 0.0 : K[op], xp1 = two ? 0.0 : x[op];
+            const double bv = b[oe];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) iu.v[q] = recip(Ku.v[q]);
+            const double io = recip(Ko);
+            const double ixp = e ? io : (two ? ic.v[1] : recip(Kp1));
+            const double vxp = e ? xo : (two ? xc.v[1] : xp1);
+            const double ixm = e ? ic.v[0] : io, vxm = e ? xc.v[0] : xo;
+            const double me = e ? ic.v[1] : ic.v[0], K2 = 2.0 * (e ? Kc.v[1] : Kc.v[0]);
+            const double iue = e ? iu.v[1] : iu.v[0], xue = e ? xu.v[1] : xu.v[0];
+            const double ide = e ? id.v[1] : id.v[0], xde = e ? xd.v[1] : xd.v[0];
+            const double f[6] = {kface(Xp, me, ixp, K2), kface(Xm, me, ixm, K2),
+                                 kface(N, me, recip(Kn), K2), kface(S, me, recip(Ks), K2),
+                                 kface(U, me, iue, K2), kface(D, me, ide, K2)};
+            double r = Xp.nb ? vxp * f[0] : 0.0;
+            r += Xm.nb ? vxm * f[1] : 0.0;
+            r += N.nb ? xn * f[2] : 0.0;
+            r += S.nb ? xs * f[3] : 0.0;
+            r += U.nb ? xue * f[4] : 0.0;
+            r += D.nb ? xde * f[5] : 0.0;
+            double aC = f[0] + f[1] + f[2] + f[3] + f[4] + f[5];
+            if (pin && oe == 0) aC *= 2.0;
+            if (live) out[oe] = quot(r - bv * dx2, aC);
+        } else {
+            const Pair Kn = ldpair<VEC>(K, o + N.off, d1), xn = ldpair<VEC>(x, o + N.off, d1);
+            const Pair Ks = ldpair<VEC>(K, o + S.off, d1), xs = ldpair<VEC>(x, o + S.off, d1);
+            const double Kw = K[o + W.off], xw = x[o + W.off];
+            const double Ke = K[o + d1 + E.off], xe = x[o + d1 + E.off];
+            Pair bv{};
+            if (KIND == COL_RES) bv = ldpair<VEC>(b, o, d1);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) iu.v[q] = recip(Ku.v[q]);
+            const double iw = recip(Kw), ie = recip(Ke);
+            const double mid = 2.0 * recip(ic.v[0] + ic.v[1]);  // between the two cells
+            double res[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const double me = ic.v[e], K2 = 2.0 * Kc.v[e], xC = xc.v[e];
+                // an odd row's single last cell has its east side on the boundary
+                const bool inner = e == 0 && two;
+                const double fe = inner ? mid : kface(E, me, ie, K2);
+                const double fw = e == 1 ? mid : kface(W, me, iw, K2);
+                const double fn = kface(N, me, recip(Kn.v[e]), K2);
+                const double fs = kface(S, me, recip(Ks.v[e]), K2);
+                const double fu = kface(U, me, iu.v[e], K2);
+                const double fd = kface(D, me, id.v[e], K2);
+                const double ve = inner ? xc.v[1] : (E.nb ? xe : 0.0);
+                const double vw = e == 1 ? xc.v[0] : (W.nb ? xw : 0.0);
+                double r = fw * (xC - vw);
+                r += fe * (xC - ve);
+                r += fs * (xC - (S.nb ? xs.v[e] : 0.0));
+                r += fn * (xC - (N.nb ? xn.v[e] : 0.0));
+                r += fd * (xC - (D.nb ? xd.v[e] : 0.0));
+                r += fu * (xC - (U.nb ? xu.v[e] : 0.0));
+                if (pin && o + e == 0) {
+                    double aC = 0.0;  // the smoother's diagonal, or in-domain faces only
+                    if (KIND == COL_RES) aC = fw + fe + fs + fn + fd + fu;
+                    else aC = (nx > 1 ? fe : 0.0) + (ny > 1 ? fn : 0.0) + (nz > 1 ? fu : 0.0);
+                    r += aC * xC;
+                }
+                res[e] = KIND == COL_RES ? bv.v[e] + r * inv_dx2 : -r * inv_dx2;
+            }
+            if (VEC) {
+                typedef double __attribute__((ext_vector_type(2))) dbl2;
+                *reinterpret_cast<dbl2*>(out + o) = dbl2{res[0], res[1]};
+            } else {
+                out[o] = res[0];
+                if (two) out[o + 1] = res[1];
+            }
         }
-        const double aC = K_xp + K_xm + K_yp + K_ym + K_zp + K_zm;
-        return (result - b[idx] * dx2) / aC;
-    }
-    double c[6], v[6];
-#pragma unroll
-    for (int d = 0; d < 6; ++d) {
-        const long n = neighbour_coef(nx, ny, nz, bc, K, i, j, k, d, KC, c[d]);
-        v[d] = (ZERO || n < 0) ? 0.0 : x[n];
-    }
-    const double result =
-        c[0] * v[0] + c[1] * v[1] + c[2] * v[2] + c[3] * v[3] + c[4] * v[4] + c[5] * v[5];
-    double aC = c[0] + c[1] + c[2] + c[3] + c[4] + c[5];
-    if (pin && idx == 0) aC *= 2.0;
-    return (result - b[idx] * dx2) / aC;
-}
-
-// One colour of one GSRB iteration. Thread t covers the pair of cells
-// (2*ii, 2*ii+1) of row (j,k) and updates the one of colour `colour`
-// ((i+j+k) even = red = 0). ZERO: x is taken as zero on entry, the partner
-// (other colour) cell is written 0 -- a fill(0) fused into the first sweep.
-template <bool ZERO>
-__global__ void __launch_bounds__(kBlock)
-    gsrb_colour_kernel(int nx, int ny, int nz, double dx2, BcTypes bc, int pin,
-                       double* __restrict__ x, const double* __restrict__ b,
-                       const double* __restrict__ K, int colour) {
-    const int nxh = (nx + 1) >> 1;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long total = (long)nxh * ny * nz;
-    if (t >= total) return;
-    const int ii = (int)(t % nxh);
-    const long row = t / nxh;
-    const int j = (int)(row % ny);
-    const int k = (int)(row / ny);
-    const int par = (j + k + colour) & 1;
-    const int i = 2 * ii + par;
-    const long rowbase = (long)nx * row;
-    if (ZERO) {
-        const int ip = 2 * ii + (par ^ 1);
-        if (ip < nx) x[rowbase + ip] = 0.0;
-    }
-    if (i >= nx) return;
-    const long idx = rowbase + i;
-    x[idx] = gsrb_value<ZERO>(nx, ny, nz, bc, pin != 0, x, b, K, i, j, k, idx, dx2);
-}
-
-// Residual value r = b - A x of one cell.
-// Interior: residual_interior_kernel (src/multigrid/smoothers/residual_3d.cu:30-80).
-// Boundary: residual_{face,edge,vertex}_kernel (residual_3d.cu:83-376), pin at
-// cell 0 adds aC*x_C (residual_3d.cu:365-368).
-__device__ inline double residual_value(int nx, int ny, int nz, const BcTypes& bc, bool pin,
-                                        const double* __restrict__ x,
-                                        const double* __restrict__ b,
-                                        const double* __restrict__ K, int i, int j, int k,
-                                        long o, double dx2, double inv_dx2) {
-    const double xc = x[o], Kc = K[o];
-    if (interior_cell(nx, ny, nz, i, j, k)) {
-        const long Nx = nx, st = (long)nx * ny;
-        const double iKc = 1.0 / Kc;
-        double Ax = 0.0;
-        Ax -= 2.0 * (xc - x[o + 1]) / (iKc + 1.0 / K[o + 1]);
-        Ax -= 2.0 * (xc - x[o + Nx]) / (iKc + 1.0 / K[o + Nx]);
-        Ax -= 2.0 * (xc - x[o - 1]) / (iKc + 1.0 / K[o - 1]);
-        Ax -= 2.0 * (xc - x[o - Nx]) / (iKc + 1.0 / K[o - Nx]);
-        Ax -= 2.0 * (xc - x[o + st]) / (iKc + 1.0 / K[o + st]);
-        Ax -= 2.0 * (xc - x[o - st]) / (iKc + 1.0 / K[o - st]);
-        return b[o] - Ax * inv_dx2;
-    }
-    double c[6], v[6];
-#pragma unroll
-    for (int d = 0; d < 6; ++d) {
-        const long n = neighbour_coef(nx, ny, nz, bc, K, i, j, k, d, Kc, c[d]);
-        v[d] = n < 0 ? (bc.t[d] == MF3D_BC_NEUMANN ? xc : 0.0) : x[n];
-    }
-    double result = c[0] * (xc - v[0]) + c[1] * (xc - v[1]) + c[2] * (xc - v[2]) +
-                    c[3] * (xc - v[3]) + c[4] * (xc - v[4]) + c[5] * (xc - v[5]);
-    if (pin && o == 0) result += (c[0] + c[1] + c[2] + c[3] + c[4] + c[5]) * xc;
-    return b[o] - (-result / dx2);
-}
-
-__global__ void __launch_bounds__(kBlock)
-    residual_kernel(int nx, int ny, int nz, double dx2, double inv_dx2, BcTypes bc, int pin,
-                    const double* __restrict__ x, const double* __restrict__ b,
-                    const double* __restrict__ K, double* __restrict__ r) {
-    const long o = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long n = (long)nx * ny * nz;
-    if (o >= n) return;
-    const int i = (int)(o % nx);
-    const long q = o / nx;
-    const int j = (int)(q % ny);
-    const int k = (int)(q / ny);
-    r[o] = residual_value(nx, ny, nz, bc, pin != 0, x, b, K, i, j, k, o, dx2, inv_dx2);
-}
-
-// Residual fused with restriction: one thread per coarse cell evaluates the
-// residual of its 8 children and averages them in the order of
-// restrict_kernel (src/multigrid/transfer/restrict_3d.cu:36-49); the fine
-// residual is never stored.
-__global__ void __launch_bounds__(kBlock)
-    residual_restrict_kernel(int nx, int ny, int nz, double dx2, double inv_dx2, BcTypes bc,
-                             int pin, const double* __restrict__ x,
-                             const double* __restrict__ b, const double* __restrict__ K,
-                             double* __restrict__ bc_out) {
-    const int NX = nx >> 1, NY = ny >> 1, NZ = nz >> 1;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)NX * NY * NZ) return;
-    const int I = (int)(t % NX);
-    const long q = t / NX;
-    const int J = (int)(q % NY);
-    const int Kc = (int)(q / NY);
-    const int i = 2 * I, j = 2 * J, k = 2 * Kc;
-    const long Nx = nx, st = (long)nx * ny;
-    const long in = i + Nx * j + st * k;
-    const bool p = pin != 0;
-    double result = 0.0;
-    result += residual_value(nx, ny, nz, bc, p, x, b, K, i, j, k, in, dx2, inv_dx2);
-    result += residual_value(nx, ny, nz, bc, p, x, b, K, i + 1, j, k, in + 1, dx2, inv_dx2);
-    result += residual_value(nx, ny, nz, bc, p, x, b, K, i, j + 1, k, in + Nx, dx2, inv_dx2);
-    result += residual_value(nx, ny, nz, bc, p, x, b, K, i + 1, j + 1, k, in + 1 + Nx, dx2,
-                             inv_dx2);
-    result += residual_value(nx, ny, nz, bc, p, x, b, K, i, j, k + 1, in + st, dx2, inv_dx2);
-    result += residual_value(nx, ny, nz, bc, p, x, b, K, i + 1, j, k + 1, in + 1 + st, dx2,
-                             inv_dx2);
-    result += residual_value(nx, ny, nz, bc, p, x, b, K, i, j + 1, k + 1, in + Nx + st, dx2,
-                             inv_dx2);
-    result += residual_value(nx, ny, nz, bc, p, x, b, K, i + 1, j + 1, k + 1,
-                             in + 1 + Nx + st, dx2, inv_dx2);
-    bc_out[t] = result / 8.0;
-}
-
-// Operator value y = A x of one cell, VarCoeffLaplacian::apply
-// (src/numerics/operators/varcoeff_laplacian.cu:38-239). The pin's diagonal
-// counts only in-domain neighbours (varcoeff_laplacian.cu:110-119, 232-234).
-__device__ inline double apply_value(int nx, int ny, int nz, const BcTypes& bc, bool pin,
-                                     const double* __restrict__ K,
-                                     const double* __restrict__ x, int i, int j, int k, long idx,
-                                     double inv_dx2) {
-    const double xC = x[idx], KC = K[idx];
-    const long Nx = nx, st = (long)nx * ny;
-    if (interior_cell(nx, ny, nz, i, j, k)) {
-        const double iKC = 1.0 / KC;
-        const double Kxm = 2.0 / (iKC + 1.0 / K[idx - 1]);
-        const double Kxp = 2.0 / (iKC + 1.0 / K[idx + 1]);
-        const double Kym = 2.0 / (iKC + 1.0 / K[idx - Nx]);
-        const double Kyp = 2.0 / (iKC + 1.0 / K[idx + Nx]);
-        const double Kzm = 2.0 / (iKC + 1.0 / K[idx - st]);
-        const double Kzp = 2.0 / (iKC + 1.0 / K[idx + st]);
-        const double Ax = Kxm * (xC - x[idx - 1]) + Kxp * (xC - x[idx + 1]) +
-                          Kym * (xC - x[idx - Nx]) + Kyp * (xC - x[idx + Nx]) +
-                          Kzm * (xC - x[idx - st]) + Kzp * (xC - x[idx + st]);
-        return -Ax * inv_dx2;
-    }
-    double Ax = 0.0, aC = 0.0;
-    const int pos[3] = {i, j, k};
-    const int lim[3] = {nx, ny, nz};
-    const long stride[3] = {1, Nx, st};
-#pragma unroll
-    for (int d = 0; d < 6; ++d) {
-        const int ax = d >> 1;
-        const bool plus = d & 1;
-        const bool inside = plus ? (pos[ax] < lim[ax] - 1) : (pos[ax] > 0);
-        if (inside) {
-            const long n = plus ? idx + stride[ax] : idx - stride[ax];
-            const double Kh = 2.0 / (1.0 / KC + 1.0 / K[n]);
-            Ax += Kh * (xC - x[n]);
-            aC += Kh;
-        } else if (bc.t[d] == MF3D_BC_PERIODIC) {
-            const long n = plus ? idx - (long)(lim[ax] - 1) * stride[ax]
-                                : idx + (long)(lim[ax] - 1) * stride[ax];
-            const double Kh = 2.0 / (1.0 / KC + 1.0 / K[n]);
-            Ax += Kh * (xC - x[n]);
-        } else if (bc.t[d] == MF3D_BC_DIRICHLET) {
-            Ax += 2.0 * KC * xC;
-        }
-    }
-    if (pin && idx == 0) Ax += aC * xC;
-    return -Ax * inv_dx2;
-}
-
-__device__ inline double block_sum(double v) {
-    __shared__ double part[kBlock / 64];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) part[w] = v;
-    __syncthreads();
-    if (w == 0) {
-        v = lane < kBlock / 64 ? part[lane] : 0.0;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    }
-    return v;
-}
-
-// y = A x
-__global__ void __launch_bounds__(kBlock)
-    apply_kernel(int nx, int ny, int nz, double inv_dx2, BcTypes bc, int pin,
-                 const double* __restrict__ K, const double* __restrict__ x,
-                 double* __restrict__ y) {
-    const long o = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long n = (long)nx * ny * nz;
-    if (o < n) {
-        const int i = (int)(o % nx);
-        const long q = o / nx;
-        const int j = (int)(q % ny);
-        const int k = (int)(q / ny);
-        y[o] = apply_value(nx, ny, nz, bc, pin != 0, K, x, i, j, k, o, inv_dx2);
+        // this plane's values become the z- ones, the loaded ones the own
+        Kd = Kc, xd = xc, id = ic;
+        Kc = Ku, xc = xu, ic = iu;
     }
 }
 
@@ -361,7 +316,7 @@ constexpr int kSmallMaxCells = kSmallBlock * kSmallPer;
 __global__ void __launch_bounds__(kSmallBlock)
     gsrb_small_kernel(int nx, int ny, int nz, double dx2, BcTypes bc, int pin,
                       double* __restrict__ x, const double* __restrict__ b,
-                      const double* __restrict__ K, int iters, int zero_init) {
+                      const double* __restrict__ K, int iters) {
     __shared__ double xs[kSmallMaxCells];
     __shared__ double iks[kSmallMaxCells];
     const int n = nx * ny * nz;
@@ -372,7 +327,7 @@ __global__ void __launch_bounds__(kSmallBlock)
         bl[m] = 0.0;
         Kl[m] = 1.0;
         if (o < n) {
-            xs[o] = zero_init ? 0.0 : x[o];
+            xs[o] = x[o];
             Kl[m] = K[o];
             iks[o] = 1.0 / Kl[m];
             bl[m] = b[o];
@@ -878,60 +833,61 @@ __global__ void __launch_bounds__(kFactorThreads)
 // ---------------------------------------------------------------------------
 namespace kern {
 
-int gsrb(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, double* x,
-         const double* b, const double* K, int iters, bool zero_init) {
-    if (iters <= 0) return zero_init ? fill(s, x, cells(g), 0.0) : MF3D_OK;
+namespace {
+// Planes per workgroup: long columns reuse the marched planes and short ones
+// fill the chip; up to 16 planes while 2048 workgroups (8 waves a SIMD pair)
+// remain.
+ColumnGeo column_geo(const mf3d_grid& g) {
+    ColumnGeo G;
+    G.nx = g.nx, G.ny = g.ny, G.nz = g.nz;
+    G.np = (g.nx + 1) / 2;
+    G.tiles = (int)(((long)G.np * g.ny + kBlock - 1) / kBlock);
+    G.kz = (int)std::max(1L, std::min(16L, (long)G.tiles * g.nz / 2048));
+    G.nblocks = (long)G.tiles * ((g.nz + G.kz - 1) / G.kz);
+    return G;
+}
+template <int KIND>
+int launch_column(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, const double* x,
+                  const double* b, const double* K, double* out, int colour) {
+    const ColumnGeo G = column_geo(g);
     const double dx2 = g.dx * g.dx;
-    const size_t n = cells(g);
-    if (n <= (size_t)kSmallMaxCells && iters > 1) {
-        gsrb_small_kernel<<<1, kSmallBlock, 0, s>>>(g.nx, g.ny, g.nz, dx2, bc, pin, x, b, K,
-                                                    iters, zero_init ? 1 : 0);
+    auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+    const unsigned nb = xcd_round((size_t)G.nblocks);
+    if (!(g.nx & 1) && al(x) && al(K) && al(out) && (KIND != COL_RES || al(b)))
+        column_kernel<KIND, true><<<nb, kBlock, 0, s>>>(G, dx2, 1.0 / dx2, bc, pin, x, b, K, out,
+                                                        colour);
+    else
+        column_kernel<KIND, false><<<nb, kBlock, 0, s>>>(G, dx2, 1.0 / dx2, bc, pin, x, b, K, out,
+                                                         colour);
+    MF3D_HIP_TRY(hipGetLastError());
+    return MF3D_OK;
+}
+}  // namespace
+
+int gsrb(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, double* x,
+         const double* b, const double* K, int iters) {
+    if (cells(g) <= (size_t)kSmallMaxCells && iters > 1) {
+        gsrb_small_kernel<<<1, kSmallBlock, 0, s>>>(g.nx, g.ny, g.nz, g.dx * g.dx, bc, pin, x, b,
+                                                    K, iters);
         MF3D_HIP_TRY(hipGetLastError());
         return MF3D_OK;
     }
-    const size_t half = (size_t)((g.nx + 1) / 2) * g.ny * g.nz;
-    const unsigned grid = grid_for(half);
-    for (int it = 0; it < iters; ++it) {
-        for (int colour = 0; colour < 2; ++colour) {
-            if (zero_init && it == 0 && colour == 0)
-                gsrb_colour_kernel<true><<<grid, kBlock, 0, s>>>(g.nx, g.ny, g.nz, dx2, bc, pin,
-                                                                 x, b, K, colour);
-            else
-                gsrb_colour_kernel<false><<<grid, kBlock, 0, s>>>(g.nx, g.ny, g.nz, dx2, bc, pin,
-                                                                  x, b, K, colour);
-        }
-    }
-    MF3D_HIP_TRY(hipGetLastError());
+    for (int it = 0; it < iters; ++it)
+        for (int colour = 0; colour < 2; ++colour)
+            MF3D_TRY(launch_column<COL_GSRB>(s, g, bc, pin, x, b, K, x, colour));
     return MF3D_OK;
 }
 
 int residual(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, const double* x,
              const double* b, const double* K, double* r) {
-    const size_t n = cells(g);
-    residual_kernel<<<grid_for(n), kBlock, 0, s>>>(g.nx, g.ny, g.nz, g.dx * g.dx,
-                                                   1.0 / (g.dx * g.dx), bc, pin, x, b, K, r);
-    MF3D_HIP_TRY(hipGetLastError());
-    return MF3D_OK;
-}
-
-int residual_restrict(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin,
-                      const double* x, const double* b, const double* K, double* b_coarse) {
-    const size_t nc = (size_t)(g.nx / 2) * (g.ny / 2) * (g.nz / 2);
-    residual_restrict_kernel<<<grid_for(nc), kBlock, 0, s>>>(
-        g.nx, g.ny, g.nz, g.dx * g.dx, 1.0 / (g.dx * g.dx), bc, pin, x, b, K, b_coarse);
-    MF3D_HIP_TRY(hipGetLastError());
-    return MF3D_OK;
+    return launch_column<COL_RES>(s, g, bc, pin, x, b, K, r, 0);
 }
 
 unsigned reduce_blocks(size_t n) { return (unsigned)((n + kReduceCells - 1) / kReduceCells); }
 
 int apply(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, const double* K,
           const double* x, double* y) {
-    const size_t n = cells(g);
-    apply_kernel<<<grid_for(n), kBlock, 0, s>>>(g.nx, g.ny, g.nz, 1.0 / (g.dx * g.dx), bc, pin, K,
-                                                x, y);
-    MF3D_HIP_TRY(hipGetLastError());
-    return MF3D_OK;
+    return launch_column<COL_APPLY>(s, g, bc, pin, x, nullptr, K, y, 0);
 }
 
 int restrict_avg(hipStream_t s, const mf3d_grid& coarse, const double* f, double* c) {
