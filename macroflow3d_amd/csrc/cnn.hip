@@ -28,6 +28,7 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -63,17 +64,31 @@ __device__ __forceinline__ bf16x8 load8(const __hip_bfloat16* p) {
 // data with the forward tap order in W). Epilogue, per output (v, c):
 //   s = acc + bias[c] (if bias) + R[v*Cs + c] (if R); s = relu(s) (if relu);
 //   s *= (M[v*Cs + c] > 0) (if M); stored to out (BF16 or FP32) for c < Cs.
-template <int CT, int VT, bool F32OUT>
-__global__ void __launch_bounds__(256)
-    conv_kernel(Geo g, int cin, int kpad, int cs, const __hip_bfloat16* __restrict__ X,
+// up: X holds the grid of half the size and a voxel reads its parent (the copy
+// to the 8 children is never stored).
+//
+// KS waves of a workgroup share one wave's output tile and split its k steps;
+// their accumulators meet in LDS, summed in wave order, and each of the KS waves
+// finishes some of the tile's CT x VT fragments. The deep layers are a chain of
+// 14-54 dependent k steps on few voxels: 8^3 voxels x 64 channels are 32 tiles,
+// so with KS = 1 the launch was 32 waves on 256 CUs and the latency of the chain
+// its whole time (8^3, 64 -> 64 channels: 33.8 us with KS = 1, 9.4 us with 16).
+template <int CT, int VT, bool F32OUT, int KS>
+__global__ void __launch_bounds__(KS > 4 ? KS * 64 : 256)
+    conv_kernel(Geo g, int cin, int kpad, int cs, int up, const __hip_bfloat16* __restrict__ X,
                 const __hip_bfloat16* __restrict__ W, const float* __restrict__ bias,
                 const __hip_bfloat16* __restrict__ R, const __hip_bfloat16* __restrict__ M,
                 int relu, int flip, void* __restrict__ out) {
-    const long nvox = g.n();
+    constexpr int WPB = KS > 4 ? KS : 4;  // waves per workgroup
+    // (voxel indices are 32-bit: a grid has at most 4e9 cells, and a 64-bit
+    // division is hundreds of instructions)
+    const unsigned nvox = (unsigned)g.n();
     const int lane = threadIdx.x & 63;
-    const long wave = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const long vbase = wave * (16L * VT);
-    if (vbase >= nvox) return;  // whole wave
+    const int wv = (int)(threadIdx.x >> 6);
+    const int part = wv % KS;  // this wave's share of the k steps
+    const unsigned tile = blockIdx.x * (WPB / KS) + wv / KS;
+    const unsigned vbase = tile * (16 * VT);
+    if (KS == 1 && vbase >= nvox) return;  // whole wave (KS > 1: the workgroup meets below)
     const int col = lane & 15;   // voxel within a tile / output channel row of A
     const int grp = lane >> 4;   // k group: k = 8 grp .. 8 grp + 7 of each 32-chunk
 
@@ -81,13 +96,13 @@ __global__ void __launch_bounds__(256)
     bool live[VT];
 #pragma unroll
     for (int t = 0; t < VT; ++t) {
-        const long v = vbase + 16 * t + col;
+        const unsigned v = vbase + 16 * t + col;
         live[t] = v < nvox;
-        const long vv = live[t] ? v : 0;
-        vi[t] = (int)(vv % g.nx);
-        const long q = vv / g.nx;
-        vj[t] = (int)(q % g.ny);
-        vk[t] = (int)(q / g.ny);
+        const unsigned vv = live[t] ? v : 0;
+        const unsigned q = vv / (unsigned)g.nx;
+        vi[t] = (int)(vv - q * g.nx);
+        vk[t] = (int)(q / (unsigned)g.ny);
+        vj[t] = (int)(q - vk[t] * (unsigned)g.ny);
     }
     f32x4 acc[VT][CT];
 #pragma unroll
@@ -96,44 +111,46 @@ __global__ void __launch_bounds__(256)
         for (int c = 0; c < CT; ++c) acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int K = 27 * cin;
+    const int sx = g.nx >> up, sy = g.ny >> up;  // the stored grid of X
     const bf16x8 zero8 = __builtin_bit_cast(bf16x8, uint4{0u, 0u, 0u, 0u});
     // the operands of one 32-wide k step: weight rows (A) and the tap's
-    // input channels at each voxel (B, zero outside the grid or past K)
+    // input channels at each voxel (B, zero outside the grid or past K). The
+    // addresses are chosen without branches (an outside voxel reads voxel 0 and
+    // is zeroed): a load under a per-lane branch would be waited for inside it
     auto load_step = [&](int k0, bf16x8 (&a)[CT], bf16x8 (&b)[VT]) {
         const int k = k0 + 8 * grp;
 #pragma unroll
         for (int c = 0; c < CT; ++c) a[c] = load8(W + (long)(c * 16 + col) * kpad + k);
-        if (k < K) {
-            int tap = k / cin;
-            const int c0 = k - tap * cin;
-            if (flip) tap = 26 - tap;
-            const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
+        const bool ok = k < K;
+        int tap = ok ? k / cin : 0;
+        const int c0 = ok ? k - tap * cin : 0;
+        if (flip) tap = 26 - tap;
+        const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
 #pragma unroll
-            for (int t = 0; t < VT; ++t) {
-                const int ii = vi[t] + dx, jj = vj[t] + dy, kk = vk[t] + dz;
-                const bool in = live[t] && ii >= 0 && ii < g.nx && jj >= 0 && jj < g.ny &&
-                                kk >= 0 && kk < g.nz;
-                b[t] = in ? load8(X + ((long)ii + (long)g.nx * (jj + (long)g.ny * kk)) * cin + c0)
-                          : zero8;
-            }
-        } else {
-#pragma unroll
-            for (int t = 0; t < VT; ++t) b[t] = zero8;
+        for (int t = 0; t < VT; ++t) {
+            const int ii = vi[t] + dx, jj = vj[t] + dy, kk = vk[t] + dz;
+            const bool in = ok && live[t] && (unsigned)ii < (unsigned)g.nx &&
+                            (unsigned)jj < (unsigned)g.ny && (unsigned)kk < (unsigned)g.nz;
+            const long o = in ? (long)(ii >> up) + (long)sx * ((jj >> up) + (long)sy * (kk >> up)) : 0;
+            const bf16x8 x = load8(X + o * cin + c0);
+            b[t] = in ? x : zero8;
         }
     };
     // the next step's operands are loaded before this step's products are
     // issued, so the load latency overlaps the MFMAs (same accumulation order)
+    const int steps = kpad / 32;
+    const int kb = 32 * (steps * part / KS), ke = 32 * (steps * (part + 1) / KS);
     bf16x8 a[CT], b[VT];
-    load_step(0, a, b);
-    for (int k0 = 0; k0 < kpad; k0 += 32) {
+    if (kb < ke) load_step(kb, a, b);
+    for (int k0 = kb; k0 < ke; k0 += 32) {
         bf16x8 an[CT], bn[VT];
-        if (k0 + 32 < kpad) load_step(k0 + 32, an, bn);
+        if (k0 + 32 < ke) load_step(k0 + 32, an, bn);
 #pragma unroll
         for (int t = 0; t < VT; ++t)
 #pragma unroll
             for (int c = 0; c < CT; ++c)
                 acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c], b[t], acc[t][c], 0, 0, 0);
-        if (k0 + 32 < kpad) {
+        if (k0 + 32 < ke) {
 #pragma unroll
             for (int c = 0; c < CT; ++c) a[c] = an[c];
 #pragma unroll
@@ -141,14 +158,30 @@ __global__ void __launch_bounds__(256)
         }
     }
     // acc[t][c][r] = out(channel c*16 + 4 grp + r, voxel vbase + 16 t + col)
+    __shared__ f32x4 red[KS > 1 ? WPB * VT * CT * 64 : 1];
+    if (KS > 1) {
+#pragma unroll
+        for (int t = 0; t < VT; ++t)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) red[((wv * VT + t) * CT + c) * 64 + lane] = acc[t][c];
+        __syncthreads();
+    }
 #pragma unroll
     for (int t = 0; t < VT; ++t) {
-        if (!live[t]) continue;
         const long v = vbase + 16 * t + col;
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
             const int ch0 = c * 16 + 4 * grp;
-            if (ch0 >= cs) continue;
+            if (KS > 1) {
+                if ((t * CT + c) % KS != part) continue;  // another wave's fragment (uniform)
+                const int w0 = wv - part;
+                f32x4 s = red[((w0 * VT + t) * CT + c) * 64 + lane];
+#pragma unroll
+                for (int w = 1; w < KS; ++w)
+                    s += red[(((w0 + w) * VT + t) * CT + c) * 64 + lane];
+                acc[t][c] = s;
+            }
+            if (!live[t] || ch0 >= cs) continue;
             float s[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -173,110 +206,235 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// ---- convolution, weight gradient ---------------------------------------------
-// dW[co][tap*Cin + ci] = sum_v dY[v][co] X[v + d(tap)][ci]; one wave per
-// (tap, voxel slice) accumulates all Cout x Cin of that tap (CT x IT tiles)
-// over its slice with the voxels as the MFMA K dimension; partial sums go to
-// P[slice][co][tap*Cin + ci] (FP32), reduced by wgrad_reduce_kernel.
-template <int CT, int IT>
-__global__ void __launch_bounds__(64)
-    wgrad_kernel(Geo g, int cin, int cout_ch, const __hip_bfloat16* __restrict__ dY,
-                 const __hip_bfloat16* __restrict__ X, int slices, float* __restrict__ P) {
-    const int tap = blockIdx.x % 27;
-    const int slice = blockIdx.x / 27;
-    const long nvox = g.n();
-    const long per = ((nvox + slices - 1) / slices + 31) / 32 * 32;
-    const long v0 = (long)slice * per;
-    const long v1 = v0 + per < nvox ? v0 + per : nvox;
-    const int lane = threadIdx.x;
-    const int col = lane & 15, grp = lane >> 4;
-    const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
-    f32x4 acc[CT][IT];
+// ---- weight and bias gradients -------------------------------------------------
+// dW[co][tap*Cin + ci] = sum_v dY[v][co] X[v + d(tap)][ci]: the voxels are the
+// MFMA's K dimension, so a lane wants 8 consecutive voxels of one channel. Gathering
+// them from the channels-last tensors cost 8 two-byte loads with their own address
+// and bounds checks per operand (32^3, 16 x 16 channels: 66.9 us). Instead one
+// launch copies every operand of every layer into a channel-first form with zero
+// borders (Planar): each lane's 8 voxels are then one 16-byte load at any tap, and
+// no bounds are checked. One more launch holds all layers' products (a wave per
+// layer, tap and slice of the voxels; the layers are small enough that only
+// together they fill the chip), and one sums the slices in order, straight into
+// the master layout. 128^3 training sample: 28 launches of 408 us became 3 of
+// 63 us (46.7 of them the products).
+
+// channel-first copy of an [N][ch] tensor: voxel (i, j, k) of channel c at
+// c * plane + lead + ((k + 1) (ny + 2) + j + 1) row + i, everything else zero.
+// row = ceil8(nx) + 8 leaves at least 8 zeros after a row, which also serve as
+// the next row's border at i = -1; lead covers the first row's.
+constexpr int kPlanarLead = 16;
+struct Planar {
+    int row;       // row stride
+    long slab;     // plane of one z: row (ny + 2)
+    long plane;    // one channel
+    int gpr;       // 8-voxel groups per row
+    long groups;   // over all rows of the grid
+    int ny;
+};
+Planar planar_of(const mf3d_grid& g) {
+    Planar P;
+    const int n8 = (g.nx + 7) / 8;
+    P.row = 8 * n8 + 8;
+    P.slab = (long)P.row * (g.ny + 2);
+    P.plane = P.slab * (g.nz + 2) + 2 * kPlanarLead;
+    P.gpr = n8;
+    P.groups = (long)n8 * g.ny * g.nz;
+    P.ny = g.ny;
+    return P;
+}
+
+struct PlanarCopy {
+    const __hip_bfloat16* src;
+    __hip_bfloat16* dst;
+    int ch, up;  // up: src is on the half-size grid (a voxel copies its parent)
+    Geo g;
+    Planar P;
+    int block0;   // first workgroup of this tensor
+    int vblocks;  // workgroups per 8 channels
+};
+constexpr int kMaxCopies = 14, kMaxWLayers = 7;
+struct PlanarCopies {
+    PlanarCopy c[kMaxCopies];
+    int n;
+};
+// a thread copies 8 channels of one voxel
+__global__ void __launch_bounds__(256) planar_kernel(PlanarCopies D) {
+    int e = 0;
+    while (e + 1 < D.n && D.c[e + 1].block0 <= (int)blockIdx.x) ++e;
+    const PlanarCopy& C = D.c[e];
+    const unsigned nv = (unsigned)C.g.n();
+    const int b = (int)blockIdx.x - C.block0, c8 = b / C.vblocks;
+    const unsigned v = (unsigned)(b - c8 * C.vblocks) * 256 + threadIdx.x;
+    if (v >= nv) return;
+    const unsigned q = v / (unsigned)C.g.nx;
+    const int i = (int)(v - q * C.g.nx);
+    const int k = (int)(q / (unsigned)C.g.ny), j = (int)(q - k * (unsigned)C.g.ny);
+    const int u = C.up;
+    const long sv = (long)(i >> u) + (long)(C.g.nx >> u) * ((j >> u) + (long)(C.g.ny >> u) * (k >> u));
+    const bf16x8 val = load8(C.src + sv * C.ch + 8 * c8);
+    __bf16* d = reinterpret_cast<__bf16*>(C.dst) + (long)8 * c8 * C.P.plane + kPlanarLead +
+                (long)(k + 1) * C.P.slab + (long)(j + 1) * C.P.row + i;
 #pragma unroll
-    for (int c = 0; c < CT; ++c)
+    for (int c = 0; c < 8; ++c) d[(long)c * C.P.plane] = val[c];
+}
+
+struct WLayer {
+    const __hip_bfloat16* dY;  // planar, 16 ct channels
+    const __hip_bfloat16* X;   // planar, 16 it channels
+    Planar P;
+    int ct, it;
+    int slices, steps;  // slices of `steps` 32-voxel steps each
+    int wave0;          // first wave of this layer in the launch
+    float* part;        // [slice][16 ct][27 * 16 it]
+    float* bpart;       // [slice][16 ct]
+    // reduction into the master layout
+    int cin, cout;
+    float* gw;
+    float* gb;
+    int elem0;  // first element of this layer in the reduction
+};
+struct WLayers {
+    WLayer l[kMaxWLayers];
+    int n, waves, elems;
+};
+
+template <int CT, int IT>
+__device__ __forceinline__ void wgrad_body(const WLayer& L, int tap, int slice) {
+    const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+    const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
+    const long shift = (long)dy * L.P.row + (long)dz * L.P.slab;
+    const bool bias = tap == 13;
+    const __bf16 one = (__bf16)1.0f;
+    const bf16x8 ones = {one, one, one, one, one, one, one, one};
+    const bf16x8 zero8 = __builtin_bit_cast(bf16x8, uint4{0u, 0u, 0u, 0u});
+    f32x4 acc[CT][IT], accb[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        accb[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < IT; ++i) acc[c][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (long vb = v0; vb < v1; vb += 32) {
-        // this lane's 8 voxels: vb + 8 grp + e
-        long nb[8];
-        bool okv[8], okn[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const long v = vb + 8 * grp + e;
-            okv[e] = v < v1;
-            const long vv = okv[e] ? v : v0;
-            const int i = (int)(vv % g.nx);
-            const long q = vv / g.nx;
-            const int j = (int)(q % g.ny), k = (int)(q / g.ny);
-            const int ii = i + dx, jj = j + dy, kk = k + dz;
-            okn[e] = okv[e] && ii >= 0 && ii < g.nx && jj >= 0 && jj < g.ny && kk >= 0 && kk < g.nz;
-            nb[e] = okn[e] ? (long)ii + (long)g.nx * (jj + (long)g.ny * kk) : 0;
-        }
-        bf16x8 a[CT], b[IT];
+    }
+    const __hip_bfloat16* A0 = L.dY + (long)col * L.P.plane + kPlanarLead;
+    const __hip_bfloat16* B0 = L.X + (long)col * L.P.plane + kPlanarLead + shift;
+    // this lane's 8 voxels of a step: group g0 + 4 st + grp of the grid's rows,
+    // its place carried from step to step (past the end: zeros)
+    int q = slice * L.steps * 4 + grp;
+    int x8 = q % L.P.gpr, j = q / L.P.gpr % L.P.ny;
+    long o = (long)(q / L.P.gpr / L.P.ny + 1) * L.P.slab + (long)(j + 1) * L.P.row + 8 * x8;
+    const int groups = (int)L.P.groups;
+    // The tap's shift along x is made in registers from an aligned load and the
+    // 4 bytes next to it: 16-byte loads at odd element offsets took 68 us
+    // for the launch instead of 51.
+    auto load = [&](bool mine, bf16x8 (&a)[CT], bf16x8 (&b)[IT]) {
+        const bool ok = mine && q < groups;
+        const long oo = ok ? o : L.P.slab + L.P.row;
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
-            alignas(16) __hip_bfloat16 tmp[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                tmp[e] = okv[e] ? dY[(vb + 8 * grp + e) * cout_ch + c * 16 + col] : f2bf(0.0f);
-            a[c] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(tmp));
+            a[c] = load8(A0 + (long)16 * c * L.P.plane + oo);
+            if (!ok) a[c] = zero8;
         }
 #pragma unroll
         for (int i = 0; i < IT; ++i) {
-            alignas(16) __hip_bfloat16 tmp[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) tmp[e] = okn[e] ? X[nb[e] * cin + i * 16 + col] : f2bf(0.0f);
-            b[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(tmp));
+            const __hip_bfloat16* p = B0 + (long)16 * i * L.P.plane + oo;
+            uint4 d = *reinterpret_cast<const uint4*>(p);
+            if (dx > 0) {  // uniform
+                const unsigned n = *reinterpret_cast<const unsigned*>(p + 8);
+                d = uint4{__builtin_amdgcn_alignbit(d.y, d.x, 16), __builtin_amdgcn_alignbit(d.z, d.y, 16),
+                          __builtin_amdgcn_alignbit(d.w, d.z, 16), __builtin_amdgcn_alignbit(n, d.w, 16)};
+            } else if (dx < 0) {
+                const unsigned n = *reinterpret_cast<const unsigned*>(p - 2);
+                d = uint4{__builtin_amdgcn_alignbit(d.x, n, 16), __builtin_amdgcn_alignbit(d.y, d.x, 16),
+                          __builtin_amdgcn_alignbit(d.z, d.y, 16), __builtin_amdgcn_alignbit(d.w, d.z, 16)};
+            }
+            b[i] = __builtin_bit_cast(bf16x8, d);
         }
+        q += 4, x8 += 4, o += 32;
+        while (x8 >= L.P.gpr) {  // rows end with 8 zeros; the next z skips the border rows
+            x8 -= L.P.gpr, o += 8;
+            if (++j == L.P.ny) j = 0, o += 2L * L.P.row;
+        }
+    };
+    // U steps' loads are issued together: the chain of steps is latency
+    constexpr int U = CT + IT <= 3 ? 4 : 1;
+    for (int st = 0; st < L.steps; st += U) {
+        bf16x8 a[U][CT], b[U][IT];
 #pragma unroll
-        for (int c = 0; c < CT; ++c)
+        for (int u = 0; u < U; ++u) load(st + u < L.steps, a[u], b[u]);
 #pragma unroll
-            for (int i = 0; i < IT; ++i)
-                acc[c][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c], b[i], acc[c][i], 0, 0, 0);
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+                if (bias)
+                    accb[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][c], ones, accb[c], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < IT; ++i)
+                    acc[c][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][c], b[u][i], acc[c][i],
+                                                                        0, 0, 0);
+            }
     }
     // acc[c][i][r] = dW(co = c*16 + 4 grp + r, ci = i*16 + col)
-    const long K = 27L * cin;
-    float* p = P + (long)slice * (CT * 16) * K;
+    const long K = 27L * 16 * IT;
+    float* p = L.part + (long)slice * (CT * 16) * K + (long)tap * (16 * IT) + col;
 #pragma unroll
     for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int i = 0; i < IT; ++i)
+        for (int r = 0; r < 4; ++r) {
+            const int co = c * 16 + 4 * grp + r;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int co = c * 16 + 4 * grp + r;
-                p[(long)co * K + (long)tap * cin + i * 16 + col] = acc[c][i][r];
-            }
+            for (int i = 0; i < IT; ++i) p[(long)co * K + i * 16] = acc[c][i][r];
+            if (bias && col == 0) L.bpart[slice * (CT * 16) + co] = accb[c][r];
+        }
 }
 
-// G[co][k] (FP32, [Cout][27 Cin] of the layer) = sum over slices of P
-__global__ void __launch_bounds__(256)
-    wgrad_reduce_kernel(const float* __restrict__ P, int slices, int cout, int cout_pad, long K,
-                        float* __restrict__ G) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (long)cout * K) return;
-    const long co = e / K, k = e - co * K;
-    float s = 0.0f;
-    for (int sl = 0; sl < slices; ++sl) s += P[((long)sl * cout_pad + co) * K + k];
-    G[e] = s;
-}
-
-// bias gradient db[c] = sum_v dY[v][c], one block per channel (deterministic)
-__global__ void __launch_bounds__(256)
-    bgrad_kernel(Geo g, int ch, int cout, const __hip_bfloat16* __restrict__ dY,
-                 float* __restrict__ db) {
-    const int c = blockIdx.x;
-    if (c >= cout) return;
-    const long n = g.n();
-    float s = 0.0f;
-    for (long v = threadIdx.x; v < n; v += blockDim.x) s += bf2f(dY[v * ch + c]);
-    __shared__ float part[256];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
+__global__ void __launch_bounds__(256, 3) wgrad_kernel(WLayers D) {
+    const int wave = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+    if (wave >= D.waves) return;
+    int e = 0;
+    while (e + 1 < D.n && D.l[e + 1].wave0 <= wave) ++e;
+    const WLayer& L = D.l[e];
+    const int w = wave - L.wave0, tap = w % 27, slice = w / 27;
+    switch (L.ct * 8 + L.it) {
+    case 8 + 1: wgrad_body<1, 1>(L, tap, slice); break;
+    case 8 + 2: wgrad_body<1, 2>(L, tap, slice); break;
+    case 16 + 1: wgrad_body<2, 1>(L, tap, slice); break;
+    case 16 + 4: wgrad_body<2, 4>(L, tap, slice); break;
+    case 32 + 2: wgrad_body<4, 2>(L, tap, slice); break;
+    default: wgrad_body<4, 4>(L, tap, slice); break;
     }
-    if (threadIdx.x == 0) db[c] = part[0];
+}
+
+// gw[co][tap][ci] and gb[co] (master layout): the slices' sums in slice order
+__global__ void __launch_bounds__(256) wgrad_reduce_kernel(WLayers D) {
+    const int t = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (t >= D.elems) return;
+    int e = 0;
+    while (e + 1 < D.n && D.l[e + 1].elem0 <= t) ++e;
+    const WLayer& L = D.l[e];
+    const int q = t - L.elem0, nw = L.cout * 27 * L.cin;
+    const int cop = 16 * L.ct, cip = 16 * L.it;
+    const float* p;
+    long stride;
+    if (q < nw) {
+        const int ci = q % L.cin, r = q / L.cin, tap = r % 27, co = r / 27;
+        p = L.part + (long)co * 27 * cip + tap * cip + ci;
+        stride = (long)cop * 27 * cip;
+    } else {
+        p = L.bpart + (q - nw);
+        stride = cop;
+    }
+    float s = 0.0f;
+    int sl = 0;
+    for (; sl + 8 <= L.slices; sl += 8) {  // 8 loads in flight
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = p[(sl + u) * stride];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    for (; sl < L.slices; ++sl) s += p[sl * stride];
+    if (q < nw) L.gw[q] = s;
+    else L.gb[q - nw] = s;
 }
 
 // ---- pooling / upsampling (channels-last), factor kF per axis ------------------
@@ -284,20 +442,18 @@ constexpr int kS = 4;  // fine cells per network cell, per axis
 constexpr int kF = 2;
 constexpr float kInvF3 = 1.0f / (kF * kF * kF);
 
-__device__ __forceinline__ long parent_of(const Geo& g, long v) {
-    const int i = (int)(v % g.nx);
-    const long q = v / g.nx;
-    const int j = (int)(q % g.ny), k = (int)(q / g.ny);
-    return (long)(i / kF) + (long)(g.nx / kF) * ((j / kF) + (long)(g.ny / kF) * (k / kF));
+__device__ __forceinline__ int parent_of(const Geo& g, int v) {
+    const int q = v / g.nx, i = v - q * g.nx;
+    const int k = q / g.ny, j = q - k * g.ny;
+    return i / kF + (g.nx / kF) * ((j / kF) + (g.ny / kF) * (k / kF));
 }
 
 // sum over the kF^3 children of coarse cell V (fine g), channel c
-__device__ __forceinline__ float child_sum(const Geo& g, int ch, const __hip_bfloat16* X, long V,
+__device__ __forceinline__ float child_sum(const Geo& g, int ch, const __hip_bfloat16* X, int V,
                                            int c) {
     const int NX = g.nx / kF, NY = g.ny / kF;
-    const int I = (int)(V % NX);
-    const long q = V / NX;
-    const int J = (int)(q % NY), K = (int)(q / NY);
+    const int q = V / NX, I = V - q * NX;
+    const int K = q / NY, J = q - K * NY;
     float s = 0.0f;
     for (int dz = 0; dz < kF; ++dz)
         for (int dy = 0; dy < kF; ++dy)
@@ -310,9 +466,9 @@ __device__ __forceinline__ float child_sum(const Geo& g, int ch, const __hip_bfl
 // pool: Y[V][c] = mean of the children of coarse cell V (fine g)
 __global__ void __launch_bounds__(256)
     pool_kernel(Geo g, int ch, const __hip_bfloat16* __restrict__ X, __hip_bfloat16* __restrict__ Y) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= g.n() / (kF * kF * kF) * ch) return;
-    Y[e] = f2bf(child_sum(g, ch, X, e / ch, (int)(e % ch)) * kInvF3);
+    Y[e] = f2bf(child_sum(g, ch, X, e / ch, e % ch) * kInvF3);
 }
 
 // pool backward with the skip gradient and the ReLU mask of the pooled input:
@@ -321,21 +477,13 @@ __global__ void __launch_bounds__(256)
     pool_bwd_kernel(Geo g, int ch, const __hip_bfloat16* __restrict__ dY,
                     const __hip_bfloat16* __restrict__ S, const __hip_bfloat16* __restrict__ M,
                     __hip_bfloat16* __restrict__ dX) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= g.n() * ch) return;
-    const int c = (int)(e % ch);
+    const int c = e % ch;
     float s = bf2f(dY[parent_of(g, e / ch) * ch + c]) * kInvF3;
     if (S) s += bf2f(S[e]);
     if (M) s = bf2f(M[e]) > 0.0f ? s : 0.0f;
     dX[e] = f2bf(s);
-}
-
-// up: Y[v][c] = X[parent(v)][c] (fine g)
-__global__ void __launch_bounds__(256)
-    up_kernel(Geo g, int ch, const __hip_bfloat16* __restrict__ X, __hip_bfloat16* __restrict__ Y) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= g.n() * ch) return;
-    Y[e] = X[parent_of(g, e / ch) * ch + (e % ch)];
 }
 
 // up backward with the ReLU mask of the coarse input:
@@ -343,9 +491,9 @@ __global__ void __launch_bounds__(256)
 __global__ void __launch_bounds__(256)
     up_bwd_kernel(Geo g, int ch, const __hip_bfloat16* __restrict__ dY,
                   const __hip_bfloat16* __restrict__ M, __hip_bfloat16* __restrict__ dX) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= g.n() / (kF * kF * kF) * ch) return;
-    float s = child_sum(g, ch, dY, e / ch, (int)(e % ch));
+    float s = child_sum(g, ch, dY, e / ch, e % ch);
     if (M) s = bf2f(M[e]) > 0.0f ? s : 0.0f;
     dX[e] = f2bf(s);
 }
@@ -472,42 +620,53 @@ __global__ void __launch_bounds__(256)
 }
 
 // per coarse cell V: target t = mean over its block of (h - h_lin) / J;
-// dOut[V][0] = 2 (y - t) / N_coarse (channels 1..dch-1 zero); loss partials
+// dOut[V][0] = 2 (y - t) / N_coarse (channels 1..15 zero); loss partials. A
+// workgroup holds 64 coarse cells x kS z-slices (one thread each, as
+// input_kernel: four times the loads in flight of a thread per cell); the
+// slices' sums are added in LDS in a fixed order.
 __global__ void __launch_bounds__(256)
-    loss_kernel(Geo g, double hw, double he, const float* __restrict__ y, int ych,
-                const double* __restrict__ h, __hip_bfloat16* __restrict__ dOut, int dch,
+    loss_kernel(Geo g, double hw, double he, const float* __restrict__ y,
+                const double* __restrict__ h, __hip_bfloat16* __restrict__ dOut,
                 float* __restrict__ partials) {
+    static_assert(kS == 4, "64 cells x 4 slices per workgroup");
     const int NX = g.nx / kS, NY = g.ny / kS, NZ = g.nz / kS;
     const long nc = (long)NX * NY * NZ;
-    const long V = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    float e2 = 0.0f;
+    const int lane = (int)(threadIdx.x & 63), dz = (int)(threadIdx.x >> 6);
+    const long V = (long)blockIdx.x * 64 + lane;
+    const double Jg = (hw - he) / g.nx;
+    double st = 0.0;
     if (V < nc) {
         const int I = (int)(V % NX);
         const long q = V / NX;
         const int J = (int)(q % NY), Kc = (int)(q / NY);
-        const double Jg = (hw - he) / g.nx;
-        double st = 0.0;
-        for (int dz = 0; dz < kS; ++dz)
-            for (int dy = 0; dy < kS; ++dy)
-                for (int dx = 0; dx < kS; ++dx) {
-                    const int i = kS * I + dx;
-                    const long o = (long)i + (long)g.nx * ((kS * J + dy) + (long)g.ny * (kS * Kc + dz));
-                    st += (h[o] - (hw + (he - hw) * (i + 0.5) / g.nx)) / Jg;
-                }
-        const float t = (float)(st / (kS * kS * kS));
-        const float d = y[V * ych] - t;
-        e2 = d * d;
-        dOut[V * dch] = f2bf(2.0f * d / (float)nc);
-        for (int c = 1; c < dch; ++c) dOut[V * dch + c] = f2bf(0.0f);
+        double hl[kS];
+#pragma unroll
+        for (int dx = 0; dx < kS; ++dx) hl[dx] = hw + (he - hw) * (kS * I + dx + 0.5) / g.nx;
+#pragma unroll
+        for (int dy = 0; dy < kS; ++dy)
+#pragma unroll
+            for (int dx = 0; dx < kS; ++dx)
+                st += h[(long)(kS * I + dx) +
+                        (long)g.nx * ((kS * J + dy) + (long)g.ny * (kS * Kc + dz))] - hl[dx];
     }
-    __shared__ float part[256];
-    part[threadIdx.x] = e2;
+    __shared__ double part[kS][64];
+    part[dz][lane] = st;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
+    if (dz != 0) return;  // whole waves
+    float e2 = 0.0f;
+    if (V < nc) {
+        st = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
+        const float t = (float)(st / Jg / (kS * kS * kS));
+        const float d = y[V * 16] - t;
+        e2 = d * d;
+        uint4* o = reinterpret_cast<uint4*>(dOut + V * 16);
+        const unsigned first = __builtin_bit_cast(unsigned short, f2bf(2.0f * d / (float)nc));
+        o[0] = uint4{first, 0u, 0u, 0u};
+        o[1] = uint4{0u, 0u, 0u, 0u};
     }
-    if (threadIdx.x == 0) partials[blockIdx.x] = part[0];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) e2 += __shfl_xor(e2, off, 64);
+    if (lane == 0) partials[blockIdx.x] = e2;
 }
 
 // ---- parameters ------------------------------------------------------------------
@@ -515,38 +674,36 @@ __global__ void __launch_bounds__(256)
 // W  [Cout_pad][Kpad]: W[co][tap*Cin_pad + ci] = w[co][tap][ci] (zero padded)
 // Wt [Cin_pad][Kpad_t]: Wt[ci][tap*Cout_pad + co] = w[co][tap][ci], used with
 //   FLIP (tap mirrored) for the data gradient
-__global__ void __launch_bounds__(256)
-    pack_kernel(const float* __restrict__ w, int cin, int cout, int cin_pad, int cout_pad,
-                int kpad, int kpad_t, __hip_bfloat16* __restrict__ W,
-                __hip_bfloat16* __restrict__ Wt) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long nW = (long)cout_pad * kpad, nWt = (long)cin_pad * kpad_t;
-    if (e < nW) {
-        const int co = (int)(e / kpad), k = (int)(e % kpad);
-        const int tap = k / cin_pad, ci = k % cin_pad;
+struct PackLayer {
+    const float* w;
+    int cin, cout, cin_pad, cout_pad, kpad, kpad_t;
+    __hip_bfloat16* W;
+    __hip_bfloat16* Wt;
+    int block0;  // first workgroup of the layer
+};
+struct PackLayers {
+    PackLayer l[kMaxWLayers];
+    int n;
+};
+__global__ void __launch_bounds__(256) pack_kernel(PackLayers D) {
+    int q = 0;
+    while (q + 1 < D.n && D.l[q + 1].block0 <= (int)blockIdx.x) ++q;
+    const PackLayer& L = D.l[q];
+    const int e = ((int)blockIdx.x - L.block0) * 256 + (int)threadIdx.x;
+    if (e < L.cout_pad * L.kpad) {
+        const int co = e / L.kpad, k = e % L.kpad;
+        const int tap = k / L.cin_pad, ci = k % L.cin_pad;
         float v = 0.0f;
-        if (co < cout && tap < 27 && ci < cin) v = w[((long)co * 27 + tap) * cin + ci];
-        W[e] = f2bf(v);
+        if (co < L.cout && tap < 27 && ci < L.cin) v = L.w[(co * 27 + tap) * L.cin + ci];
+        L.W[e] = f2bf(v);
     }
-    if (e < nWt) {
-        const int ci = (int)(e / kpad_t), k = (int)(e % kpad_t);
-        const int tap = k / cout_pad, co = k % cout_pad;
+    if (e < L.cin_pad * L.kpad_t) {
+        const int ci = e / L.kpad_t, k = e % L.kpad_t;
+        const int tap = k / L.cout_pad, co = k % L.cout_pad;
         float v = 0.0f;
-        if (ci < cin && tap < 27 && co < cout) v = w[((long)co * 27 + tap) * cin + ci];
-        Wt[e] = f2bf(v);
+        if (ci < L.cin && tap < 27 && co < L.cout) v = L.w[(co * 27 + tap) * L.cin + ci];
+        L.Wt[e] = f2bf(v);
     }
-}
-
-// layer weight gradient in the master layout from G[co][tap*Cin_pad + ci]
-__global__ void __launch_bounds__(256)
-    unpack_grad_kernel(const float* __restrict__ G, int cin, int cout, int cin_pad,
-                       float* __restrict__ gw) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (long)cout * 27 * cin) return;
-    const int ci = (int)(e % cin);
-    const long q = e / cin;
-    const int tap = (int)(q % 27), co = (int)(q / 27);
-    gw[e] = G[(long)co * 27 * cin_pad + (long)tap * cin_pad + ci];
 }
 
 // Adam (Kingma & Ba 2015) with bias correction folded into the step size
@@ -595,6 +752,15 @@ long param_count() {
 using namespace mf3d;
 using namespace mf3d::cnn;
 
+// Weight gradients of up to kMaxWLayers layers: channel-first operand copies
+// and per-slice partial sums in one zeroed allocation
+struct WeightScratch {
+    void* mem = nullptr;
+    PlanarCopies copies{};
+    int copy_blocks = 0;
+    WLayers layers{};
+};
+
 struct mf3d_wsnet {
     float* params = nullptr;  // FP32 master: per layer w then bias
     float* grads = nullptr;
@@ -611,17 +777,14 @@ struct mf3d_wsnet {
     int gx = 0, gy = 0, gz = 0;
     std::vector<void*> act;
     __hip_bfloat16 *x0 = nullptr, *e0 = nullptr, *p1 = nullptr, *e1 = nullptr, *p2 = nullptr,
-                   *e2 = nullptr, *e2b = nullptr, *u1 = nullptr, *d1 = nullptr, *u0 = nullptr,
-                   *d0 = nullptr;
+                   *e2 = nullptr, *e2b = nullptr, *d1 = nullptr, *d0 = nullptr;
     float* y = nullptr;  // [N0][16] FP32 (channel 0 used)
     float* yd = nullptr; // [N0] channel 0 of y, dense (read by the output interpolation)
-    // backward scratch
-    __hip_bfloat16 *g0a = nullptr, *g0b = nullptr, *g0c = nullptr, *g1a = nullptr,
-                   *g1b = nullptr, *g2a = nullptr, *g2b = nullptr;
-    float* wpart = nullptr;
-    long wpart_cap = 0;
-    float* G = nullptr;
-    long G_cap = 0;
+    // backward: the layers' pre-activation gradients (kept until the weight
+    // gradients, which run for all layers at once) and upsampled ones
+    __hip_bfloat16 *g0a = nullptr, *g0b = nullptr, *g0c = nullptr, *g0d = nullptr, *g1a = nullptr,
+                   *g1b = nullptr, *g1c = nullptr, *g2a = nullptr, *g2b = nullptr, *g2c = nullptr;
+    WeightScratch wg;
     float* lpart = nullptr;
     float* host_lpart = nullptr;
     long lpart_cap = 0;
@@ -638,12 +801,12 @@ void free_acts(mf3d_wsnet* net) {
     for (void* p : net->act) (void)hipFree(p);
     net->act.clear();
     net->gx = net->gy = net->gz = 0;
-    if (net->wpart) (void)hipFree(net->wpart);
-    if (net->G) (void)hipFree(net->G);
+    if (net->wg.mem) (void)hipFree(net->wg.mem);
+    net->wg = WeightScratch{};
     if (net->lpart) (void)hipFree(net->lpart);
     if (net->host_lpart) (void)hipHostFree(net->host_lpart);
-    net->wpart = net->G = net->lpart = net->host_lpart = nullptr;
-    net->wpart_cap = net->G_cap = net->lpart_cap = 0;
+    net->lpart = net->host_lpart = nullptr;
+    net->lpart_cap = 0;
 }
 
 int check_grid(const mf3d_grid* g) {
@@ -654,7 +817,85 @@ int check_grid(const mf3d_grid* g) {
     return MF3D_OK;
 }
 
-constexpr int kSlices = 64;
+// one layer whose weight gradient is wanted (dY, X: channels-last, 16 ct and 16
+// it channels; up: X on the half-size grid)
+struct WeightTask {
+    mf3d_grid g;
+    const __hip_bfloat16* dY;
+    const __hip_bfloat16* X;
+    int ct, it, up, cin, cout;
+    float* gw;
+    float* gb;
+};
+
+// Slices of a layer: 16 steps (512 voxels) a wave amortise its partial sums;
+// fewer steps where the layer would otherwise have under 8 slices (27 taps x 8
+// waves), more above 64 slices (whose partial sums would grow with the grid).
+int make_scratch(WeightScratch& S, const WeightTask* T, int n) {
+    S.copies.n = 0;
+    S.copy_blocks = 0;
+    S.layers.n = n;
+    S.layers.waves = S.layers.elems = 0;
+    size_t bytes = 0;
+    auto take = [&](size_t b) {
+        const size_t at = bytes;
+        bytes += (b + 255) / 256 * 256;
+        return at;
+    };
+    std::vector<size_t> at;
+    for (int e = 0; e < n; ++e) {
+        const WeightTask& t = T[e];
+        WLayer& L = S.layers.l[e];
+        L.P = planar_of(t.g);
+        L.ct = t.ct, L.it = t.it;
+        const long steps = (L.P.groups + 3) / 4;
+        L.steps = (int)std::max({1L, std::min(16L, steps / 8), (steps + 63) / 64});
+        L.slices = (int)((steps + L.steps - 1) / L.steps);
+        L.wave0 = S.layers.waves;
+        S.layers.waves += 27 * L.slices;
+        L.cin = t.cin, L.cout = t.cout, L.gw = t.gw, L.gb = t.gb;
+        L.elem0 = S.layers.elems;
+        S.layers.elems += 27 * t.cin * t.cout + t.cout;
+        at.push_back(take((size_t)16 * L.ct * L.P.plane * 2));
+        at.push_back(take((size_t)16 * L.it * L.P.plane * 2));
+        at.push_back(take((size_t)L.slices * 16 * L.ct * 27 * 16 * L.it * 4));
+        at.push_back(take((size_t)L.slices * 16 * L.ct * 4));
+        for (int q = 0; q < 2; ++q) {
+            PlanarCopy& C = S.copies.c[S.copies.n++];
+            C.src = q ? t.X : t.dY;
+            C.ch = 16 * (q ? t.it : t.ct);
+            C.up = q ? t.up : 0;
+            C.g = Geo{t.g.nx, t.g.ny, t.g.nz};
+            C.P = L.P;
+            C.block0 = S.copy_blocks;
+            C.vblocks = (int)blocks((long)cells(t.g));
+            S.copy_blocks += C.vblocks * (C.ch / 8);
+        }
+    }
+    MF3D_TRY(net_alloc(&S.mem, bytes));
+    // the copies' borders stay zero: planar_kernel writes the voxels only
+    MF3D_HIP_TRY(hipMemset(S.mem, 0, bytes));
+    MF3D_HIP_TRY(hipDeviceSynchronize());
+    char* m = static_cast<char*>(S.mem);
+    for (int e = 0; e < n; ++e) {
+        WLayer& L = S.layers.l[e];
+        __hip_bfloat16* d[2] = {(__hip_bfloat16*)(m + at[4 * e]), (__hip_bfloat16*)(m + at[4 * e + 1])};
+        L.dY = d[0], L.X = d[1];
+        S.copies.c[2 * e].dst = d[0];
+        S.copies.c[2 * e + 1].dst = d[1];
+        L.part = (float*)(m + at[4 * e + 2]);
+        L.bpart = (float*)(m + at[4 * e + 3]);
+    }
+    return MF3D_OK;
+}
+
+int run_weight_grads(hipStream_t s, const WeightScratch& S) {
+    planar_kernel<<<S.copy_blocks, 256, 0, s>>>(S.copies);
+    wgrad_kernel<<<(S.layers.waves + 3) / 4, 256, 0, s>>>(S.layers);
+    wgrad_reduce_kernel<<<blocks(S.layers.elems), 256, 0, s>>>(S.layers);
+    MF3D_HIP_TRY(hipGetLastError());
+    return MF3D_OK;
+}
 
 int ensure_acts(mf3d_wsnet* net, const mf3d_grid& g) {
     if (net->gx == g.nx && net->gy == g.ny && net->gz == g.nz) return MF3D_OK;
@@ -674,13 +915,14 @@ int ensure_acts(mf3d_wsnet* net, const mf3d_grid& g) {
     MF3D_TRY(bf(&net->p2, n2 * 32));
     MF3D_TRY(bf(&net->e2, n2 * 64));
     MF3D_TRY(bf(&net->e2b, n2 * 64));
-    MF3D_TRY(bf(&net->u1, n1 * 64));
     MF3D_TRY(bf(&net->d1, n1 * 32));
-    MF3D_TRY(bf(&net->u0, n0 * 32));
     MF3D_TRY(bf(&net->d0, n0 * 16));
     MF3D_TRY(bf(&net->g0a, n0 * 32));
     MF3D_TRY(bf(&net->g0b, n0 * 32));
     MF3D_TRY(bf(&net->g0c, n0 * 16));
+    MF3D_TRY(bf(&net->g0d, n0 * 16));
+    MF3D_TRY(bf(&net->g1c, n1 * 16));
+    MF3D_TRY(bf(&net->g2c, n2 * 32));
     MF3D_TRY(bf(&net->g1a, n1 * 64));
     MF3D_TRY(bf(&net->g1b, n1 * 64));
     MF3D_TRY(bf(&net->g2a, n2 * 64));
@@ -692,16 +934,7 @@ int ensure_acts(mf3d_wsnet* net, const mf3d_grid& g) {
     MF3D_TRY(net_alloc(&q, n0 * sizeof(float)));
     net->act.push_back(q);
     net->yd = static_cast<float*>(q);
-    long wp = 0, gmax = 0;
-    for (int l = 0; l < kNumLayers; ++l) {
-        wp = std::max(wp, (long)kSlices * net->cout_pad[l] * 27L * net->cin_pad[l]);
-        gmax = std::max(gmax, (long)net->cout_pad[l] * 27L * net->cin_pad[l]);
-    }
-    MF3D_TRY(net_alloc((void**)&net->wpart, wp * sizeof(float)));
-    MF3D_TRY(net_alloc((void**)&net->G, gmax * sizeof(float)));
-    net->wpart_cap = wp;
-    net->G_cap = gmax;
-    const long nb = (long)blocks((long)n0);
+    const long nb = ((long)n0 + 63) / 64;  // workgroups of loss_kernel
     MF3D_TRY(net_alloc((void**)&net->lpart, nb * sizeof(float)));
     MF3D_HIP_TRY(hipHostMalloc((void**)&net->host_lpart, nb * sizeof(float), hipHostMallocDefault));
     net->lpart_cap = nb;
@@ -711,15 +944,21 @@ int ensure_acts(mf3d_wsnet* net, const mf3d_grid& g) {
     return MF3D_OK;
 }
 
+// appends a layer to D; returns the workgroups so far
+int add_pack(PackLayers& D, int block0, const float* w, int cin, int cout, int cin_pad,
+             int cout_pad, __hip_bfloat16* W, __hip_bfloat16* Wt) {
+    const int kp = kpad_of(cin_pad), kpt = kpad_of(cout_pad);
+    D.l[D.n++] = PackLayer{w, cin, cout, cin_pad, cout_pad, kp, kpt, W, Wt, block0};
+    return block0 + (int)blocks(std::max((long)cout_pad * kp, (long)cin_pad * kpt));
+}
+
 int pack(mf3d_wsnet* net, hipStream_t s) {
-    for (int l = 0; l < kNumLayers; ++l) {
-        const LayerDef& L = kLayers[l];
-        const long n = std::max((long)net->cout_pad[l] * net->kpad[l],
-                                (long)net->cin_pad[l] * net->kpad_t[l]);
-        pack_kernel<<<blocks(n), 256, 0, s>>>(net->params + net->woff[l], L.cin, L.cout,
-                                              net->cin_pad[l], net->cout_pad[l], net->kpad[l],
-                                              net->kpad_t[l], net->W[l], net->Wt[l]);
-    }
+    PackLayers D{};
+    int nb = 0;
+    for (int l = 0; l < kNumLayers; ++l)
+        nb = add_pack(D, nb, net->params + net->woff[l], kLayers[l].cin, kLayers[l].cout,
+                      net->cin_pad[l], net->cout_pad[l], net->W[l], net->Wt[l]);
+    pack_kernel<<<nb, 256, 0, s>>>(D);
     MF3D_HIP_TRY(hipGetLastError());
     net->packed = true;
     return MF3D_OK;
@@ -729,26 +968,32 @@ int pack(mf3d_wsnet* net, hipStream_t s) {
 int conv(hipStream_t s, const mf3d_grid& g, int cin_ch, int cout_pad, int kp, int cs,
          const __hip_bfloat16* X, const __hip_bfloat16* W, const float* bias,
          const __hip_bfloat16* R, const __hip_bfloat16* M, bool relu, bool flip, void* out,
-         bool f32out) {
+         bool f32out, bool up = false) {
     const Geo G{g.nx, g.ny, g.nz};
     // 16-voxel tiles per wave: kVT on large grids, fewer where that would
     // leave the launch with fewer than kConvWaves waves (the small grids of
-    // the deeper layers; same products and order per output either way)
+    // the deeper layers; same products and order per output either way); below
+    // that, waves share a tile's k steps (kConvWaves / 4 tiles and fewer: 4, a
+    // sixteenth and fewer: 16)
     const long nv = (long)cells(g);
     const int vt = (nv + 16 * kVT - 1) / (16 * kVT) >= kConvWaves ? kVT
                    : (nv + 31) / 32 >= kConvWaves                   ? 2
                                                                     : 1;
-    const long waves = (nv + 16L * vt - 1) / (16L * vt);
-    const unsigned nb = (unsigned)((waves + 3) / 4);
+    const long tiles = (nv + 16L * vt - 1) / (16L * vt);
+    const int ks = vt > 1 ? 1 : tiles <= kConvWaves / 16 ? 16 : tiles <= kConvWaves / 4 ? 4 : 1;
+    const int wpb = ks > 4 ? ks : 4;
+    const unsigned nb = (unsigned)((tiles * ks + wpb - 1) / wpb);
     const int ct = cout_pad / 16;
-#define MF3D_CONV(CTV, VTV, F32)                                                               \
-    conv_kernel<CTV, VTV, F32><<<nb, 256, 0, s>>>(G, cin_ch, kp, cs, X, W, bias, R, M,        \
-                                                  relu ? 1 : 0, flip ? 1 : 0, out)
+#define MF3D_CONV(CTV, VTV, F32, KSV)                                                          \
+    conv_kernel<CTV, VTV, F32, KSV><<<nb, wpb * 64, 0, s>>>(                                    \
+        G, cin_ch, kp, cs, up ? 1 : 0, X, W, bias, R, M, relu ? 1 : 0, flip ? 1 : 0, out)
 #define MF3D_CONV_VT(CTV, F32)                                                                 \
     do {                                                                                       \
-        if (vt == kVT) MF3D_CONV(CTV, kVT, F32);                                               \
-        else if (vt == 2) MF3D_CONV(CTV, 2, F32);                                              \
-        else MF3D_CONV(CTV, 1, F32);                                                           \
+        if (vt == kVT) MF3D_CONV(CTV, kVT, F32, 1);                                            \
+        else if (vt == 2) MF3D_CONV(CTV, 2, F32, 1);                                           \
+        else if (ks == 1) MF3D_CONV(CTV, 1, F32, 1);                                           \
+        else if (ks == 4) MF3D_CONV(CTV, 1, F32, 4);                                           \
+        else MF3D_CONV(CTV, 1, F32, 16);                                                       \
     } while (0)
     if (f32out) {
         if (ct != 1) return fail(MF3D_ERR_UNSUPPORTED, "FP32 output only for 16 channels");
@@ -759,31 +1004,6 @@ int conv(hipStream_t s, const mf3d_grid& g, int cin_ch, int cout_pad, int kp, in
     else return fail(MF3D_ERR_UNSUPPORTED, "convolution: unsupported channel count");
 #undef MF3D_CONV_VT
 #undef MF3D_CONV
-    MF3D_HIP_TRY(hipGetLastError());
-    return MF3D_OK;
-}
-
-// weight gradient (G[co][tap*cin_ch + ci], FP32) of a layer from dY (cout_ch
-// channels) and its input X (cin_ch channels)
-int wgrad(mf3d_wsnet* net, hipStream_t s, const mf3d_grid& g, int cin_ch, int cout_ch,
-          int cout, const __hip_bfloat16* dY, const __hip_bfloat16* X, float* G) {
-    const Geo geo{g.nx, g.ny, g.nz};
-    const int ct = cout_ch / 16, it = cin_ch / 16;
-    const long K = 27L * cin_ch;
-    if ((long)kSlices * cout_ch * K > net->wpart_cap)
-        return fail(MF3D_ERR_UNSUPPORTED, "weight-gradient scratch too small");
-    const unsigned nb = 27 * kSlices;
-#define MF3D_WG(C, I) wgrad_kernel<C, I><<<nb, 64, 0, s>>>(geo, cin_ch, cout_ch, dY, X, kSlices, net->wpart)
-    if (ct == 1 && it == 1) MF3D_WG(1, 1);
-    else if (ct == 1 && it == 2) MF3D_WG(1, 2);
-    else if (ct == 2 && it == 1) MF3D_WG(2, 1);
-    else if (ct == 2 && it == 4) MF3D_WG(2, 4);
-    else if (ct == 4 && it == 2) MF3D_WG(4, 2);
-    else if (ct == 4 && it == 4) MF3D_WG(4, 4);
-    else return fail(MF3D_ERR_UNSUPPORTED, "weight gradient: unsupported channel counts");
-#undef MF3D_WG
-    wgrad_reduce_kernel<<<blocks((long)cout * K), 256, 0, s>>>(net->wpart, kSlices, cout, cout_ch,
-                                                               K, G);
     MF3D_HIP_TRY(hipGetLastError());
     return MF3D_OK;
 }
@@ -817,12 +1037,10 @@ int forward(mf3d_wsnet* net, hipStream_t s, const mf3d_grid& gf, const double* K
                   nullptr, true, false, net->e2, false));
     MF3D_TRY(conv(s, g2, 64, 64, net->kpad[3], 64, net->e2, net->W[3], P + net->boff[3], nullptr,
                   nullptr, true, false, net->e2b, false));
-    up_kernel<<<blocks(n1 * 64), 256, 0, s>>>(Geo{g1.nx, g1.ny, g1.nz}, 64, net->e2b, net->u1);
-    MF3D_TRY(conv(s, g1, 64, 32, net->kpad[4], 32, net->u1, net->W[4], P + net->boff[4], net->e1,
-                  nullptr, true, false, net->d1, false));
-    up_kernel<<<blocks(n0 * 32), 256, 0, s>>>(G0, 32, net->d1, net->u0);
-    MF3D_TRY(conv(s, g, 32, 16, net->kpad[5], 16, net->u0, net->W[5], P + net->boff[5], net->e0,
-                  nullptr, true, false, net->d0, false));
+    MF3D_TRY(conv(s, g1, 64, 32, net->kpad[4], 32, net->e2b, net->W[4], P + net->boff[4], net->e1,
+                  nullptr, true, false, net->d1, false, true));
+    MF3D_TRY(conv(s, g, 32, 16, net->kpad[5], 16, net->d1, net->W[5], P + net->boff[5], net->e0,
+                  nullptr, true, false, net->d0, false, true));
     MF3D_TRY(conv(s, g, 16, 16, net->kpad[6], 16, net->d0, net->W[6], P + net->boff[6], nullptr,
                   nullptr, false, false, net->y, true));
     MF3D_HIP_TRY(hipGetLastError());
@@ -836,51 +1054,50 @@ int backward(mf3d_wsnet* net, hipStream_t s, const mf3d_grid& gf, double hw, dou
     const mf3d_grid g1 = coarse(g, kF), g2 = coarse(g, kF * kF);
     const Geo G0{g.nx, g.ny, g.nz}, G1{g1.nx, g1.ny, g1.nz};
     const long n0 = (long)cells(g), n1 = (long)cells(g1), n2 = (long)cells(g2);
-    const unsigned lb = blocks(n0);
+    const unsigned lb = (unsigned)((n0 + 63) / 64);
     float* GR = net->grads;
     // dY of conv_g (16 channels, channel 0 live) -> g0c
-    loss_kernel<<<lb, 256, 0, s>>>(Geo{gf.nx, gf.ny, gf.nz}, hw, he, net->y, 16, h, net->g0c, 16,
+    loss_kernel<<<lb, 256, 0, s>>>(Geo{gf.nx, gf.ny, gf.nz}, hw, he, net->y, h, net->g0c,
                                    net->lpart);
-    auto grads_of = [&](int l, const mf3d_grid& gg, int cin_ch, int cout_ch,
-                        const __hip_bfloat16* dY, const __hip_bfloat16* X) -> int {
-        const LayerDef& L = kLayers[l];
-        MF3D_TRY(wgrad(net, s, gg, cin_ch, cout_ch, L.cout, dY, X, net->G));
-        unpack_grad_kernel<<<blocks(27L * L.cin * L.cout), 256, 0, s>>>(net->G, L.cin, L.cout,
-                                                                       cin_ch, GR + net->woff[l]);
-        bgrad_kernel<<<L.cout, 256, 0, s>>>(Geo{gg.nx, gg.ny, gg.nz}, cout_ch, L.cout, dY,
-                                            GR + net->boff[l]);
-        MF3D_HIP_TRY(hipGetLastError());
-        return MF3D_OK;
-    };
-    // conv_g: input d0 (16); data gradient masked by d0 > 0 -> g0b (16 ch)
-    MF3D_TRY(grads_of(6, g, 16, 16, net->g0c, net->d0));
+    // conv_g: data gradient masked by d0 > 0 -> dPre_f (g0b, 16 ch), also e0's skip gradient
     MF3D_TRY(conv(s, g, 16, 16, net->kpad_t[6], 16, net->g0c, net->Wt[6], nullptr, nullptr,
                   net->d0, false, true, net->g0b, false));
-    // conv_f (dPre_f = g0b): input u0 (32); skip gradient to e0 = g0b
-    MF3D_TRY(grads_of(5, g, 32, 16, net->g0b, net->u0));
     MF3D_TRY(conv(s, g, 16, 32, net->kpad_t[5], 32, net->g0b, net->Wt[5], nullptr, nullptr,
                   nullptr, false, true, net->g0a, false));  // du0 (32 ch)
     // up bwd into d1, masked by d1 > 0 -> dPre_e (g1a, 32 ch)
     up_bwd_kernel<<<blocks(n1 * 32), 256, 0, s>>>(G0, 32, net->g0a, net->d1, net->g1a);
-    MF3D_TRY(grads_of(4, g1, 64, 32, net->g1a, net->u1));
     MF3D_TRY(conv(s, g1, 32, 64, net->kpad_t[4], 64, net->g1a, net->Wt[4], nullptr, nullptr,
                   nullptr, false, true, net->g1b, false));  // du1 (64 ch)
     // up bwd into e2b, masked -> dPre_d (g2a)
     up_bwd_kernel<<<blocks(n2 * 64), 256, 0, s>>>(G1, 64, net->g1b, net->e2b, net->g2a);
-    MF3D_TRY(grads_of(3, g2, 64, 64, net->g2a, net->e2));
     MF3D_TRY(conv(s, g2, 64, 64, net->kpad_t[3], 64, net->g2a, net->Wt[3], nullptr, nullptr,
                   net->e2, false, true, net->g2b, false));  // dPre_c (64 ch)
-    MF3D_TRY(grads_of(2, g2, 32, 64, net->g2b, net->p2));
     MF3D_TRY(conv(s, g2, 64, 32, net->kpad_t[2], 32, net->g2b, net->Wt[2], nullptr, nullptr,
-                  nullptr, false, true, net->g2a, false));  // dp2 (32 ch)
+                  nullptr, false, true, net->g2c, false));  // dp2 (32 ch)
     // pool bwd into e1 + skip gradient (g1a), masked by e1 -> dPre_b (g1b, 32 ch)
-    pool_bwd_kernel<<<blocks(n1 * 32), 256, 0, s>>>(G1, 32, net->g2a, net->g1a, net->e1, net->g1b);
-    MF3D_TRY(grads_of(1, g1, 16, 32, net->g1b, net->p1));
+    pool_bwd_kernel<<<blocks(n1 * 32), 256, 0, s>>>(G1, 32, net->g2c, net->g1a, net->e1, net->g1b);
     MF3D_TRY(conv(s, g1, 32, 16, net->kpad_t[1], 16, net->g1b, net->Wt[1], nullptr, nullptr,
-                  nullptr, false, true, net->g1a, false));  // dp1 (16 ch)
-    // pool bwd into e0 + skip gradient (g0b), masked by e0 -> dPre_a (g0c, 16 ch)
-    pool_bwd_kernel<<<blocks(n0 * 16), 256, 0, s>>>(G0, 16, net->g1a, net->g0b, net->e0, net->g0c);
-    MF3D_TRY(grads_of(0, g, 16, 16, net->g0c, net->x0));
+                  nullptr, false, true, net->g1c, false));  // dp1 (16 ch)
+    // pool bwd into e0 + skip gradient (g0b), masked by e0 -> dPre_a (g0d, 16 ch)
+    pool_bwd_kernel<<<blocks(n0 * 16), 256, 0, s>>>(G0, 16, net->g1c, net->g0b, net->e0, net->g0d);
+    MF3D_HIP_TRY(hipGetLastError());
+    if (!net->wg.mem) {
+        const struct {
+            const mf3d_grid* g;
+            const __hip_bfloat16 *dY, *X;
+            int up;
+        } in[kNumLayers] = {{&g, net->g0d, net->x0, 0},   {&g1, net->g1b, net->p1, 0},
+                            {&g2, net->g2b, net->p2, 0},  {&g2, net->g2a, net->e2, 0},
+                            {&g1, net->g1a, net->e2b, 1}, {&g, net->g0b, net->d1, 1},
+                            {&g, net->g0c, net->d0, 0}};
+        WeightTask T[kNumLayers];
+        for (int l = 0; l < kNumLayers; ++l)
+            T[l] = WeightTask{*in[l].g, in[l].dY, in[l].X, net->cout_pad[l] / 16,
+                              net->cin_pad[l] / 16, in[l].up, kLayers[l].cin, kLayers[l].cout,
+                              GR + net->woff[l], GR + net->boff[l]};
+        MF3D_TRY(make_scratch(net->wg, T, kNumLayers));
+    }
+    MF3D_TRY(run_weight_grads(s, net->wg));
     if (loss) {
         MF3D_HIP_TRY(hipMemcpyAsync(net->host_lpart, net->lpart, lb * sizeof(float),
                                     hipMemcpyDeviceToHost, s));
@@ -1068,8 +1285,9 @@ int mf3d_conv3d_forward(mf3d_stream stream, const mf3d_grid* grid, int cin, int 
     MF3D_TRY(net_alloc((void**)&W, (size_t)cout * kp * 2));
     int st = net_alloc((void**)&Wt, (size_t)pad16(cin) * kpt * 2);
     if (st == MF3D_OK) {
-        pack_kernel<<<blocks(std::max((long)cout * kp, (long)pad16(cin) * kpt)), 256, 0, s>>>(
-            w, cin, cout, cin, cout, kp, kpt, W, Wt);
+        PackLayers D{};
+        const int nb = add_pack(D, 0, w, cin, cout, cin, cout, W, Wt);
+        pack_kernel<<<nb, 256, 0, s>>>(D);
         st = conv(s, *grid, cin, cout, kp, cout, (const __hip_bfloat16*)X, W, bias,
                   (const __hip_bfloat16*)R, nullptr, relu != 0, false, Y, false);
     }
@@ -1097,8 +1315,9 @@ int mf3d_conv3d_backward_data(mf3d_stream stream, const mf3d_grid* grid, int cin
     MF3D_TRY(net_alloc((void**)&W, (size_t)cout * kp * 2));
     int st = net_alloc((void**)&Wt, (size_t)cin * kpt * 2);
     if (st == MF3D_OK) {
-        pack_kernel<<<blocks(std::max((long)cout * kp, (long)cin * kpt)), 256, 0, s>>>(
-            w, cin, cout, cin, cout, kp, kpt, W, Wt);
+        PackLayers D{};
+        const int nb = add_pack(D, 0, w, cin, cout, cin, cout, W, Wt);
+        pack_kernel<<<nb, 256, 0, s>>>(D);
         st = conv(s, *grid, cout, cin, kpt, cin, (const __hip_bfloat16*)dY, Wt, nullptr, nullptr,
                   (const __hip_bfloat16*)M, false, true, dX, false);
     }
@@ -1121,25 +1340,20 @@ int mf3d_conv3d_backward_weights(mf3d_stream stream, const mf3d_grid* grid, int 
         return fail(MF3D_ERR_UNSUPPORTED, "cin and cout must be 16/32/64");
     (void)hipGetLastError();
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    mf3d_wsnet tmp;
-    const long K = 27L * cin;
-    tmp.wpart_cap = (long)kSlices * cout * K;
-    MF3D_TRY(net_alloc((void**)&tmp.wpart, tmp.wpart_cap * sizeof(float)));
-    float* G = nullptr;
-    int st = net_alloc((void**)&G, (size_t)cout * K * sizeof(float));
-    if (st == MF3D_OK)
-        st = wgrad(&tmp, s, *grid, cin, cout, cout, (const __hip_bfloat16*)dY,
-                   (const __hip_bfloat16*)X, G);
+    const int ct = cout / 16, it = cin / 16;
+    const bool known = (ct == 1 && it <= 2) || (ct == 2 && (it == 1 || it == 4)) ||
+                       (ct == 4 && (it == 2 || it == 4));
+    if (!known) return fail(MF3D_ERR_UNSUPPORTED, "weight gradient: unsupported channel counts");
+    const WeightTask T{*grid, (const __hip_bfloat16*)dY, (const __hip_bfloat16*)X, ct, it, 0, cin,
+                       cout, gw, gb};
+    WeightScratch S;
+    int st = make_scratch(S, &T, 1);
+    if (st == MF3D_OK) st = run_weight_grads(s, S);
     if (st == MF3D_OK) {
-        unpack_grad_kernel<<<blocks((long)cout * K), 256, 0, s>>>(G, cin, cout, cin, gw);
-        bgrad_kernel<<<cout, 256, 0, s>>>(Geo{grid->nx, grid->ny, grid->nz}, cout, cout,
-                                          (const __hip_bfloat16*)dY, gb);
         const hipError_t e = hipStreamSynchronize(s);
         if (e != hipSuccess) st = fail(MF3D_ERR_HIP, hipGetErrorString(e));
     }
-    (void)hipFree(tmp.wpart);
-    tmp.wpart = nullptr;
-    if (G) (void)hipFree(G);
+    if (S.mem) (void)hipFree(S.mem);
     return st;
 }
 
