@@ -167,34 +167,50 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
             for (int q = 0; q < 2; ++q) iu.v[q] = recip(Ku.v[q]);
             const double iw = recip(Kw), ie = recip(Ke);
-            const double mid = 2.0 * recip(ic.v[0] + ic.v[1]);  // between the two cells
+            const double imid = ic.v[0] + ic.v[1];  // between the two cells
+            const double tmid = KIND == COL_RES ? quot(2.0 * (xc.v[0] - xc.v[1]), imid) : 0.0;
             double res[2];
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 const double me = ic.v[e], K2 = 2.0 * Kc.v[e], xC = xc.v[e];
                 // an odd row's single last cell has its east side on the boundary
                 const bool inner = e == 0 && two;
-                const double fe = inner ? mid : kface(E, me, ie, K2);
-                const double fw = e == 1 ? mid : kface(W, me, iw, K2);
-                const double fn = kface(N, me, recip(Kn.v[e]), K2);
-                const double fs = kface(S, me, recip(Ks.v[e]), K2);
-                const double fu = kface(U, me, iu.v[e], K2);
-                const double fd = kface(D, me, id.v[e], K2);
-                const double ve = inner ? xc.v[1] : (E.nb ? xe : 0.0);
-                const double vw = e == 1 ? xc.v[0] : (W.nb ? xw : 0.0);
-                double r = fw * (xC - vw);
-                r += fe * (xC - ve);
-                r += fs * (xC - (S.nb ? xs.v[e] : 0.0));
-                r += fn * (xC - (N.nb ? xn.v[e] : 0.0));
-                r += fd * (xC - (D.nb ? xd.v[e] : 0.0));
-                r += fu * (xC - (U.nb ? xu.v[e] : 0.0));
-                if (pin && o + e == 0) {
-                    double aC = 0.0;  // the smoother's diagonal, or in-domain faces only
-                    if (KIND == COL_RES) aC = fw + fe + fs + fn + fd + fu;
-                    else aC = (nx > 1 ? fe : 0.0) + (ny > 1 ? fn : 0.0) + (nz > 1 ? fu : 0.0);
-                    r += aC * xC;
+                const double in = recip(Kn.v[e]), is = recip(Ks.v[e]);
+                if (KIND == COL_RES) {
+                    // 2 (x_C - x_nb) / (1/K_C + 1/K_nb), one rounding per term
+                    auto term = [&](const Side& s, double ib, double v) {
+                        return s.nb ? quot(2.0 * (xC - v), me + ib) : (s.face ? K2 * xC : 0.0);
+                    };
+                    double r = inner ? tmid : term(E, ie, xe);
+                    r += term(N, in, xn.v[e]);
+                    r += e == 1 ? -tmid : term(W, iw, xw);
+                    r += term(S, is, xs.v[e]);
+                    r += term(U, iu.v[e], xu.v[e]);
+                    r += term(D, id.v[e], xd.v[e]);
+                    if (pin && o + e == 0) {  // the smoother's diagonal (cell 0: the pair's first)
+                        double aC = kface(W, me, iw, K2);
+                        aC += inner ? 2.0 * recip(imid) : kface(E, me, ie, K2);
+                        aC += kface(S, me, is, K2) + kface(N, me, in, K2);
+                        aC += kface(D, me, id.v[e], K2) + kface(U, me, iu.v[e], K2);
+                        r += aC * xC;
+                    }
+                    res[e] = bv.v[e] + r * inv_dx2;
+                } else {
+                    const double mid = 2.0 * recip(imid);
+                    const double fe = inner ? mid : kface(E, me, ie, K2);
+                    const double fw = e == 1 ? mid : kface(W, me, iw, K2);
+                    const double fn = kface(N, me, in, K2), fs = kface(S, me, is, K2);
+                    const double fu = kface(U, me, iu.v[e], K2), fd = kface(D, me, id.v[e], K2);
+                    double r = fw * (xC - (e == 1 ? xc.v[0] : (W.nb ? xw : 0.0)));
+                    r += fe * (xC - (inner ? xc.v[1] : (E.nb ? xe : 0.0)));
+                    r += fs * (xC - (S.nb ? xs.v[e] : 0.0));
+                    r += fn * (xC - (N.nb ? xn.v[e] : 0.0));
+                    r += fd * (xC - (D.nb ? xd.v[e] : 0.0));
+                    r += fu * (xC - (U.nb ? xu.v[e] : 0.0));
+                    if (pin && o + e == 0)  // in-domain faces only
+                        r += ((nx > 1 ? fe : 0.0) + (ny > 1 ? fn : 0.0) + (nz > 1 ? fu : 0.0)) * xC;
+                    res[e] = -r * inv_dx2;
                 }
-                res[e] = KIND == COL_RES ? bv.v[e] + r * inv_dx2 : -r * inv_dx2;
             }
             if (VEC) {
                 typedef double __attribute__((ext_vector_type(2))) dbl2;
