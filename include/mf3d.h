@@ -252,9 +252,12 @@ enum {
     MF3D_TUNE_OP_CHUNK = 15,            /* 16 (default): the FP64 operator's z-planes per
                                            workgroup, at most (1..64; fewer where the launch
                                            would have too few workgroups) */
-    MF3D_TUNE_MARCH_BLOCKS = 16         /* 2048 (default): workgroups an FP64 colour-split
+    MF3D_TUNE_MARCH_BLOCKS = 16,        /* 2048 (default): workgroups an FP64 colour-split
                                            sweep aims for (256..8192) by shortening its chunks
                                            of planes */
+    MF3D_TUNE_FUSE = 17                 /* two GSRB iterations of a large colour-split level in
+                                           one pass: 1 wherever the sizes allow, 0 never, -1
+                                           (default): on the levels where it is faster */
 };
 int mf3d_workspace_set_tuning(mf3d_workspace* ws, int key, long value);
 

@@ -20,15 +20,12 @@
 // so that fp16 keeps its range); the kernels take bs = cs * dx^2 and
 // rs = 1 / (cs * dx^2) so every result is unchanged by the scaling.
 
-#include <hip/hip_bf16.h>
-#include <hip/hip_fp16.h>
-
 #include <algorithm>
 #include <type_traits>
 
 #include "faces.hpp"
-#include "hface.hpp"
 #include "reduce.hpp"
+#include "split32.hpp"
 
 namespace mf3d {
 namespace {
@@ -51,19 +48,6 @@ __device__ __forceinline__ void cstore(__hip_bfloat16* p, long i, double v) {
     p[i] = __float2bfloat16((float)v);
 }
 __device__ __forceinline__ void cstore(__half* p, long i, double v) { p[i] = __float2half((float)v); }
-
-struct Dims {
-    int nx, ny, nz;
-    __device__ long fx(int i, int j, int k) const {
-        return (long)i + (long)(nx + 1) * ((long)j + (long)ny * k);
-    }
-    __device__ long fy(int i, int j, int k) const {
-        return (long)i + (long)nx * ((long)j + (long)(ny + 1) * k);
-    }
-    __device__ long fz(int i, int j, int k) const {
-        return (long)i + (long)nx * ((long)j + (long)ny * k);
-    }
-};
 
 __device__ __forceinline__ double bface(int t, double Kc) {
     return t == MF3D_BC_DIRICHLET ? 2.0 * Kc : 0.0;
@@ -142,26 +126,6 @@ __device__ __forceinline__ void cell_faces(const Dims& d, const TC* FX, const TC
     f[5] = (T)cload(FZ, d.fz(i, j, k));
 }
 
-// GSRB cell value (sum f x_nb - b cs dx^2) / sum f, summed x+, x-, y+, y-,
-// z+, z- as in gsrb_interior_kernel (gsrb_3d.cu:53-69); pin doubles the
-// diagonal of cell 0 (gsrb_3d.cu:360-362). The multiply-adds are written as
-// fma: the first product is rounded, each later one is fused into the running
-// sum, and b bs into the last step. Left to contraction, the compiler may
-// fuse either product of a pair depending on the code around a call, and two
-// kernels calling this would then differ in the last bit.
-template <typename T>
-__device__ __forceinline__ T gs_value(const T (&f)[6], const T (&v)[6], T b, T bs, bool pin0) {
-    T result = v[0] * f[0];
-    result = fma(v[1], f[1], result);
-    result = fma(v[2], f[2], result);
-    result = fma(v[3], f[3], result);
-    result = fma(v[4], f[4], result);
-    result = fma(v[5], f[5], result);
-    T aC = f[0] + f[1] + f[2] + f[3] + f[4] + f[5];
-    if (pin0) aC *= T(2);
-    return fma(-b, bs, result) / aC;
-}
-
 // ---- one colour of GSRB on any level -----------------------------------------
 template <typename T, typename TC, bool ZERO>
 __global__ void __launch_bounds__(kBlock)
@@ -197,32 +161,6 @@ __global__ void __launch_bounds__(kBlock)
         neighbours(d, bc, x, o, i, j, k, v);
     }
     x[o] = gs_value(f, v, b[o], bs, pin && o == 0);
-}
-
-// ---- colour-split storage of the FP32 V-cycle levels -----------------------------
-// With even nx, ny, nz a level's x and b may be stored colour by colour: the
-// cells of colour c = (i+j+k) & 1 at c*N/2 + (i >> 1) + (nx/2)(j + ny k). A
-// half-sweep then reads only the opposite colour's x and its own colour's b
-// and writes only its own colour, all with unit stride.
-// Every neighbour of a cell has the other colour: the y and z neighbours sit at
-// the same (i >> 1) one row or plane away, the x neighbours at ((i +- 1) >> 1)
-// of the same row.
-// The face coefficients of such a level are stored the same way, each face
-// with the cell on its upper side: LX/LY/LZ[split(i,j,k)] hold the faces
-// between (i-1,j,k)|(i,j,k), (i,j-1,k)|(i,j,k), (i,j,k-1)|(i,j,k) (the MAC
-// entries FX(i,j,k), FY(i,j,k), FZ(i,j,k)); the faces on the upper domain
-// boundary, owned by no cell, go to UX[j + ny k], UY[i + nx k], UZ[i + nx j]
-// (FX(nx,j,k), FY(i,ny,k), FZ(i,j,nz)). A cell's lower faces are then at its
-// own index, its upper faces at its +x/+y/+z neighbours' indices.
-struct Split {
-    int h;       // nx / 2
-    long half;   // N / 2
-    __device__ long at(const Dims& d, int i, int j, int k) const {
-        return (long)((i + j + k) & 1) * half + (long)(i >> 1) + (long)h * ((long)j + (long)d.ny * k);
-    }
-};
-__device__ __forceinline__ Split split_of(const Dims& d) {
-    return Split{d.nx >> 1, (long)(d.nx >> 1) * d.ny * d.nz};
 }
 
 // neighbours (x+, x-, y+, y-, z+, z-) of cell (i,j,k) from the opposite
@@ -266,38 +204,6 @@ __device__ __forceinline__ bool nb_coord(const Dims& d, const BcTypes& bc, int q
     }
     return true;
 }
-
-// The FP64 Krylov vectors that the mixed-precision iteration's r-update sweep
-// and x/p update touch (r, A p, x, p: 128 MiB each at 256^3) are each read or
-// written once per kernel, so they move with non-temporal loads and stores:
-// that keeps them from displacing the FP32 V-cycle's x, b and faces (224 MiB
-// at 256^3) from the 256 MB Infinity Cache between that V-cycle's
-// half-sweeps. (The (r, z) sweep's read of r measured faster without it.)
-typedef double __attribute__((ext_vector_type(2))) ntd2;
-__device__ __forceinline__ double2 ldnt(const double* p) {
-    const ntd2 v = __builtin_nontemporal_load(reinterpret_cast<const ntd2*>(p));
-    return make_double2(v.x, v.y);
-}
-__device__ __forceinline__ void stnt(double* p, double a, double b) {
-    ntd2 v;
-    v.x = a;
-    v.y = b;
-    __builtin_nontemporal_store(v, reinterpret_cast<ntd2*>(p));
-}
-
-template <typename TC>
-struct SFaces {
-    const TC* lx;
-    const TC* ly;
-    const TC* lz;
-    const TC* ux;
-    const TC* uy;
-    const TC* uz;
-};
-
-__device__ __forceinline__ float cvt(float v) { return v; }
-__device__ __forceinline__ float cvt(__hip_bfloat16 v) { return __bfloat162float(v); }
-__device__ __forceinline__ float cvt(__half v) { return __half2float(v); }
 
 // faces (x+, x-, y+, y-, z+, z-) of cell (i,j,k) of a colour-split level
 template <typename TC>

@@ -92,6 +92,29 @@ int residual_restrict_faces(hipStream_t s, const mf3d_grid& g, const BcTypes& bc
                             int corder = ORDER_NATURAL, bool red_only = false,
                             float* xcoarse = nullptr, const FaceSet* Fc = nullptr,
                             double bsc = 0.0);
+// ---- fused smoothing passes of large colour-split FP32 levels (fused32.hip) -----
+bool fused32_ok(const mf3d_grid& g, CoefType t);
+// the level's face records, made from its half-sweep faces
+size_t fused32_face_bytes(const mf3d_grid& g);
+int fused32_pack(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, const FaceSet& F,
+                 void* faces);
+// (r, z) partials of fused32_post
+unsigned fused32_partials(const mf3d_grid& g);
+// two GSRB iterations from zero: xb = the black values, bcoarse = restriction of
+// the residual's red cells. b (and bcoarse with pairs): (red, black) per place;
+// bcoarse without pairs: colour-split
+int fused32_pre(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, double bs,
+                double rs, float* xb, const float* b, CoefType t, const void* faces,
+                float* bcoarse, bool pairs);
+// x (colour-split) = two GSRB iterations from xb + the prolonged xc
+// (colour-split); rz (nullable): the (r, x) partials too
+int fused32_post(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, double bs,
+                 const float* xb, float* x, const float* b, CoefType t, const void* faces,
+                 const float* xc, const RzDot* rz);
+// b = (float) r in pairs; ru: the PCG residual update first, with the (r, r)
+// partials (one per 2048 cells)
+int r_to_b(hipStream_t s, const mf3d_grid& g, const double* r, const RUpd* ru, float* b);
+
 // FP64 operator with FP64 faces (cs = 1). mode 0: y = A x, partials (x, y);
 // mode 1: y = b - A x (y nullable), partials (y, y). It writes op_partials(g)
 // partials: one per (plane tile of 256 cells, z-chunk of kz planes).

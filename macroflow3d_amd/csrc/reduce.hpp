@@ -7,6 +7,15 @@
 
 namespace mf3d {
 
+// Workgroup barrier for data exchanged through LDS only. __syncthreads also waits
+// for the wave's global loads and stores, which would end every prefetch at
+// the barrier it is meant to cross.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // sum over a workgroup of BS threads (wave64 shuffle tree, then the waves'
 // sums in LDS); the result is valid in thread 0
 template <int BS>

@@ -82,6 +82,10 @@ struct Level {
     double* K = nullptr;    // coarsened conductivity (levels > 0)
     float* x32 = nullptr;   // FP32 V-cycle buffers
     float* b32 = nullptr;
+    bool fused = false;     // FP32 smoothing in fused passes, which use
+    float* xb = nullptr;    // the black values between pre- and post-smoothing,
+    float* b2 = nullptr;    // the right-hand side as (red, black) pairs
+    void* rec = nullptr;    // and face records
     FaceSet f64;            // FP64 faces (operator on level 0, FP64 V-cycle)
     FaceSet flo;            // low-precision faces of the FP32 V-cycle
     bool has_f64 = false;
@@ -94,6 +98,12 @@ struct Level {
     double* hs = nullptr;
     SmoothPlan plan;
 };
+
+// FP32 levels smoothed by fused passes: from 2^23 cells their tiles and z-chunks
+// occupy most of the 256 CUs (256^3: 220 workgroups, 216 us a V-cycle level for
+// 271 us of half-sweeps); a 128^3 level would have 72 workgroups of 41 planes
+// (about 100 us for 56 us of launch-bound half-sweeps).
+constexpr size_t kFuseMinCells32 = size_t(1) << 23;
 
 inline hipStream_t as_stream(mf3d_stream s) { return reinterpret_cast<hipStream_t>(s); }
 
@@ -186,6 +196,9 @@ struct mf3d_workspace {
     // rr_partials) done by the V-cycle's first finest-level half-sweep
     bool fold_r = true;
     double* rr_partials = nullptr;
+    // fused smoothing passes (MF3D_TUNE_FUSE): 1 wherever the sizes allow, 0
+    // never, -1 on levels of at least kFuseMinCells32 cells
+    int fuse = -1;
     // ... and the (r, z) partials by its last finest-level half-sweep
     bool fold_rz = true;
     size_t bytes = 0;
@@ -679,6 +692,20 @@ int mg_setup(mf3d_workspace* ws, hipStream_t s, const mf3d_grid& g, const mf3d_b
         if (!L.x32) MF3D_TRY(ws->alloc(&L.x32, L.n));
         if (!L.b32) MF3D_TRY(ws->alloc(&L.b32, L.n));
     }
+    // fused smoothing passes: V(2,2) on colour-split levels with a colour-split
+    // coarse level
+    for (size_t l = 0; l < ws->lv.size(); ++l) {
+        Level& L = ws->lv[l];
+        L.fused = mixed && ws->fuse != 0 && !defer_coarse && L.order == ORDER_SPLIT &&
+                  ws->lv[l + 1].order == ORDER_SPLIT && ws->pre == 2 && ws->post == 2 &&
+                  kern::fused32_ok(L.g, L.flo.type) &&
+                  (ws->fuse == 1 || L.n >= kFuseMinCells32);
+        if (!L.fused) continue;
+        if (!L.xb) MF3D_TRY(ws->alloc(&L.xb, L.n / 2));
+        if (!L.b2) MF3D_TRY(ws->alloc(&L.b2, L.n));
+        if (!L.rec) MF3D_TRY(ws->alloc_bytes(&L.rec, kern::fused32_face_bytes(L.g)));
+        MF3D_TRY(kern::fused32_pack(s, L.g, ws->bct, L.flo, L.rec));
+    }
     // the FP64 operator's h = 1 / (2 K): built together with the 16-bit faces
     // when level 0 is the colour-split level of the FP32 V-cycle (decided
     // above), on its own otherwise (FP64 V-cycle, a finest level too small
@@ -729,6 +756,7 @@ int build_coarse_inverses(mf3d_workspace* const* ws, int count, hipStream_t s,
 // per-type views of a level's V-cycle buffers
 template <typename T> struct LevelView;
 template <> struct LevelView<double> {
+    static bool fused(const Level&) { return false; }
     static double* x(Level& L) { return L.x; }
     static double* b(Level& L) { return L.b; }
     static const FaceSet& F(const Level& L) { return L.f64; }
@@ -736,6 +764,7 @@ template <> struct LevelView<double> {
     static int order(const Level&) { return ORDER_NATURAL; }
 };
 template <> struct LevelView<float> {
+    static bool fused(const Level& L) { return L.fused; }
     static float* x(Level& L) { return L.x32; }
     static float* b(Level& L) { return L.b32; }
     static const FaceSet& F(const Level& L) { return L.flo; }
@@ -769,6 +798,15 @@ int vcycle(mf3d_workspace* ws, hipStream_t s, size_t l, T* x, const T* b, bool z
     }
     Level& C = ws->lv[l + 1];
     const int fo = V::order(L), co = V::order(C);
+    if constexpr (std::is_same<T, float>::value) {
+        if (L.fused) {  // zero start; b is in b2
+            MF3D_TRY(kern::fused32_pre(s, L.g, ws->bct, ws->pin, cs * dx2, 1.0 / (cs * dx2), L.xb,
+                                       L.b2, F.type, L.rec, C.fused ? C.b2 : V::b(C), C.fused));
+            MF3D_TRY(vcycle<T>(ws, s, l + 1, V::x(C), V::b(C), true));
+            return kern::fused32_post(s, L.g, ws->bct, ws->pin, cs * dx2, L.xb, x, L.b2, F.type,
+                                      L.rec, V::x(C), rz);
+        }
+    }
     MF3D_TRY(kern::smooth_faces(s, L.g, ws->bct, ws->pin, cs * dx2, x, b, F, ws->pre,
                                 zero_init, (const T*)nullptr, L.plan, fo, co, r64, red_done,
                                 ru));
@@ -777,7 +815,7 @@ int vcycle(mf3d_workspace* ws, hipStream_t s, size_t l, T* x, const T* b, bool z
     // coarse level (not the coarsest) gets its first red half-sweep here too
     const bool fold = std::is_same<T, float>::value && ws->fold_first && ws->pre > 0 &&
                       fo == ORDER_SPLIT && co == ORDER_SPLIT && l + 2 < nl &&
-                      C.plan.kind == SMOOTH_COLOUR;
+                      C.plan.kind == SMOOTH_COLOUR && !V::fused(C);
     const double bsc = V::cs(C) * C.g.dx * C.g.dx;
     MF3D_TRY(kern::residual_restrict_faces(s, L.g, ws->bct, ws->pin, 1.0 / (cs * dx2), x, b, F,
                                            V::b(C), fo, co, ws->pre > 0,
@@ -826,9 +864,11 @@ bool z_in_x32(const mf3d_workspace* ws, bool flexible) {
            L0.order == ORDER_SPLIT && !(L0.g.nx & 7);
 }
 
-// partials of a finest-level split4 sweep: one per workgroup
+// (r, r) partials of the r update that rides on the first finest-level sweep:
+// one per workgroup of a split4 sweep, or of r_to_b before a fused pass
 unsigned sweep_partials(const mf3d_workspace* ws) {
     const Level& L0 = ws->lv[0];
+    if (L0.fused) return kern::reduce_blocks(L0.n);
     return (unsigned)((L0.n / 8 + L0.plan.block - 1) / L0.plan.block);
 }
 
@@ -880,14 +920,17 @@ int precondition(mf3d_workspace* ws, hipStream_t s, const double* r, double* z,
     }
     const bool fold = r_in_first_sweep(ws);
     if (ru && !fold) return fail(MF3D_ERR_UNSUPPORTED, "the r update needs the folded r sweep");
-    if (!fold) MF3D_TRY(kern::to_f32(s, r, L0.b32, L0.g, L0.order));
+    // fused passes take b as it is; the r update makes it (or the conversion)
+    const bool sweep_r = fold && !L0.fused;
+    if (L0.fused) MF3D_TRY(kern::r_to_b(s, L0.g, r, ru, L0.b2));
+    else if (!sweep_r) MF3D_TRY(kern::to_f32(s, r, L0.b32, L0.g, L0.order));
     // the last finest half-sweep forms (r, z): z in x32, post-smoothing on level 0
     const bool rz_fold = !z && rz_partials && ws->fold_rz && ws->post > 0 && fold;
     const RzDot rzd{r, rz_partials};
-    MF3D_TRY(vcycle<float>(ws, s, 0, L0.x32, L0.b32, true, fold ? r : nullptr, false, ru,
-                           rz_fold ? &rzd : nullptr));
+    MF3D_TRY(vcycle<float>(ws, s, 0, L0.x32, L0.b32, true, sweep_r ? r : nullptr, false,
+                           sweep_r ? ru : nullptr, rz_fold ? &rzd : nullptr));
     if (rz_fold) {
-        if (np_rz) *np_rz = sweep_partials(ws);
+        if (np_rz) *np_rz = L0.fused ? kern::fused32_partials(L0.g) : sweep_partials(ws);
         return MF3D_OK;
     }
     if (!z) return rz_partials ? kern::rz_split8(s, L0.x32, L0.g, r, rz_partials) : MF3D_OK;
@@ -2055,6 +2098,10 @@ int mf3d_workspace_set_tuning(mf3d_workspace* ws, int key, long value) {
         if (value < kern::kMarchMinBlocks || value > kern::kMarchMaxBlocks)
             return fail(MF3D_ERR_INVALID_ARGUMENT, "march workgroup target must be 256..8192");
         ws->march_blocks = value;
+        break;
+    case MF3D_TUNE_FUSE:
+        if (value < -1 || value > 1) return fail(MF3D_ERR_INVALID_ARGUMENT, "fuse must be -1, 0 or 1");
+        ws->fuse = (int)value;
         break;
     case MF3D_TUNE_GRAPH:
         if (value < -1 || value > 1) return fail(MF3D_ERR_INVALID_ARGUMENT, "graph must be -1, 0 or 1");

@@ -188,6 +188,7 @@ class FlowWorkspace:
     TUNE_GRAPH = 14
     TUNE_OP_CHUNK = 15
     TUNE_MARCH_BLOCKS = 16
+    TUNE_FUSE = 17
 
     def set_tuning(self, key: int, value: int) -> None:
         """Kernel-layout knobs (colour-split storage, sweep workgroup size,
