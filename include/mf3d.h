@@ -256,8 +256,9 @@ enum {
                                            sweep aims for (256..8192) by shortening its chunks
                                            of planes */
     MF3D_TUNE_FUSE = 17                 /* two GSRB iterations of a large colour-split level in
-                                           one pass: 1 wherever the sizes allow, 0 never, -1
-                                           (default): on the levels where it is faster */
+                                           one pass: 1 wherever the sizes allow, 0 never (nor
+                                           in windows of a small one), -1 (default): on the
+                                           levels where it is faster */
 };
 int mf3d_workspace_set_tuning(mf3d_workspace* ws, int key, long value);
 

@@ -35,13 +35,6 @@ inline unsigned grid_for(size_t n) { return (unsigned)((n + kBlock - 1) / kBlock
 // grid of a 1-D launch remapped by xcd_block: padded to a multiple of 8 blocks
 inline unsigned xcd_grid(size_t n) { return xcd_round(grid_for(n)); }
 
-// ---- coefficient storage conversions ---------------------------------------
-__device__ __forceinline__ double cload(const double* p, long i) { return p[i]; }
-__device__ __forceinline__ float cload(const float* p, long i) { return p[i]; }
-__device__ __forceinline__ float cload(const __hip_bfloat16* p, long i) {
-    return __bfloat162float(p[i]);
-}
-__device__ __forceinline__ float cload(const __half* p, long i) { return __half2float(p[i]); }
 __device__ __forceinline__ void cstore(double* p, long i, double v) { p[i] = v; }
 __device__ __forceinline__ void cstore(float* p, long i, double v) { p[i] = (float)v; }
 __device__ __forceinline__ void cstore(__hip_bfloat16* p, long i, double v) {
@@ -113,17 +106,6 @@ __device__ __forceinline__ void neighbours(const Dims& d, const BcTypes& bc, con
     v[3] = j > 0 ? x[o - sy] : (bc.t[2] == MF3D_BC_PERIODIC ? x[o + (long)(d.ny - 1) * sy] : T(0));
     v[4] = k < d.nz - 1 ? x[o + sz] : (bc.t[5] == MF3D_BC_PERIODIC ? x[o - (long)(d.nz - 1) * sz] : T(0));
     v[5] = k > 0 ? x[o - sz] : (bc.t[4] == MF3D_BC_PERIODIC ? x[o + (long)(d.nz - 1) * sz] : T(0));
-}
-
-template <typename T, typename TC>
-__device__ __forceinline__ void cell_faces(const Dims& d, const TC* FX, const TC* FY,
-                                           const TC* FZ, int i, int j, int k, T (&f)[6]) {
-    f[0] = (T)cload(FX, d.fx(i + 1, j, k));
-    f[1] = (T)cload(FX, d.fx(i, j, k));
-    f[2] = (T)cload(FY, d.fy(i, j + 1, k));
-    f[3] = (T)cload(FY, d.fy(i, j, k));
-    f[4] = (T)cload(FZ, d.fz(i, j, k + 1));
-    f[5] = (T)cload(FZ, d.fz(i, j, k));
 }
 
 // ---- one colour of GSRB on any level -----------------------------------------
@@ -203,20 +185,6 @@ __device__ __forceinline__ bool nb_coord(const Dims& d, const BcTypes& bc, int q
     default: if (--k < 0) { if (bc.t[4] != MF3D_BC_PERIODIC) return false; k = d.nz - 1; } break;
     }
     return true;
-}
-
-// faces (x+, x-, y+, y-, z+, z-) of cell (i,j,k) of a colour-split level
-template <typename TC>
-__device__ __forceinline__ void cell_faces_split(const Dims& d, const Split& sp,
-                                                 const SFaces<TC>& F, int i, int j, int k,
-                                                 float (&f)[6]) {
-    const long own = sp.at(d, i, j, k);
-    f[1] = cvt(F.lx[own]);
-    f[3] = cvt(F.ly[own]);
-    f[5] = cvt(F.lz[own]);
-    f[0] = i < d.nx - 1 ? cvt(F.lx[sp.at(d, i + 1, j, k)]) : cvt(F.ux[j + (long)d.ny * k]);
-    f[2] = j < d.ny - 1 ? cvt(F.ly[sp.at(d, i, j + 1, k)]) : cvt(F.uy[i + (long)d.nx * k]);
-    f[4] = k < d.nz - 1 ? cvt(F.lz[sp.at(d, i, j, k + 1)]) : cvt(F.uz[i + (long)d.nx * j]);
 }
 
 // adds the parent coarse value to each in-domain neighbour value (MODE 2)

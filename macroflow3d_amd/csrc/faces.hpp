@@ -115,6 +115,36 @@ int fused32_post(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin,
 // partials (one per 2048 cells)
 int r_to_b(hipStream_t s, const mf3d_grid& g, const double* r, const RUpd* ru, float* b);
 
+// ---- fused smoothing of small levels (block.hip) --------------------------------
+// One launch of `iters` (1 or 2) GSRB iterations on a level of any storage.
+// xin null: zero start; else from xin (a buffer other than xout), plus the
+// prolonged xc when given. bcoarse: also the restricted residual (after a zero
+// start, or one iteration). z: the result in natural order there instead of xout,
+// with block_windows(g) partials of (r, z) when partials is given.
+template <typename T>
+struct BlockPass {
+    int iters;
+    double bs, rs;
+    const T* xin;
+    T* xout;
+    const T* b;
+    const T* xc;
+    T* bcoarse;
+    int corder;  // storage order of xc / bcoarse
+    double* z;
+    const double* r;
+    double* partials;
+};
+unsigned block_windows(const mf3d_grid& g);
+int block_pass(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, const FaceSet& F,
+               const BlockPass<float>& p);
+// hs: colour-split level with faces from h, else natural order with FP64 faces F
+int block_pass(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, const FaceSet& F,
+               const double* hs, const BlockPass<double>& p);
+// b = r in colour-split order; ru: r -= alpha Ap first, with the (r, r) partials
+// (one per 2048 cells)
+int r_to_split64(hipStream_t s, const mf3d_grid& g, const double* r, const RUpd* ru, double* b);
+
 // FP64 operator with FP64 faces (cs = 1). mode 0: y = A x, partials (x, y);
 // mode 1: y = b - A x (y nullable), partials (y, y). It writes op_partials(g)
 // partials: one per (plane tile of 256 cells, z-chunk of kz planes).

@@ -82,6 +82,11 @@ struct Level {
     double* K = nullptr;    // coarsened conductivity (levels > 0)
     float* x32 = nullptr;   // FP32 V-cycle buffers
     float* b32 = nullptr;
+    // smoothing of a small level in window passes, which read one x and write
+    // another (block.hip)
+    bool block = false;
+    double* x2 = nullptr;
+    float* x32s = nullptr;
     bool fused = false;     // FP32 smoothing in fused passes, which use
     float* xb = nullptr;    // the black values between pre- and post-smoothing,
     float* b2 = nullptr;    // the right-hand side as (red, black) pairs
@@ -99,6 +104,11 @@ struct Level {
     SmoothPlan plan;
 };
 
+// Levels of at most so many 8^3 windows are smoothed by window passes: two FP32
+// workgroups fit a CU, so 512 are one wave (64^3: 19 us a V(2,2) level for 36 of
+// half-sweeps); FP64 ones fit once, and 512 are two waves (72x56x40, 315
+// windows: 36 us for 42; 64^3 takes the same 36). Another wave would cost what the launches do.
+constexpr size_t kBlockMaxWindows32 = 512, kBlockMaxWindows64 = 512;
 // FP32 levels smoothed by fused passes: from 2^23 cells their tiles and z-chunks
 // occupy most of the 256 CUs (256^3: 220 workgroups, 216 us a V-cycle level for
 // 271 us of half-sweeps); a 128^3 level would have 72 workgroups of 41 planes
@@ -340,7 +350,7 @@ int ensure_workspace(mf3d_workspace* ws, const mf3d_grid& g, int levels) {
     const size_t march_cap =
         (size_t)kern::kMarchMaxBlocks + ((size_t)g.nx * g.ny / 4 + 63) / 64;
     ws->partials_cap = std::max<size_t>({kern::reduce_blocks(n), kern::op_partials(g), n / 256,
-                                         march_cap}) + 64;
+                                         march_cap, kBlockMaxWindows64}) + 64;
     MF3D_TRY(ws->alloc(&ws->partials, ws->partials_cap));
     // one per workgroup of the finest sweep (8 cells per thread, >= 64 threads;
     // FP64: one per march workgroup)
@@ -706,6 +716,17 @@ int mg_setup(mf3d_workspace* ws, hipStream_t s, const mf3d_grid& g, const mf3d_b
         if (!L.rec) MF3D_TRY(ws->alloc_bytes(&L.rec, kern::fused32_face_bytes(L.g)));
         MF3D_TRY(kern::fused32_pack(s, L.g, ws->bct, L.flo, L.rec));
     }
+    // window passes on small levels (the batched solve has its own launches, whose
+    // (r, z) grouping the FP32 finest level shares)
+    for (size_t l = 0; l < ws->lv.size(); ++l) {
+        Level& L = ws->lv[l];
+        L.block = ws->fuse != 0 && !defer_coarse && l + 1 < ws->lv.size() && ws->pre > 0 &&
+                  ws->post > 0 && !L.fused && (!mixed || l > 0) &&
+                  kern::block_windows(L.g) <= (mixed ? kBlockMaxWindows32 : kBlockMaxWindows64);
+        if (!L.block) continue;
+        if (mixed && !L.x32s) MF3D_TRY(ws->alloc(&L.x32s, L.n));
+        if (!mixed && !L.x2) MF3D_TRY(ws->alloc(&L.x2, L.n));
+    }
     // the FP64 operator's h = 1 / (2 K): built together with the 16-bit faces
     // when level 0 is the colour-split level of the FP32 V-cycle (decided
     // above), on its own otherwise (FP64 V-cycle, a finest level too small
@@ -756,7 +777,7 @@ int build_coarse_inverses(mf3d_workspace* const* ws, int count, hipStream_t s,
 // per-type views of a level's V-cycle buffers
 template <typename T> struct LevelView;
 template <> struct LevelView<double> {
-    static bool fused(const Level&) { return false; }
+    static double* x2(Level& L) { return L.x2; }
     static double* x(Level& L) { return L.x; }
     static double* b(Level& L) { return L.b; }
     static const FaceSet& F(const Level& L) { return L.f64; }
@@ -764,13 +785,20 @@ template <> struct LevelView<double> {
     static int order(const Level&) { return ORDER_NATURAL; }
 };
 template <> struct LevelView<float> {
-    static bool fused(const Level& L) { return L.fused; }
+    static float* x2(Level& L) { return L.x32s; }
     static float* x(Level& L) { return L.x32; }
     static float* b(Level& L) { return L.b32; }
     static const FaceSet& F(const Level& L) { return L.flo; }
     static double cs(const Level& L) { return L.cs; }
     static int order(const Level& L) { return L.order; }
 };
+
+int vcycle64(mf3d_workspace* ws, hipStream_t s, size_t l, bool zero_init, const double* r64,
+             double* z, const double* rdot, double* partials, unsigned* np,
+             const RUpd* ru = nullptr);
+template <typename T>
+int vcycle_block(mf3d_workspace* ws, hipStream_t s, size_t l, T* x, const T* b,
+                 double* z = nullptr, const double* rdot = nullptr, double* partials = nullptr);
 
 // v_cycle_recursive (src/multigrid/cycle/v_cycle.cu:36-74) in precision T.
 // zero_init: x is zero on entry (the fills of v_cycle.cu:62 and
@@ -796,6 +824,7 @@ int vcycle(mf3d_workspace* ws, hipStream_t s, size_t l, T* x, const T* b, bool z
         return kern::smooth_faces(s, L.g, ws->bct, ws->pin, cs * dx2, x, b, F,
                                   ws->coarse_iters, zero_init, (const T*)nullptr, L.plan);
     }
+    if (L.block && zero_init) return vcycle_block<T>(ws, s, l, x, b);
     Level& C = ws->lv[l + 1];
     const int fo = V::order(L), co = V::order(C);
     if constexpr (std::is_same<T, float>::value) {
@@ -815,7 +844,7 @@ int vcycle(mf3d_workspace* ws, hipStream_t s, size_t l, T* x, const T* b, bool z
     // coarse level (not the coarsest) gets its first red half-sweep here too
     const bool fold = std::is_same<T, float>::value && ws->fold_first && ws->pre > 0 &&
                       fo == ORDER_SPLIT && co == ORDER_SPLIT && l + 2 < nl &&
-                      C.plan.kind == SMOOTH_COLOUR && !V::fused(C);
+                      C.plan.kind == SMOOTH_COLOUR && !C.fused && !C.block;
     const double bsc = V::cs(C) * C.g.dx * C.g.dx;
     MF3D_TRY(kern::residual_restrict_faces(s, L.g, ws->bct, ws->pin, 1.0 / (cs * dx2), x, b, F,
                                            V::b(C), fo, co, ws->pre > 0,
@@ -835,11 +864,15 @@ int vcycle(mf3d_workspace* ws, hipStream_t s, size_t l, T* x, const T* b, bool z
 // the last half-sweep writes the result there in natural order (with the
 // (rdot, z) partials when rdot is given) instead of into the split x.
 int vcycle64(mf3d_workspace* ws, hipStream_t s, size_t l, bool zero_init, const double* r64,
-             double* z, const double* rdot, double* partials, unsigned* np,
-             const RUpd* ru = nullptr) {
+             double* z, const double* rdot, double* partials, unsigned* np, const RUpd* ru) {
     Level& L = ws->lv[l];
     Level& C = ws->lv[l + 1];  // a split level is never the coarsest
     const double dx2 = L.g.dx * L.g.dx;
+    if (L.block && zero_init) {
+        if (r64) MF3D_TRY(kern::r_to_split64(s, L.g, r64, ru, L.b));
+        if (np) *np = kern::block_windows(L.g);
+        return vcycle_block<double>(ws, s, l, L.x, L.b, z, rdot, rdot ? partials : nullptr);
+    }
     const int tb = L.plan.block;
     MF3D_TRY(kern::smooth_split64(s, L.g, ws->bct, ws->pin, dx2, L.x, L.b, L.hs, ws->pre,
                                   zero_init, nullptr, ORDER_NATURAL, tb, r64, nullptr, nullptr,
@@ -853,6 +886,79 @@ int vcycle64(mf3d_workspace* ws, hipStream_t s, size_t l, bool zero_init, const 
     return kern::smooth_split64(s, L.g, ws->bct, ws->pin, dx2, L.x, L.b, L.hs, ws->post, false,
                                 C.x, C.order64, tb, nullptr, z, rdot, partials, np,
                                 ws->march_blocks);
+}
+
+// The V-cycle from a small level l whose x starts at zero (v_cycle.cu:36-74) in
+// window passes of up to two iterations each, alternating between x and the
+// level's second buffer so that the last one leaves its result in x (or, in
+// natural order with the (rdot, z) partials, in z). The restriction rides on the
+// last pre-smoothing pass where its window allows (from zero, or one iteration).
+template <typename T>
+int vcycle_block(mf3d_workspace* ws, hipStream_t s, size_t l, T* x, const T* b, double* z,
+                 const double* rdot, double* partials) {
+    using V = LevelView<T>;
+    constexpr bool F64 = std::is_same<T, double>::value;
+    Level& L = ws->lv[l];
+    Level& C = ws->lv[l + 1];
+    const double dx2 = L.g.dx * L.g.dx, cs = V::cs(L);
+    const bool split = F64 ? L.order64 == ORDER_SPLIT : L.order == ORDER_SPLIT;
+    const int co = F64 ? C.order64 : C.order;
+    const int npre = (ws->pre + 1) / 2, npost = (ws->post + 1) / 2;
+    int left = npre + npost;
+    T* cur = nullptr;
+    kern::BlockPass<T> p{};
+    p.bs = cs * dx2, p.rs = 1.0 / (cs * dx2);
+    p.b = b;
+    p.corder = co;
+    auto pass = [&](int iters) -> int {
+        --left;
+        p.iters = iters;
+        p.xin = cur;
+        p.xout = left % 2 ? V::x2(L) : x;
+        cur = p.xout;
+        if constexpr (F64)
+            return kern::block_pass(s, L.g, ws->bct, ws->pin, L.f64, split ? L.hs : nullptr, p);
+        else
+            return kern::block_pass(s, L.g, ws->bct, ws->pin, L.flo, p);
+    };
+    bool restricted = false;
+    for (int q = 0, done = 0; q < npre; ++q) {
+        const int it = std::min(2, ws->pre - done);
+        done += it;
+        restricted = q == npre - 1 && (q == 0 || it == 1);
+        p.bcoarse = restricted ? V::b(C) : nullptr;
+        MF3D_TRY(pass(it));
+    }
+    p.bcoarse = nullptr;
+    if (!restricted) {
+        if constexpr (F64) {
+            if (split)
+                MF3D_TRY(kern::residual_restrict_split64(s, L.g, ws->bct, ws->pin, p.rs, cur, b,
+                                                         L.hs, C.b, co, true));
+            else
+                MF3D_TRY(kern::residual_restrict_faces(s, L.g, ws->bct, ws->pin, p.rs, cur, b,
+                                                       L.f64, C.b));
+        } else {
+            MF3D_TRY(kern::residual_restrict_faces(s, L.g, ws->bct, ws->pin, p.rs, cur, b, L.flo,
+                                                   V::b(C), L.order, co, true));
+        }
+    }
+    if constexpr (F64) {
+        if (co == ORDER_SPLIT)
+            MF3D_TRY(vcycle64(ws, s, l + 1, true, nullptr, nullptr, nullptr, nullptr, nullptr));
+        else
+            MF3D_TRY(vcycle<double>(ws, s, l + 1, C.x, C.b, true));
+    } else {
+        MF3D_TRY(vcycle<T>(ws, s, l + 1, V::x(C), V::b(C), true));
+    }
+    for (int q = 0, done = 0; q < npost; ++q) {
+        const int it = std::min(2, ws->post - done);
+        done += it;
+        p.xc = q == 0 ? V::x(C) : nullptr;
+        if (q == npost - 1) p.z = z, p.r = rdot, p.partials = partials;
+        MF3D_TRY(pass(it));
+    }
+    return MF3D_OK;
 }
 
 // PCG may leave z = x32 unstored (the (r, z) partials and the p update read the
@@ -1050,8 +1156,9 @@ int run_pcg(mf3d_workspace* ws, hipStream_t s, const mf3d_grid& g,
     const bool fuse64 = !flexible && ws->fold_r && r_in_first_sweep64(ws);
     const bool fuse_r = (zx && ws->fold_r && r_in_first_sweep(ws)) || fuse64;
     const unsigned np_sweep =
-        fuse64 ? kern::split64_partials(L0.g, L0.plan.block, ws->march_blocks)
-               : sweep_partials(ws);
+        !fuse64    ? sweep_partials(ws)
+        : L0.block ? kern::reduce_blocks(n)
+                   : kern::split64_partials(L0.g, L0.plan.block, ws->march_blocks);
     unsigned nprz = 0;  // (r, z) partials of the last preconditioner application
     // the reference's own rule (||r||/||r0||, FP64) keeps its exact semantics
     const bool true_check =

@@ -23,6 +23,14 @@ struct Dims {
     }
 };
 
+// ---- coefficient storage conversions ---------------------------------------
+__device__ __forceinline__ double cload(const double* p, long i) { return p[i]; }
+__device__ __forceinline__ float cload(const float* p, long i) { return p[i]; }
+__device__ __forceinline__ float cload(const __hip_bfloat16* p, long i) {
+    return __bfloat162float(p[i]);
+}
+__device__ __forceinline__ float cload(const __half* p, long i) { return __half2float(p[i]); }
+
 // GSRB cell value (sum f x_nb - b cs dx^2) / sum f, summed x+, x-, y+, y-,
 // z+, z- as in gsrb_interior_kernel (gsrb_3d.cu:53-69); pin doubles the
 // diagonal of cell 0 (gsrb_3d.cu:360-362). The multiply-adds are written as
@@ -50,6 +58,18 @@ __device__ __forceinline__ T gs_value(const T (&f)[6], const T (&v)[6], T b, T b
     T aC = f[0] + f[1] + f[2] + f[3] + f[4] + f[5];
     if (pin0) aC *= T(2);
     return gs_quot(fma(-b, bs, result), aC);
+}
+
+// faces (x+, x-, y+, y-, z+, z-) of cell (i,j,k) of a natural-order level
+template <typename T, typename TC>
+__device__ __forceinline__ void cell_faces(const Dims& d, const TC* FX, const TC* FY,
+                                           const TC* FZ, int i, int j, int k, T (&f)[6]) {
+    f[0] = (T)cload(FX, d.fx(i + 1, j, k));
+    f[1] = (T)cload(FX, d.fx(i, j, k));
+    f[2] = (T)cload(FY, d.fy(i, j + 1, k));
+    f[3] = (T)cload(FY, d.fy(i, j, k));
+    f[4] = (T)cload(FZ, d.fz(i, j, k + 1));
+    f[5] = (T)cload(FZ, d.fz(i, j, k));
 }
 
 // ---- colour-split storage of the FP32 V-cycle levels -----------------------------
@@ -109,5 +129,19 @@ struct SFaces {
 __device__ __forceinline__ float cvt(float v) { return v; }
 __device__ __forceinline__ float cvt(__hip_bfloat16 v) { return __bfloat162float(v); }
 __device__ __forceinline__ float cvt(__half v) { return __half2float(v); }
+
+// faces (x+, x-, y+, y-, z+, z-) of cell (i,j,k) of a colour-split level
+template <typename TC>
+__device__ __forceinline__ void cell_faces_split(const Dims& d, const Split& sp,
+                                                 const SFaces<TC>& F, int i, int j, int k,
+                                                 float (&f)[6]) {
+    const long own = sp.at(d, i, j, k);
+    f[1] = cvt(F.lx[own]);
+    f[3] = cvt(F.ly[own]);
+    f[5] = cvt(F.lz[own]);
+    f[0] = i < d.nx - 1 ? cvt(F.lx[sp.at(d, i + 1, j, k)]) : cvt(F.ux[j + (long)d.ny * k]);
+    f[2] = j < d.ny - 1 ? cvt(F.ly[sp.at(d, i, j + 1, k)]) : cvt(F.uy[i + (long)d.nx * k]);
+    f[4] = k < d.nz - 1 ? cvt(F.lz[sp.at(d, i, j, k + 1)]) : cvt(F.uz[i + (long)d.nx * j]);
+}
 
 }  // namespace mf3d

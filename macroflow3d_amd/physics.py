@@ -193,7 +193,8 @@ class FlowWorkspace:
     def set_tuning(self, key: int, value: int) -> None:
         """Kernel-layout knobs (colour-split storage, sweep workgroup size,
         folded PCG steps, plane-tile operator and its chunk depth, the FP64
-        sweeps' workgroup target, graph replay); applied at the next set-up
+        sweeps' workgroup target, graph replay, fused smoothing passes);
+        applied at the next set-up
         or solve. None changes the result beyond rounding; the sweep block
         size of the mixed V-cycle and the graph replay leave it bit-identical,
         the operator tile and chunk depth regroup the (p, Ap) partials, the

@@ -1,0 +1,91 @@
+"""Window passes of the V-cycle's small levels (block.hip) against the half-sweep
+kernels they replace, at sizes whose windows end unevenly, wrap onto themselves or
+leave the window mostly empty, for every boundary mix and smoothing count."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import BC_MIXES, bc_pair, random_K, rel_l2
+from macroflow3d_amd import numerics as nm
+from macroflow3d_amd import physics as ph
+from macroflow3d_amd.core import Grid3D
+from macroflow3d_amd.kfield import lognormal_lnK
+
+pytestmark = pytest.mark.gpu
+
+F32 = ph.PrecondPrecision.FP32
+# finest shape, levels: natural and colour-split levels below and at the top, one
+# window and many, axes of 2 and 4 cells under a periodic window of 16
+SHAPES = [((16, 16, 16), 2), ((48, 32, 16), 3), ((80, 48, 32), 4), ((136, 16, 8), 3),
+          ((24, 8, 112), 3), ((104, 56, 40), 4)]
+COUNTS = [(2, 2), (1, 1), (3, 2), (4, 5)]
+
+
+def _apply(ctx, shape, levels, mix, counts, precision, fuse, coef=ph.CoefFormat.BF16):
+    g = Grid3D(*shape)
+    bc, _ = bc_pair(mix)
+    n = g.num_cells()
+    K = torch.as_tensor(random_K(n, 51)).to(ctx.device)
+    r = torch.as_tensor(np.random.default_rng(52).standard_normal(n)).to(ctx.device)
+    # the direct coarsest solve: GSRB has no fixed order on odd periodic axes
+    cfg = ph.HeadSolveConfig.fp64_direct(1e-10, levels)
+    cfg.precond_precision, cfg.coef_format = precision, coef
+    cfg.mg_pre_smooth, cfg.mg_post_smooth = counts
+    ws = ph.FlowWorkspace()
+    ws.set_tuning(ph.FlowWorkspace.TUNE_FUSE, fuse)
+    M = nm.MultigridPreconditioner.build(ctx, ws, g, bc, cfg, K)
+    out = ctx.empty(n)
+    M.apply(ctx, r, out)
+    ctx.synchronize()
+    ws.close()
+    return out
+
+
+@pytest.mark.parametrize("counts", COUNTS)
+@pytest.mark.parametrize("mix", list(BC_MIXES))
+@pytest.mark.parametrize("shape,levels", SHAPES)
+def test_fp32_window_passes_equal_half_sweeps(ctx, shape, levels, mix, counts):
+    """The FP32 sums are the same, in the same order: bit for bit."""
+    coef = ph.CoefFormat.FP16 if counts == (1, 1) else ph.CoefFormat.BF16
+    z = [_apply(ctx, shape, levels, mix, counts, F32, fuse, coef) for fuse in (0, -1)]
+    assert torch.isfinite(z[1]).all()
+    assert torch.equal(z[0], z[1])
+
+
+@pytest.mark.parametrize("counts", COUNTS)
+@pytest.mark.parametrize("mix", list(BC_MIXES))
+@pytest.mark.parametrize("shape,levels", SHAPES)
+def test_fp64_window_passes_match_half_sweeps(ctx, shape, levels, mix, counts):
+    """FP64 differs by the order of the x terms and the quotients' last bit: some
+    1e-16 a cell and half-sweep, times the coarsest system's condition (< 1e4)."""
+    z = [_apply(ctx, shape, levels, mix, counts, ph.PrecondPrecision.FP64, fuse).cpu().numpy()
+         for fuse in (0, -1)]
+    assert np.isfinite(z[1]).all()
+    assert rel_l2(z[1], z[0]) < 1e-11
+
+
+@pytest.mark.parametrize("graph", [0, 1])
+@pytest.mark.parametrize("fold_r", [0, 1])
+@pytest.mark.parametrize("shape", [(32, 32, 32), (40, 56, 24)])
+def test_fp64_solve_on_window_passes(ctx, shape, fold_r, graph):
+    """The solve around them: r update, (r, r) and (r, z) grouped differently, so
+    heads equal to the stopping tolerance's rounding and equal iterations."""
+    g = Grid3D(*shape)
+    bc, _ = bc_pair("darcy_x")
+    K = torch.exp(lognormal_lnK(*shape, 2.0, 5.0, 41, device=ctx.device)[0])
+    heads, its = [], []
+    for fuse in (0, -1):
+        ws = ph.FlowWorkspace()
+        ws.set_tuning(ph.FlowWorkspace.TUNE_FUSE, fuse)
+        ws.set_tuning(ph.FlowWorkspace.TUNE_FOLD_R, fold_r)
+        ws.set_tuning(ph.FlowWorkspace.TUNE_GRAPH, graph)
+        h = ctx.zeros(g.num_cells())
+        res = ph.solve_head(h, K, g, bc, ph.HeadSolveConfig.fp64_direct(1e-10, 3), ctx, ws)
+        assert res.converged and res.true_residual <= 1e-10 * res.bnorm
+        heads.append(h.cpu().numpy())
+        its.append(res.num_iterations)
+        ws.close()
+    assert its[0] == its[1]
+    assert rel_l2(heads[1], heads[0]) < 1e-11
