@@ -183,19 +183,6 @@ struct Split64 {  // FP64 colour-split level, faces from h
     }
 };
 
-// n / d from the reciprocal estimate r of d, corrected once by the remainder, with
-// the hardware's fix-up for zeros and infinities (FP32: gs_quot)
-__device__ __forceinline__ float recip_of(float d) { return __builtin_amdgcn_rcpf(d); }
-__device__ __forceinline__ double recip_of(double d) { return rcp_nr(d); }
-__device__ __forceinline__ float quot_by(float n, float d, float r) {
-    const float q = n * r;
-    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, d, n), r, q), d, n);
-}
-__device__ __forceinline__ double quot_by(double n, double d, double r) {
-    const double q = n * r;
-    return __builtin_amdgcn_div_fixup(fma(fma(-q, d, n), r, q), d, n);
-}
-
 template <typename T>
 struct BArgs {
     BcTypes bc;

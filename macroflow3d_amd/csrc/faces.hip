@@ -655,66 +655,91 @@ __global__ void __launch_bounds__(kBlock)
 constexpr int kSmallBlock = 1024;
 constexpr int kSmallPer = 4;
 
-// Thread t owns cells o = 2t + (m & 1) + 2048 (m >> 1), m = 0..3: two
-// x-adjacent pairs, one cell of each colour per pair when nx is even, so every
-// lane has work in every half-sweep. The neighbours' LDS slots (-1 for a
-// non-periodic boundary, whose ghost value is 0), the faces and b are
-// gathered once; the iterations then touch LDS only. Per cell the same sums
-// as colour_kernel (neighbours x+, x-, y+, y-, z+, z-; gs_value).
+// Bound: a half-sweep of one workgroup is a barrier, an LDS round trip and a chain
+// of six multiply-adds and a quotient; 50 coarsest iterations are 100 of them in
+// a row. Thread t owns the pairs (2q, 2q + 1) of the linear order, q = t and t +
+// 1024: whatever the sizes, a pair holds one cell of each colour (in a row of even
+// nx; with odd nx the colours alternate along the linear order up to the end of a
+// plane, and an even ny ends planes on whole pairs), so every lane works in every
+// half-sweep without divergence. x is kept in LDS colour by colour (slot 2048
+// colour + q), where the neighbours of consecutive cells are consecutive. The
+// neighbours' slots (one that holds 0, the ghost value, beyond a non-periodic
+// boundary), the faces, b, the diagonal and its reciprocal are gathered once. Per
+// cell the sums are colour_kernel's (neighbours x+, x-, y+, y-, z+, z-; gs_value).
+// MI355X, 50 FP64 iterations of 18x14x10: 77 us with the pair's cells taken in
+// linear order (each half-sweep ran both under half the lanes) and a division per
+// update, 30 us now.
+constexpr int kSmallSlots = kSmallBlock * kSmallPer + 1;  // the last one holds 0
 template <typename T, typename TC>
 __device__ __forceinline__ void small_body(T* xs, const Dims& d, const BcTypes& bc, int pin, T bs,
                                            T* __restrict__ x, const T* __restrict__ b,
                                            const TC* __restrict__ FX, const TC* __restrict__ FY,
                                            const TC* __restrict__ FZ, int iters, int zero_init,
                                            const T* __restrict__ xc) {
+    constexpr int kS = kSmallPer / 2, kHalf = kSmallBlock * kS;
     const int nx = d.nx, ny = d.ny, nz = d.nz;
     const int n = nx * ny * nz;
-    const long sy = nx, sz = (long)nx * ny;
-    T f[kSmallPer][6], bl[kSmallPer];
-    int nb[kSmallPer][6];
-    int colour[kSmallPer];  // -1: no cell
     const int NXc = nx >> 1, NYc = ny >> 1;
+    T f[kS][2][6], bl[kS][2], dg[kS][2], rd[kS][2];
+    int nb[kS][2][6], own[kS][2];  // own cell (-1: none); its slot is own_slot(s, c)
+    auto own_slot = [&](int s, int c) { return c * kHalf + (int)threadIdx.x + s * kSmallBlock; };
+    if (threadIdx.x == 0) xs[2 * kHalf] = T(0);
 #pragma unroll
-    for (int m = 0; m < kSmallPer; ++m) {
-        const int o = 2 * (int)threadIdx.x + (m & 1) + 2 * kSmallBlock * (m >> 1);
-        bl[m] = T(0);
-        colour[m] = -1;
-        if (o < n) {
-            const int i = o % nx, q = o / nx, j = q % ny, k = q / ny;
-            colour[m] = (i + j + k) & 1;
+    for (int s = 0; s < kS; ++s) {
+        const int o0 = 2 * ((int)threadIdx.x + s * kSmallBlock);
+        const int q0 = o0 / nx, a = (o0 - q0 * nx + q0 % ny + q0 / ny) & 1;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int o = o0 + (c ^ a);
+            own[s][c] = o < n ? o : -1;
+            if (o >= n) continue;
+            const int q = o / nx, i = o - q * nx, k = q / ny, j = q - k * ny;
             T v = zero_init ? T(0) : x[o];
             if (xc) v += xc[(i >> 1) + NXc * ((j >> 1) + NYc * (k >> 1))];
-            xs[o] = v;
-            cell_faces(d, FX, FY, FZ, i, j, k, f[m]);
-            bl[m] = b[o];
-            nb[m][0] = i < nx - 1 ? o + 1 : (bc.t[1] == MF3D_BC_PERIODIC ? o - (nx - 1) : -1);
-            nb[m][1] = i > 0 ? o - 1 : (bc.t[0] == MF3D_BC_PERIODIC ? o + (nx - 1) : -1);
-            nb[m][2] = j < ny - 1 ? (int)(o + sy)
-                                  : (bc.t[3] == MF3D_BC_PERIODIC ? (int)(o - (ny - 1) * sy) : -1);
-            nb[m][3] = j > 0 ? (int)(o - sy)
-                             : (bc.t[2] == MF3D_BC_PERIODIC ? (int)(o + (ny - 1) * sy) : -1);
-            nb[m][4] = k < nz - 1 ? (int)(o + sz)
-                                  : (bc.t[5] == MF3D_BC_PERIODIC ? (int)(o - (nz - 1) * sz) : -1);
-            nb[m][5] = k > 0 ? (int)(o - sz)
-                             : (bc.t[4] == MF3D_BC_PERIODIC ? (int)(o + (nz - 1) * sz) : -1);
+            xs[own_slot(s, c)] = v;
+            cell_faces(d, FX, FY, FZ, i, j, k, f[s][c]);
+            bl[s][c] = b[o];
+            const int pos[3] = {i, j, k}, lim[3] = {nx, ny, nz}, st[3] = {1, nx, nx * ny};
+#pragma unroll
+            for (int e = 0; e < 6; ++e) {  // x+, x-, y+, y-, z+, z-
+                const int ax = e >> 1, up = !(e & 1);
+                const bool in = up ? pos[ax] < lim[ax] - 1 : pos[ax] > 0;
+                const int off = in ? st[ax] : -(lim[ax] - 1) * st[ax];
+                const int on = o + (up ? off : -off);
+                // the wrapped cell of an odd axis has the same colour
+                const int cn = in || !(lim[ax] & 1) ? c ^ 1 : c;
+                nb[s][c][e] = in || bc.t[2 * ax + up] == MF3D_BC_PERIODIC ? cn * kHalf + (on >> 1)
+                                                                          : 2 * kHalf;
+            }
+            T aC = f[s][c][0] + f[s][c][1] + f[s][c][2] + f[s][c][3] + f[s][c][4] + f[s][c][5];
+            if (pin && o == 0) aC *= T(2);
+            dg[s][c] = aC;
+            rd[s][c] = recip_of(aC);
         }
     }
     __syncthreads();
     for (int it = 0; it < iters; ++it) {
+#pragma unroll
         for (int c = 0; c < 2; ++c) {
 #pragma unroll
-            for (int m = 0; m < kSmallPer; ++m) {
-                if (colour[m] != c) continue;
-                const int o = 2 * (int)threadIdx.x + (m & 1) + 2 * kSmallBlock * (m >> 1);
+            for (int s = 0; s < kS; ++s) {
+                if (own[s][c] < 0) continue;
                 T v[6];
 #pragma unroll
-                for (int q = 0; q < 6; ++q) v[q] = nb[m][q] >= 0 ? xs[nb[m][q]] : T(0);
-                xs[o] = gs_value(f[m], v, bl[m], bs, pin && o == 0);
+                for (int e = 0; e < 6; ++e) v[e] = xs[nb[s][c][e]];
+                T sum = v[0] * f[s][c][0];
+#pragma unroll
+                for (int e = 1; e < 6; ++e) sum = fma(v[e], f[s][c][e], sum);
+                xs[own_slot(s, c)] = quot_by(fma(-bl[s][c], bs, sum), dg[s][c], rd[s][c]);
             }
             __syncthreads();
         }
     }
-    for (int o = threadIdx.x; o < n; o += kSmallBlock) x[o] = xs[o];
+#pragma unroll
+    for (int s = 0; s < kS; ++s)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+            if (own[s][c] >= 0) x[own[s][c]] = xs[own_slot(s, c)];
 }
 
 template <typename T, typename TC>
@@ -722,7 +747,7 @@ __global__ void __launch_bounds__(kSmallBlock)
     small_kernel(Dims d, BcTypes bc, int pin, T bs, T* __restrict__ x, const T* __restrict__ b,
                  const TC* __restrict__ FX, const TC* __restrict__ FY,
                  const TC* __restrict__ FZ, int iters, int zero_init, const T* __restrict__ xc) {
-    __shared__ T xs[kSmallBlock * kSmallPer];
+    __shared__ T xs[kSmallSlots];
     small_body<T, TC>(xs, d, bc, pin, bs, x, b, FX, FY, FZ, iters, zero_init, xc);
 }
 
@@ -1662,7 +1687,7 @@ __global__ void __launch_bounds__(kBlock)
 template <typename TC>
 __global__ void __launch_bounds__(kSmallBlock)
     small_batch_kernel(const BatchLevel* __restrict__ Ls, int iters, int zero_init, int use_xc) {
-    __shared__ float xs[kSmallBlock * kSmallPer];
+    __shared__ float xs[kSmallSlots];
     const BatchLevel& L = Ls[blockIdx.x];
     if (L.st->stop) return;
     small_body<float, TC>(xs, Dims{L.nx, L.ny, L.nz}, L.bc, L.pin, L.bs, L.x, L.b,

@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import BC_MIXES, bc_pair, random_K, rel_l2
+import oracle as O
+from helpers import BC_MIXES, bc_pair, grid_pair, random_K, rel_l2
 from macroflow3d_amd import numerics as nm
 from macroflow3d_amd import physics as ph
 from macroflow3d_amd.core import Grid3D
@@ -89,3 +90,26 @@ def test_fp64_solve_on_window_passes(ctx, shape, fold_r, graph):
         ws.close()
     assert its[0] == its[1]
     assert rel_l2(heads[1], heads[0]) < 1e-11
+
+
+@pytest.mark.parametrize("shape,mix", [
+    ((16, 16, 16), "all_periodic"), ((18, 14, 10), "all_neumann"), ((2, 4, 512), "periodic_yz"),
+    ((15, 13, 11), "darcy_x"), ((7, 16, 31), "all_dirichlet"), ((14, 9, 3), "all_neumann"),
+    ((3, 5, 273), "darcy_x"), ((5, 2, 2), "periodic_yz")])
+def test_small_level_iterations_match_oracle(ctx, shape, mix):
+    """One-workgroup GSRB of a whole small level (pairs of the linear order, odd
+    and even axes), 7 iterations from zero: the same sums to rounding."""
+    g, og = grid_pair(*shape)
+    bc, obc = bc_pair(mix)
+    n = g.num_cells()
+    K, r = random_K(n, 61), np.random.default_rng(62).standard_normal(n)
+    cfg = ph.HeadSolveConfig(mg_levels=1, mg_coarse_iters=7)
+    ws = ph.FlowWorkspace()
+    M = nm.MultigridPreconditioner.build(ctx, ws, g, bc, cfg, torch.as_tensor(K).to(ctx.device))
+    out = ctx.empty(n)
+    M.apply(ctx, torch.as_tensor(r).to(ctx.device), out)
+    ctx.synchronize()
+    ref = O.gsrb_smooth_3d(og, obc, mix == "all_neumann" or mix == "all_periodic",
+                           np.zeros(n), r, K, 7)
+    assert rel_l2(out.cpu().numpy(), ref) < 1e-12
+    ws.close()
