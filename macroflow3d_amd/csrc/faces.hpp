@@ -141,6 +141,15 @@ int block_pass(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, c
 // hs: colour-split level with faces from h, else natural order with FP64 faces F
 int block_pass(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, const FaceSet& F,
                const double* hs, const BlockPass<double>& p);
+// Fused smoothing pass of a large FP64 colour-split level with a colour-split coarse
+// level (fused64.hip): BlockPass with two iterations, from zero with bcoarse (xout then
+// gets the black values alone) or from xin (black values) with xc. z as in block_pass,
+// with fused64_partials(g) partials of (b, z), b = r.
+bool fused64_ok(const mf3d_grid& g);
+bool fused64_pays(const mf3d_grid& g);  // faster there than half-sweeps
+unsigned fused64_partials(const mf3d_grid& g);
+int fused64_pass(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin,
+                 const double* hs, const BlockPass<double>& p);
 // b = r in colour-split order; ru: r -= alpha Ap first, with the (r, r) partials
 // (one per 2048 cells)
 int r_to_split64(hipStream_t s, const mf3d_grid& g, const double* r, const RUpd* ru, double* b);

@@ -520,12 +520,15 @@ FGeo fgeo_of(const mf3d_grid& g) {
     G.half = (long)G.h * g.ny * g.nz;
     G.tx = (G.h + kIX - 1) / kIX;
     G.ty = (g.ny + kIY - 1) / kIY;
-    // one workgroup runs on a CU at a time (its registers); chunks of planes fill
-    // the 256 CUs, as long as a chunk keeps its 8 or 9 extra planes a small part
-    const int want = std::max(1, 256 / (G.tx * G.ty));
-    const int chunks = std::max(1, std::min(want, g.nz / 32));
-    G.kz = ((g.nz + chunks - 1) / chunks + 1) / 2 * 2;
-    G.chunks = (g.nz + G.kz - 1) / G.kz;
+    // One workgroup runs on a CU at a time (its registers): as many chunks of planes
+    // as make the fewest steps, (256 workgroups in flight) x (planes of a chunk and
+    // the nine around it); more chunks read more rims, so only for a twentieth less
+    long best = -1;
+    for (int c = 1; c <= std::max(1, g.nz / 32); ++c) {
+        const int kz = ((g.nz + c - 1) / c + 1) / 2 * 2, chunks = (g.nz + kz - 1) / kz;
+        const long t = ((long)G.tx * G.ty * chunks + 255) / 256 * (kz + 9);
+        if (best < 0 || 20 * t < 19 * best) best = t, G.kz = kz, G.chunks = chunks;
+    }
     return G;
 }
 

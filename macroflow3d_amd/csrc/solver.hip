@@ -85,6 +85,7 @@ struct Level {
     // smoothing of a small level in window passes, which read one x and write
     // another (block.hip)
     bool block = false;
+    bool fused64 = false;   // FP64 smoothing in fused passes (fused64.hip), the same way
     double* x2 = nullptr;
     float* x32s = nullptr;
     bool fused = false;     // FP32 smoothing in fused passes, which use
@@ -350,7 +351,8 @@ int ensure_workspace(mf3d_workspace* ws, const mf3d_grid& g, int levels) {
     const size_t march_cap =
         (size_t)kern::kMarchMaxBlocks + ((size_t)g.nx * g.ny / 4 + 63) / 64;
     ws->partials_cap = std::max<size_t>({kern::reduce_blocks(n), kern::op_partials(g), n / 256,
-                                         march_cap, kBlockMaxWindows64}) + 64;
+                                         march_cap, kBlockMaxWindows64,
+                                         kern::fused64_partials(g)}) + 64;
     MF3D_TRY(ws->alloc(&ws->partials, ws->partials_cap));
     // one per workgroup of the finest sweep (8 cells per thread, >= 64 threads;
     // FP64: one per march workgroup)
@@ -723,7 +725,11 @@ int mg_setup(mf3d_workspace* ws, hipStream_t s, const mf3d_grid& g, const mf3d_b
         L.block = ws->fuse != 0 && !defer_coarse && l + 1 < ws->lv.size() && ws->pre > 0 &&
                   ws->post > 0 && !L.fused && (!mixed || l > 0) &&
                   kern::block_windows(L.g) <= (mixed ? kBlockMaxWindows32 : kBlockMaxWindows64);
-        if (!L.block) continue;
+        L.fused64 = ws->fuse != 0 && !mixed && !L.block && !defer_coarse &&
+                    L.order64 == ORDER_SPLIT && ws->lv[l + 1].order64 == ORDER_SPLIT &&
+                    ws->pre == 2 && ws->post == 2 && kern::fused64_ok(L.g) &&
+                    (ws->fuse == 1 || kern::fused64_pays(L.g));
+        if (!L.block && !L.fused64) continue;
         if (mixed && !L.x32s) MF3D_TRY(ws->alloc(&L.x32s, L.n));
         if (!mixed && !L.x2) MF3D_TRY(ws->alloc(&L.x2, L.n));
     }
@@ -868,9 +874,9 @@ int vcycle64(mf3d_workspace* ws, hipStream_t s, size_t l, bool zero_init, const 
     Level& L = ws->lv[l];
     Level& C = ws->lv[l + 1];  // a split level is never the coarsest
     const double dx2 = L.g.dx * L.g.dx;
-    if (L.block && zero_init) {
+    if ((L.block || L.fused64) && zero_init) {
         if (r64) MF3D_TRY(kern::r_to_split64(s, L.g, r64, ru, L.b));
-        if (np) *np = kern::block_windows(L.g);
+        if (np) *np = L.fused64 ? kern::fused64_partials(L.g) : kern::block_windows(L.g);
         return vcycle_block<double>(ws, s, l, L.x, L.b, z, rdot, rdot ? partials : nullptr);
     }
     const int tb = L.plan.block;
@@ -917,7 +923,9 @@ int vcycle_block(mf3d_workspace* ws, hipStream_t s, size_t l, T* x, const T* b, 
         p.xout = left % 2 ? V::x2(L) : x;
         cur = p.xout;
         if constexpr (F64)
-            return kern::block_pass(s, L.g, ws->bct, ws->pin, L.f64, split ? L.hs : nullptr, p);
+            return L.fused64 ? kern::fused64_pass(s, L.g, ws->bct, ws->pin, L.hs, p)
+                             : kern::block_pass(s, L.g, ws->bct, ws->pin, L.f64,
+                                                split ? L.hs : nullptr, p);
         else
             return kern::block_pass(s, L.g, ws->bct, ws->pin, L.flo, p);
     };
@@ -1157,7 +1165,7 @@ int run_pcg(mf3d_workspace* ws, hipStream_t s, const mf3d_grid& g,
     const bool fuse_r = (zx && ws->fold_r && r_in_first_sweep(ws)) || fuse64;
     const unsigned np_sweep =
         !fuse64    ? sweep_partials(ws)
-        : L0.block ? kern::reduce_blocks(n)
+        : L0.block || L0.fused64 ? kern::reduce_blocks(n)
                    : kern::split64_partials(L0.g, L0.plan.block, ws->march_blocks);
     unsigned nprz = 0;  // (r, z) partials of the last preconditioner application
     // the reference's own rule (||r||/||r0||, FP64) keeps its exact semantics
