@@ -24,6 +24,20 @@ __device__ __forceinline__ double rcp_nr(double s) {
     return fma(r, e, r);
 }
 
+// n / d from the reciprocal estimate r of d, corrected once by the remainder, with
+// the hardware's fix-up for zeros and infinities (FP32: gs_quot's value; FP64: within
+// the last bit of the quotient). For diagonals that divide more than once.
+__device__ __forceinline__ float recip_of(float d) { return __builtin_amdgcn_rcpf(d); }
+__device__ __forceinline__ double recip_of(double d) { return rcp_nr(d); }
+__device__ __forceinline__ float quot_by(float n, float d, float r) {
+    const float q = n * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, d, n), r, q), d, n);
+}
+__device__ __forceinline__ double quot_by(double n, double d, double r) {
+    const double q = n * r;
+    return __builtin_amdgcn_div_fixup(fma(fma(-q, d, n), r, q), d, n);
+}
+
 // Boundary of one side of a cell: the neighbour's offset (0 without one), and
 // whether the neighbour exists (in the domain or periodic) and the face does
 // (neighbour or Dirichlet).

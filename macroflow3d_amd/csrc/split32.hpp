@@ -47,20 +47,6 @@ __device__ __forceinline__ float gs_quot(float n, float d) {
     return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, d, n), r, q), d, n);
 }
 __device__ __forceinline__ double gs_quot(double n, double d) { return n / d; }
-// n / d from the reciprocal estimate r of d, corrected once by the remainder, with
-// the hardware's fix-up for zeros and infinities (FP32: gs_quot's value; FP64: within
-// the last bit of the quotient). For diagonals that divide more than once.
-__device__ __forceinline__ float recip_of(float d) { return __builtin_amdgcn_rcpf(d); }
-__device__ __forceinline__ double recip_of(double d) { return rcp_nr(d); }
-__device__ __forceinline__ float quot_by(float n, float d, float r) {
-    const float q = n * r;
-    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, d, n), r, q), d, n);
-}
-__device__ __forceinline__ double quot_by(double n, double d, double r) {
-    const double q = n * r;
-    return __builtin_amdgcn_div_fixup(fma(fma(-q, d, n), r, q), d, n);
-}
-
 template <typename T>
 __device__ __forceinline__ T gs_value(const T (&f)[6], const T (&v)[6], T b, T bs, bool pin0) {
     T result = v[0] * f[0];

@@ -16,6 +16,7 @@
 #include <algorithm>
 
 #include "kernels.hpp"
+#include "reduce.hpp"
 
 namespace mf3d {
 namespace {
@@ -130,21 +131,41 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // ---- velocity diagnostics (velocity_diagnostics.cu:46-177) -------------------
-// One workgroup owns a tile of 64 x 4 cell columns (one wave per x row) and
-// marches kz planes up in z. Along z each thread carries the face values it
-// needs again one plane later (U and V of its column at k-1, k, k+1; W at k
-// and k+1 for itself and its four x/y neighbours), so a cell costs 9 marching
-// loads plus 8 loads of the x/y neighbours' U and V at plane k, which the
-// neighbouring lanes and rows bring into L1/L2. Algorithmic traffic: the three
-// padded components read once and the three cell fields written once.
-constexpr int kDiagX = 64, kDiagY = 4;
+// Everything but the divergence is differences of cell-centred means (u: of the
+// cell's two x faces, and so on), so a cell needs its own six faces and its
+// neighbours' means. A workgroup owns 64 x 16 columns (a wave a row; rows 0 and 15
+// only supply means: 64 x 14 cells a tile) and marches kz planes up: each thread
+// forms its column's means from five loads a plane, two planes ahead of their use,
+// keeps them for three planes (z differences) and shares plane k's through LDS (two
+// buffers, one barrier a plane).
+// Bound: HBM, the three padded components read once and the three cell fields
+// written once, 48 bytes a cell. 250x190x130: with 17 loads a cell and plane, each
+// plane's waited for at once, 105 us (2.8 TB/s); now 77 us (3.9 TB/s), 94 with
+// ordinary stores, which push the velocities out of the Infinity Cache.
+constexpr int kDiagX = 64, kDiagRows = 16, kDiagY = kDiagRows - 2;
+constexpr int kDiagBlock = kDiagX * kDiagRows;
 constexpr int kDiagQ = 9;  // per-workgroup partials: (min, max, sum) x 3 fields
+
+// the number of z-chunks that makes the fewest steps with one workgroup a CU
+struct Tiles {
+    int tx, ty, kz;
+    long nblocks;
+};
+Tiles tiles_of(int nx, int ny, int nz) {
+    Tiles t{(nx + kDiagX - 1) / kDiagX, (ny + kDiagY - 1) / kDiagY, 0, 0};
+    long best = -1;
+    for (int c = 1; c <= nz; ++c) {
+        const int kz = (nz + c - 1) / c, chunks = (nz + kz - 1) / kz;
+        const long nb = (long)t.tx * t.ty * chunks;
+        const long steps = (nb + 255) / 256 * (kz + 2);  // two planes before the first step
+        if (best < 0 || steps < best) best = steps, t.kz = kz, t.nblocks = nb;
+    }
+    return t;
+}
 
 struct DiagDims {
     int nx, ny, nz;
-    int tx, kz;    // tiles along x; planes per workgroup
-    int tiles;     // tiles per plane chunk
-    long nblocks;  // tiles x chunks
+    Tiles t;
     double ix, iy, iz;
     int curl;      // all dimensions >= 3
 };
@@ -168,8 +189,9 @@ struct MinMaxSum {
     }
 };
 
-// min, max and sum over the workgroup (kBlock threads), valid in thread 0;
-// wv: LDS of 3 * kBlock / 64 doubles
+// min, max and sum over the workgroup (BS threads), valid in thread 0;
+// wv: LDS of 3 * BS / 64 doubles
+template <int BS>
 __device__ inline void block_mms(MinMaxSum& a, double* wv) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -177,7 +199,7 @@ __device__ inline void block_mms(MinMaxSum& a, double* wv) {
         a.hi = fmax(a.hi, __shfl_xor(a.hi, off, 64));
         a.sum += __shfl_xor(a.sum, off, 64);
     }
-    constexpr int W = kBlock / 64;
+    constexpr int W = BS / 64;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     __syncthreads();  // wv may still be read by a previous call
     if (lane == 0) {
@@ -197,90 +219,102 @@ __device__ inline void block_mms(MinMaxSum& a, double* wv) {
     }
 }
 
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kDiagBlock)
     diag_kernel(DiagDims d, const double* __restrict__ U, const double* __restrict__ V,
                 const double* __restrict__ W, double* __restrict__ dv, double* __restrict__ om,
                 double* __restrict__ he, double* __restrict__ partials) {
-    const long blk = xcd_block(d.nblocks);
-    if (blk < 0) return;  // padding block: uniform exit before the reductions
-    const int tile = (int)(blk % d.tiles), chunk = (int)(blk / d.tiles);
-    const int i = (tile % d.tx) * kDiagX + (int)(threadIdx.x & 63);
-    const int j = (tile / d.tx) * kDiagY + (int)(threadIdx.x >> 6);
-    const int k0 = chunk * d.kz, k1 = min(k0 + d.kz, d.nz);
-    const bool active = i < d.nx && j < d.ny;
-    // every load stays inside the padded arrays: columns clamped to the grid,
-    // neighbours to [0, n] (the padded extent), planes to [0, nz]
-    const int ic = min(i, d.nx - 1), jc = min(j, d.ny - 1);
-    const int im = max(ic - 1, 0), ip = ic + 1, jm = max(jc - 1, 0), jp = jc + 1;
-    const bool colin = d.curl && ic >= 1 && ic <= d.nx - 2 && jc >= 1 && jc <= d.ny - 2;
+    constexpr int kRow = kDiagX + 2;
+    __shared__ double mu[2][kDiagRows][kRow], mv[2][kDiagRows][kRow], mw[2][kDiagRows][kRow];
+    const long blk = xcd_block(d.t.nblocks);
+    if (blk < 0) return;  // padding block: uniform exit before the barriers
+    const long tiles = (long)d.t.tx * d.t.ty;
+    const int tile = (int)(blk % tiles), chunk = (int)(blk / tiles);
+    const int lane = (int)(threadIdx.x & 63), row = (int)(threadIdx.x >> 6);
+    const int i = tile % d.t.tx * kDiagX + lane, j = tile / d.t.tx * kDiagY - 1 + row;
+    const int k0 = chunk * d.t.kz, k1 = min(k0 + d.t.kz, d.nz);
+    const bool active = i < d.nx && j >= 0 && j < d.ny && row > 0 && row < kDiagRows - 1;
+    // every load stays inside the padded arrays: columns clamped to the grid, planes
+    // to [0, nz] (a clamped column's means are not used)
+    const int ic = min(i, d.nx - 1), jc = min(max(j, 0), d.ny - 1);
+    const bool colin = d.curl && i >= 1 && i <= d.nx - 2 && j >= 1 && j <= d.ny - 2;
     const double hx = 0.5 * d.ix, hy = 0.5 * d.iy, hz = 0.5 * d.iz;
+    // the columns beyond the tile: the left one for lanes 0..31, the right one for the
+    // others, every lane loading so that all loads are in flight together
+    const bool left = lane < kDiagX / 2, edge = lane == 0 || lane == kDiagX - 1;
+    const int ie = min(max(i - lane + (left ? -1 : kDiagX), 0), d.nx - 1);
+    const int eslot = left ? 0 : kRow - 1;
+    const long sp = (long)(d.nx + 1) * (d.ny + 1);
+    const long o = pad_idx(d, ic, jc, 0), oe = pad_idx(d, ie, jc, 0);
+    const int yp = d.nx + 1;
 
-    // U(i), U(i+1) and V(j), V(j+1) of the column at planes k-1, k, k+1
-    const int kb = max(k0 - 1, 0);
-    double ua0 = U[pad_idx(d, ic, jc, kb)], ub0 = U[pad_idx(d, ip, jc, kb)];
-    double va0 = V[pad_idx(d, ic, jc, kb)], vb0 = V[pad_idx(d, ic, jp, kb)];
-    double ua1 = U[pad_idx(d, ic, jc, k0)], ub1 = U[pad_idx(d, ip, jc, k0)];
-    double va1 = V[pad_idx(d, ic, jc, k0)], vb1 = V[pad_idx(d, ic, jp, k0)];
-    // W at plane k of the column and of its x/y neighbours
-    double w0 = W[pad_idx(d, ic, jc, k0)];
-    double wxm0 = W[pad_idx(d, im, jc, k0)], wxp0 = W[pad_idx(d, ip, jc, k0)];
-    double wym0 = W[pad_idx(d, ic, jm, k0)], wyp0 = W[pad_idx(d, ic, jp, k0)];
+    struct Plane {  // plane k as loaded; w: of plane k + 1
+        double ua, ub, va, vb, w, ea, eb, ew;
+    };
+    auto load = [&](int k) {
+        const long q = sp * min(max(k, 0), d.nz), qw = sp * min(max(k + 1, 0), d.nz);
+        return Plane{U[q + o], U[q + o + 1], V[q + o],       V[q + o + yp],
+                     W[qw + o], V[q + oe],    V[q + oe + yp], W[qw + oe]};
+    };
+    double w0 = W[sp * k0 + o], ew0 = W[sp * k0 + oe];
+    Plane below = load(k0 - 1), cur = load(k0), nxt = load(k0 + 1);
+    double u0 = 0.5 * (below.ua + below.ub), v0 = 0.5 * (below.va + below.vb);
 
     MinMaxSum sd, so, sh;
     sd.init();
     so.init();
     sh.init();
     for (int k = k0; k < k1; ++k) {
-        const int kn = k + 1;  // <= nz
-        const double ua2 = U[pad_idx(d, ic, jc, kn)], ub2 = U[pad_idx(d, ip, jc, kn)];
-        const double va2 = V[pad_idx(d, ic, jc, kn)], vb2 = V[pad_idx(d, ic, jp, kn)];
-        const double w1 = W[pad_idx(d, ic, jc, kn)];
-        const double wxm1 = W[pad_idx(d, im, jc, kn)], wxp1 = W[pad_idx(d, ip, jc, kn)];
-        const double wym1 = W[pad_idx(d, ic, jm, kn)], wyp1 = W[pad_idx(d, ic, jp, kn)];
-        const double uym_a = U[pad_idx(d, ic, jm, k)], uym_b = U[pad_idx(d, ip, jm, k)];
-        const double uyp_a = U[pad_idx(d, ic, jp, k)], uyp_b = U[pad_idx(d, ip, jp, k)];
-        const double vxm_a = V[pad_idx(d, im, jc, k)], vxm_b = V[pad_idx(d, im, jp, k)];
-        const double vxp_a = V[pad_idx(d, ip, jc, k)], vxp_b = V[pad_idx(d, ip, jp, k)];
-
-        const double divv = (ub1 - ua1) * d.ix + (vb1 - va1) * d.iy + (w1 - w0) * d.iz;
-        double omv = 0.0, hev = 0.0;
-        if (colin && k >= 1 && k <= d.nz - 2) {
-            const double uc = 0.5 * (ua1 + ub1), vc = 0.5 * (va1 + vb1), wc = 0.5 * (w0 + w1);
-            const double wx = (0.5 * (wyp0 + wyp1) - 0.5 * (wym0 + wym1)) * hy -
-                              (0.5 * (va2 + vb2) - 0.5 * (va0 + vb0)) * hz;
-            const double wy = (0.5 * (ua2 + ub2) - 0.5 * (ua0 + ub0)) * hz -
-                              (0.5 * (wxp0 + wxp1) - 0.5 * (wxm0 + wxm1)) * hx;
-            const double wz = (0.5 * (vxp_a + vxp_b) - 0.5 * (vxm_a + vxm_b)) * hx -
-                              (0.5 * (uyp_a + uyp_b) - 0.5 * (uym_a + uym_b)) * hy;
-            omv = sqrt(wx * wx + wy * wy + wz * wz);
-            hev = uc * wx + vc * wy + wc * wz;
+        const Plane ahead = load(k + 2);  // (the chunk's last ones unused)
+        const int buf = k & 1;
+        const double uc = 0.5 * (cur.ua + cur.ub), vc = 0.5 * (cur.va + cur.vb),
+                     wc = 0.5 * (w0 + cur.w);
+        const double u2 = 0.5 * (nxt.ua + nxt.ub), v2 = 0.5 * (nxt.va + nxt.vb);
+        mu[buf][row][lane + 1] = uc;
+        mv[buf][row][lane + 1] = vc;
+        mw[buf][row][lane + 1] = wc;
+        if (edge) {
+            mv[buf][row][eslot] = 0.5 * (cur.ea + cur.eb);
+            mw[buf][row][eslot] = 0.5 * (ew0 + cur.ew);
         }
+        lds_barrier();
         if (active) {
+            const double divv = (cur.ub - cur.ua) * d.ix + (cur.vb - cur.va) * d.iy +
+                                (cur.w - w0) * d.iz;
+            double omv = 0.0, hev = 0.0;
+            if (colin && k >= 1 && k <= d.nz - 2) {
+                const double wx = (mw[buf][row + 1][lane + 1] - mw[buf][row - 1][lane + 1]) * hy -
+                                  (v2 - v0) * hz;
+                const double wy = (u2 - u0) * hz -
+                                  (mw[buf][row][lane + 2] - mw[buf][row][lane]) * hx;
+                const double wz = (mv[buf][row][lane + 2] - mv[buf][row][lane]) * hx -
+                                  (mu[buf][row + 1][lane + 1] - mu[buf][row - 1][lane + 1]) * hy;
+                omv = sqrt(wx * wx + wy * wy + wz * wz);
+                hev = uc * wx + vc * wy + wc * wz;
+            }
             const long c = (long)i + (long)d.nx * ((long)j + (long)d.ny * k);
-            dv[c] = divv;
-            om[c] = omv;
-            he[c] = hev;
+            __builtin_nontemporal_store(divv, dv + c);
+            __builtin_nontemporal_store(omv, om + c);
+            __builtin_nontemporal_store(hev, he + c);
             if (partials) {
                 sd.add(divv);
                 so.add(omv);
                 sh.add(hev);
             }
         }
-        ua0 = ua1, ub0 = ub1, va0 = va1, vb0 = vb1;
-        ua1 = ua2, ub1 = ub2, va1 = va2, vb1 = vb2;
-        w0 = w1, wxm0 = wxm1, wxp0 = wxp1, wym0 = wym1, wyp0 = wyp1;
+        u0 = uc, v0 = vc, w0 = cur.w, ew0 = cur.ew;
+        cur = nxt, nxt = ahead;
     }
     if (!partials) return;  // uniform across the grid
-    __shared__ double wv[3 * kBlock / 64];
-    block_mms(sd, wv);
-    block_mms(so, wv);
-    block_mms(sh, wv);
+    __shared__ double wv[3 * kDiagBlock / 64];
+    block_mms<kDiagBlock>(sd, wv);
+    block_mms<kDiagBlock>(so, wv);
+    block_mms<kDiagBlock>(sh, wv);
     if (threadIdx.x == 0) {
         const MinMaxSum* f[3] = {&sd, &so, &sh};
         for (int q = 0; q < 3; ++q) {
-            partials[(3 * q + 0) * d.nblocks + blk] = f[q]->lo;
-            partials[(3 * q + 1) * d.nblocks + blk] = f[q]->hi;
-            partials[(3 * q + 2) * d.nblocks + blk] = f[q]->sum;
+            partials[(3 * q + 0) * d.t.nblocks + blk] = f[q]->lo;
+            partials[(3 * q + 1) * d.t.nblocks + blk] = f[q]->hi;
+            partials[(3 * q + 2) * d.t.nblocks + blk] = f[q]->sum;
         }
     }
 }
@@ -301,7 +335,7 @@ __global__ void __launch_bounds__(kBlock)
     for (int u = 0; u < kPer; ++u)
         if (base + (long)u * kBlock < n) a.add(v[u]);
     __shared__ double wv[3 * kBlock / 64];
-    block_mms(a, wv);
+    block_mms<kBlock>(a, wv);
     if (threadIdx.x == 0) {
         partials[blockIdx.x] = a.lo;
         partials[gridDim.x + blockIdx.x] = a.hi;
@@ -309,29 +343,28 @@ __global__ void __launch_bounds__(kBlock)
     }
 }
 
-// second stage: nq fields, each with (min, max, sum) partials of np blocks;
+// second stage, a workgroup per field with its (min, max, sum) partials of np blocks;
 // out[3q..3q+2] = min, max, sum / n (fixed summation order)
 __global__ void __launch_bounds__(kBlock)
-    stats_final_kernel(const double* __restrict__ partials, long np, int nq, double n,
+    stats_final_kernel(const double* __restrict__ partials, long np, double n,
                        double* __restrict__ out) {
     __shared__ double wv[3 * kBlock / 64];
-    for (int q = 0; q < nq; ++q) {
-        const double* lo = partials + (3 * q + 0) * np;
-        const double* hi = partials + (3 * q + 1) * np;
-        const double* sm = partials + (3 * q + 2) * np;
-        MinMaxSum a;
-        a.init();
-        for (long b = threadIdx.x; b < np; b += kBlock) {
-            a.lo = fmin(a.lo, lo[b]);
-            a.hi = fmax(a.hi, hi[b]);
-            a.sum += sm[b];
-        }
-        block_mms(a, wv);
-        if (threadIdx.x == 0) {
-            out[3 * q + 0] = a.lo;
-            out[3 * q + 1] = a.hi;
-            out[3 * q + 2] = a.sum / n;
-        }
+    const int q = (int)blockIdx.x;
+    const double* lo = partials + (3 * q + 0) * np;
+    const double* hi = partials + (3 * q + 1) * np;
+    const double* sm = partials + (3 * q + 2) * np;
+    MinMaxSum a;
+    a.init();
+    for (long b = threadIdx.x; b < np; b += kBlock) {
+        a.lo = fmin(a.lo, lo[b]);
+        a.hi = fmax(a.hi, hi[b]);
+        a.sum += sm[b];
+    }
+    block_mms<kBlock>(a, wv);
+    if (threadIdx.x == 0) {
+        out[3 * q + 0] = a.lo;
+        out[3 * q + 1] = a.hi;
+        out[3 * q + 2] = a.sum / n;
     }
 }
 
@@ -340,12 +373,7 @@ DiagDims diag_dims(const mf3d_grid& g) {
     d.nx = g.nx;
     d.ny = g.ny;
     d.nz = g.nz;
-    d.tx = (g.nx + kDiagX - 1) / kDiagX;
-    d.tiles = d.tx * ((g.ny + kDiagY - 1) / kDiagY);
-    // enough plane chunks for ~2048 workgroups, at most 16 planes each
-    const long want = 2048;
-    d.kz = (int)std::max(1L, std::min(16L, (long)g.nz * d.tiles / want));
-    d.nblocks = (long)d.tiles * ((g.nz + d.kz - 1) / d.kz);
+    d.t = tiles_of(g.nx, g.ny, g.nz);
     d.ix = 1.0 / g.dx;
     d.iy = 1.0 / g.dy;
     d.iz = 1.0 / g.dz;
@@ -357,17 +385,17 @@ DiagDims diag_dims(const mf3d_grid& g) {
 
 namespace kern {
 
-size_t diag_partials(const mf3d_grid& g) { return (size_t)kDiagQ * diag_dims(g).nblocks; }
+size_t diag_partials(const mf3d_grid& g) { return (size_t)kDiagQ * diag_dims(g).t.nblocks; }
 
 int velocity_diagnostics(hipStream_t s, const mf3d_grid& g, const double* U, const double* V,
                          const double* W, double* div, double* omag, double* hel,
                          double* partials, double* stats) {
     const DiagDims d = diag_dims(g);
-    diag_kernel<<<xcd_round((size_t)d.nblocks), kBlock, 0, s>>>(d, U, V, W, div, omag, hel,
-                                                               stats ? partials : nullptr);
+    diag_kernel<<<xcd_round((size_t)d.t.nblocks), kDiagBlock, 0, s>>>(d, U, V, W, div, omag, hel,
+                                                                     stats ? partials : nullptr);
     MF3D_HIP_TRY(hipGetLastError());
     if (stats) {
-        stats_final_kernel<<<1, kBlock, 0, s>>>(partials, d.nblocks, 3, (double)cells(g), stats);
+        stats_final_kernel<<<3, kBlock, 0, s>>>(partials, d.t.nblocks, (double)cells(g), stats);
         MF3D_HIP_TRY(hipGetLastError());
     }
     return MF3D_OK;
@@ -379,7 +407,7 @@ int field_stats(hipStream_t s, const double* x, size_t n, double* partials, doub
     const long nb = (long)((n + 2047) / 2048);
     stats_kernel<<<(unsigned)nb, kBlock, 0, s>>>(x, (long)n, partials);
     MF3D_HIP_TRY(hipGetLastError());
-    stats_final_kernel<<<1, kBlock, 0, s>>>(partials, nb, 1, (double)n, out);
+    stats_final_kernel<<<1, kBlock, 0, s>>>(partials, nb, (double)n, out);
     MF3D_HIP_TRY(hipGetLastError());
     return MF3D_OK;
 }
