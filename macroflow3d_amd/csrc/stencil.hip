@@ -323,7 +323,7 @@ __global__ void __launch_bounds__(kBlock)
 
 // Whole GSRB smoothing of a small level by one workgroup: x and 1/K in LDS,
 // each thread's own K and b in registers. Same per-cell values as
-// gsrb_colour_kernel up to the summation order of boundary cells; replaces
+// column_kernel up to the summation order of boundary cells; replaces
 // 2*iters launches (the coarsest level runs 50 iterations, v_cycle.cu:41-45).
 constexpr int kSmallBlock = 1024;
 constexpr int kSmallPer = 4;
