@@ -279,6 +279,11 @@ __global__ void __launch_bounds__(256) planar_kernel(PlanarCopies D) {
     for (int c = 0; c < 8; ++c) d[(long)c * C.P.plane] = val[c];
 }
 
+__global__ void __launch_bounds__(256) zero_kernel(uint4* __restrict__ p, long n) {
+    const long e = (long)blockIdx.x * 256 + threadIdx.x;
+    if (e < n) p[e] = uint4{0u, 0u, 0u, 0u};
+}
+
 struct WLayer {
     const __hip_bfloat16* dY;  // planar, 16 ct channels
     const __hip_bfloat16* X;   // planar, 16 it channels
@@ -753,7 +758,7 @@ using namespace mf3d;
 using namespace mf3d::cnn;
 
 // Weight gradients of up to kMaxWLayers layers: channel-first operand copies
-// and per-slice partial sums in one zeroed allocation
+// (zeroed) and per-slice partial sums in one allocation
 struct WeightScratch {
     void* mem = nullptr;
     PlanarCopies copies{};
@@ -831,11 +836,12 @@ struct WeightTask {
 // Slices of a layer: 16 steps (512 voxels) a wave amortise its partial sums;
 // fewer steps where the layer would otherwise have under 8 slices (27 taps x 8
 // waves), more above 64 slices (whose partial sums would grow with the grid).
-int make_scratch(WeightScratch& S, const WeightTask* T, int n) {
-    S.copies.n = 0;
-    S.copy_blocks = 0;
+// out is written last, once all of it is ready: a scratch with memory counts as
+// usable, so a failed zeroing must leave none. The zeroing goes to the stream of
+// the gradients that need it and waits for nothing.
+int make_scratch(hipStream_t s, WeightScratch& out, const WeightTask* T, int n) {
+    WeightScratch S;
     S.layers.n = n;
-    S.layers.waves = S.layers.elems = 0;
     size_t bytes = 0;
     auto take = [&](size_t b) {
         const size_t at = bytes;
@@ -843,11 +849,18 @@ int make_scratch(WeightScratch& S, const WeightTask* T, int n) {
         return at;
     };
     std::vector<size_t> at;
-    for (int e = 0; e < n; ++e) {
+    for (int e = 0; e < n; ++e) {  // the operand copies first: they are zeroed
         const WeightTask& t = T[e];
         WLayer& L = S.layers.l[e];
         L.P = planar_of(t.g);
         L.ct = t.ct, L.it = t.it;
+        at.push_back(take((size_t)16 * L.ct * L.P.plane * 2));
+        at.push_back(take((size_t)16 * L.it * L.P.plane * 2));
+    }
+    const size_t copies = bytes;
+    for (int e = 0; e < n; ++e) {
+        const WeightTask& t = T[e];
+        WLayer& L = S.layers.l[e];
         const long steps = (L.P.groups + 3) / 4;
         L.steps = (int)std::max({1L, std::min(16L, steps / 8), (steps + 63) / 64});
         L.slices = (int)((steps + L.steps - 1) / L.steps);
@@ -856,8 +869,6 @@ int make_scratch(WeightScratch& S, const WeightTask* T, int n) {
         L.cin = t.cin, L.cout = t.cout, L.gw = t.gw, L.gb = t.gb;
         L.elem0 = S.layers.elems;
         S.layers.elems += 27 * t.cin * t.cout + t.cout;
-        at.push_back(take((size_t)16 * L.ct * L.P.plane * 2));
-        at.push_back(take((size_t)16 * L.it * L.P.plane * 2));
         at.push_back(take((size_t)L.slices * 16 * L.ct * 27 * 16 * L.it * 4));
         at.push_back(take((size_t)L.slices * 16 * L.ct * 4));
         for (int q = 0; q < 2; ++q) {
@@ -874,18 +885,24 @@ int make_scratch(WeightScratch& S, const WeightTask* T, int n) {
     }
     MF3D_TRY(net_alloc(&S.mem, bytes));
     // the copies' borders stay zero: planar_kernel writes the voxels only
-    MF3D_HIP_TRY(hipMemset(S.mem, 0, bytes));
-    MF3D_HIP_TRY(hipDeviceSynchronize());
+    zero_kernel<<<blocks((long)(copies / 16)), 256, 0, s>>>(static_cast<uint4*>(S.mem),
+                                                           (long)(copies / 16));
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) {
+        (void)hipFree(S.mem);
+        return fail(MF3D_ERR_HIP, std::string("weight-gradient scratch: ") + hipGetErrorString(err));
+    }
     char* m = static_cast<char*>(S.mem);
     for (int e = 0; e < n; ++e) {
         WLayer& L = S.layers.l[e];
-        __hip_bfloat16* d[2] = {(__hip_bfloat16*)(m + at[4 * e]), (__hip_bfloat16*)(m + at[4 * e + 1])};
+        __hip_bfloat16* d[2] = {(__hip_bfloat16*)(m + at[2 * e]), (__hip_bfloat16*)(m + at[2 * e + 1])};
         L.dY = d[0], L.X = d[1];
         S.copies.c[2 * e].dst = d[0];
         S.copies.c[2 * e + 1].dst = d[1];
-        L.part = (float*)(m + at[4 * e + 2]);
-        L.bpart = (float*)(m + at[4 * e + 3]);
+        L.part = (float*)(m + at[2 * n + 2 * e]);
+        L.bpart = (float*)(m + at[2 * n + 2 * e + 1]);
     }
+    out = S;
     return MF3D_OK;
 }
 
@@ -1095,7 +1112,7 @@ int backward(mf3d_wsnet* net, hipStream_t s, const mf3d_grid& gf, double hw, dou
             T[l] = WeightTask{*in[l].g, in[l].dY, in[l].X, net->cout_pad[l] / 16,
                               net->cin_pad[l] / 16, in[l].up, kLayers[l].cin, kLayers[l].cout,
                               GR + net->woff[l], GR + net->boff[l]};
-        MF3D_TRY(make_scratch(net->wg, T, kNumLayers));
+        MF3D_TRY(make_scratch(s, net->wg, T, kNumLayers));
     }
     MF3D_TRY(run_weight_grads(s, net->wg));
     if (loss) {
@@ -1347,7 +1364,7 @@ int mf3d_conv3d_backward_weights(mf3d_stream stream, const mf3d_grid* grid, int 
     const WeightTask T{*grid, (const __hip_bfloat16*)dY, (const __hip_bfloat16*)X, ct, it, 0, cin,
                        cout, gw, gb};
     WeightScratch S;
-    int st = make_scratch(S, &T, 1);
+    int st = make_scratch(s, S, &T, 1);
     if (st == MF3D_OK) st = run_weight_grads(s, S);
     if (st == MF3D_OK) {
         const hipError_t e = hipStreamSynchronize(s);
