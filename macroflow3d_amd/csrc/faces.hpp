@@ -94,6 +94,7 @@ int residual_restrict_faces(hipStream_t s, const mf3d_grid& g, const BcTypes& bc
                             double bsc = 0.0);
 // ---- fused smoothing passes of large colour-split FP32 levels (fused32.hip) -----
 bool fused32_ok(const mf3d_grid& g, CoefType t);
+bool fused32_pays(const mf3d_grid& g);  // faster than the half-sweeps there
 // the level's face records, made from its half-sweep faces
 size_t fused32_face_bytes(const mf3d_grid& g);
 int fused32_pack(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, const FaceSet& F,

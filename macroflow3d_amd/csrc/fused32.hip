@@ -512,6 +512,12 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+constexpr int kExtra = 9;  // planes around a chunk
+// one workgroup runs on a CU at a time (its registers): 256 in flight
+long steps_of(int tiles, int chunks, int kz) {
+    return ((long)tiles * chunks + 255) / 256 * (kz + kExtra);
+}
+
 FGeo fgeo_of(const mf3d_grid& g) {
     FGeo G;
     G.nx = g.nx, G.ny = g.ny, G.nz = g.nz;
@@ -520,13 +526,12 @@ FGeo fgeo_of(const mf3d_grid& g) {
     G.half = (long)G.h * g.ny * g.nz;
     G.tx = (G.h + kIX - 1) / kIX;
     G.ty = (g.ny + kIY - 1) / kIY;
-    // One workgroup runs on a CU at a time (its registers): as many chunks of planes
-    // as make the fewest steps, (256 workgroups in flight) x (planes of a chunk and
-    // the nine around it); more chunks read more rims, so only for a twentieth less
+    // as many chunks of planes as make the fewest steps; more chunks read more rims,
+    // so only for a twentieth less
     long best = -1;
     for (int c = 1; c <= std::max(1, g.nz / 32); ++c) {
         const int kz = ((g.nz + c - 1) / c + 1) / 2 * 2, chunks = (g.nz + kz - 1) / kz;
-        const long t = ((long)G.tx * G.ty * chunks + 255) / 256 * (kz + 9);
+        const long t = steps_of(G.tx * G.ty, chunks, kz);
         if (best < 0 || 20 * t < 19 * best) best = t, G.kz = kz, G.chunks = chunks;
     }
     return G;
@@ -562,6 +567,20 @@ bool fused32_ok(const mf3d_grid& g, CoefType t) {
     return (t == COEF_BF16 || t == COEF_F16) && g.nx % 4 == 0 && g.ny % 4 == 0 && g.nz % 4 == 0 &&
            g.nz >= 8 && (size_t)g.nx * g.ny < ((size_t)1 << 28) &&
            cells(g) < ((size_t)1 << 32);
+}
+
+// From 2^23 cells, where the tiles and z-chunks occupy most of the 256 CUs (256^3: 220
+// workgroups, 187 us a level for 271 us of half-sweeps; a 128^3 level would have 72
+// workgroups of 41 planes, about 100 us for 56 us of launch-bound half-sweeps), and
+// where the tiles are full enough: a step takes 2.4 us, what it replaces 20 ps a cell.
+// V-cycles with the passes and with half-sweeps, by cells a step: 8x1024x1024 39 000
+// 602 us for 241; 16x1024x512 74 000 376 for 259; 1024x8x1024 94 000 296 for 243;
+// 8192x32x32 102 000 300 for 318; 2048x512x8 123 000 248 for 290; 256^3 230 000 378 for
+// 499.
+bool fused32_pays(const mf3d_grid& g) {
+    const FGeo G = fgeo_of(g);
+    return cells(g) >= ((size_t)1 << 23) &&
+           steps_of(G.tx * G.ty, G.chunks, G.kz) <= (long)(cells(g) / 100000);
 }
 
 size_t fused32_face_bytes(const mf3d_grid& g) {

@@ -110,11 +110,6 @@ struct Level {
 // half-sweeps); FP64 ones fit once, and 512 are two waves (72x56x40, 315
 // windows: 36 us for 42; 64^3 takes the same 36). Another wave would cost what the launches do.
 constexpr size_t kBlockMaxWindows32 = 512, kBlockMaxWindows64 = 512;
-// FP32 levels smoothed by fused passes: from 2^23 cells their tiles and z-chunks
-// occupy most of the 256 CUs (256^3: 220 workgroups, 216 us a V-cycle level for
-// 271 us of half-sweeps); a 128^3 level would have 72 workgroups of 41 planes
-// (about 100 us for 56 us of launch-bound half-sweeps).
-constexpr size_t kFuseMinCells32 = size_t(1) << 23;
 
 inline hipStream_t as_stream(mf3d_stream s) { return reinterpret_cast<hipStream_t>(s); }
 
@@ -207,11 +202,12 @@ struct mf3d_workspace {
     // rr_partials) done by the V-cycle's first finest-level half-sweep
     bool fold_r = true;
     double* rr_partials = nullptr;
-    // fused smoothing passes (MF3D_TUNE_FUSE): 1 wherever the sizes allow, 0
-    // never, -1 on levels of at least kFuseMinCells32 cells
-    int fuse = -1;
     // ... and the (r, z) partials by its last finest-level half-sweep
     bool fold_rz = true;
+    // fused passes of large levels and window passes of small ones (MF3D_TUNE_FUSE):
+    // 1 wherever the sizes allow, 0 never, -1 where they are faster (fused32_pays,
+    // fused64_pays, kBlockMaxWindows)
+    int fuse = -1;
     size_t bytes = 0;
     std::vector<void*> owned;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -705,13 +701,14 @@ int mg_setup(mf3d_workspace* ws, hipStream_t s, const mf3d_grid& g, const mf3d_b
         if (!L.b32) MF3D_TRY(ws->alloc(&L.b32, L.n));
     }
     // fused smoothing passes: V(2,2) on colour-split levels with a colour-split
-    // coarse level
+    // coarse level, from the finest one down without a gap (a fused level's b is
+    // in b2, which the r update or the finer level's fused restriction writes)
     for (size_t l = 0; l < ws->lv.size(); ++l) {
         Level& L = ws->lv[l];
         L.fused = mixed && ws->fuse != 0 && !defer_coarse && L.order == ORDER_SPLIT &&
                   ws->lv[l + 1].order == ORDER_SPLIT && ws->pre == 2 && ws->post == 2 &&
-                  kern::fused32_ok(L.g, L.flo.type) &&
-                  (ws->fuse == 1 || L.n >= kFuseMinCells32);
+                  kern::fused32_ok(L.g, L.flo.type) && (l == 0 || ws->lv[l - 1].fused) &&
+                  (ws->fuse == 1 || kern::fused32_pays(L.g));
         if (!L.fused) continue;
         if (!L.xb) MF3D_TRY(ws->alloc(&L.xb, L.n / 2));
         if (!L.b2) MF3D_TRY(ws->alloc(&L.b2, L.n));

@@ -48,3 +48,39 @@ def test_first_gradients_wait_for_their_own_stream_only():
     log, = host_runs.run(NET + "show(gradients()[1])")
     assert "hipDeviceSynchronize" not in log and "hipMemset" not in log
     assert any("wgrad_kernel" in n for n in log)
+
+
+VCYCLE = """
+def vcycle(shape, levels, mixed, counts=(2, 2), fuse=-1):
+    g, bc = core.Grid3D(*shape).c(), core.BCSpec.darcy_x().c()
+    cfg = _lib.mf3d_head_solve_config()
+    lib.mf3d_default_config(ref(cfg))
+    cfg.mg_levels, cfg.precond_precision = levels, int(mixed)
+    cfg.coef_format = 1  # BF16
+    cfg.mg_pre_smooth, cfg.mg_post_smooth = counts
+    ws, v, n = C.c_void_p(), C.c_void_p(1 << 43), g.nx * g.ny * g.nz
+    assert lib.mf3d_workspace_create(ref(ws)) == 0
+    assert lib.mf3d_workspace_set_tuning(ws, 17, fuse) == 0
+    assert lib.mf3d_mg_setup(ws, None, ref(g), ref(bc), ref(cfg), v, n) == 0
+    stub.clear()
+    assert lib.mf3d_mg_precondition(ws, None, v, v, n) == 0
+    lib.mf3d_workspace_destroy(ws)
+    return stub.log()
+"""
+
+
+def _count(log, name):
+    return sum(name in n for n in log)
+
+
+@pytest.mark.parametrize("shape,levels,fused", [
+    ((256, 256, 256), 5, 1), ((1024, 128, 128), 5, 1), ((64, 64, 2048), 4, 1),
+    ((8192, 32, 32), 4, 1), ((2048, 512, 8), 3, 1), ((512, 512, 512), 5, 2),
+    # tiles of 28 places x 24 rows mostly outside the domain
+    ((1024, 8, 1024), 3, 0), ((16, 1024, 512), 3, 0), ((8, 1024, 1024), 3, 0),
+    ((16, 4096, 4096), 3, 0),
+    ((128, 128, 128), 5, 0)])
+def test_fp32_levels_in_fused_passes(shape, levels, fused):
+    """Two fused passes for each level whose tiles are full, counted from the finest."""
+    log, = host_runs.run(VCYCLE + f"show(vcycle({shape}, {levels}, True))")
+    assert _count(log, "fused_kernel") == 2 * fused
