@@ -105,11 +105,24 @@ struct Level {
     SmoothPlan plan;
 };
 
-// Levels of at most so many 8^3 windows are smoothed by window passes: two FP32
+// Levels of at most so many 8^3 windows may be smoothed by window passes: two FP32
 // workgroups fit a CU, so 512 are one wave (64^3: 19 us a V(2,2) level for 36 of
 // half-sweeps); FP64 ones fit once, and 512 are two waves (72x56x40, 315
 // windows: 36 us for 42; 64^3 takes the same 36). Another wave would cost what the launches do.
 constexpr size_t kBlockMaxWindows32 = 512, kBlockMaxWindows64 = 512;
+// Whether they are faster there. A pass holds up to two iterations; the restriction
+// rides on the last pre-smoothing one if that starts from zero or holds one, else it
+// is a launch more. A wave of windows takes about 9 us, twice a half-sweep launch of
+// such a level. One-workgroup levels (at most 4096 cells) run any number of
+// iterations in one launch, which two passes and more on a side do not beat.
+// FP64 V-cycles, windows / without: V(1,1) of 64^3 93 / 89 us, of 2048x16x4 44 / 34;
+// V(3,3) of 2048x16x4 76 / 69, of 16^3 80 / 51; V(4,4) of 16^3 96 / 53.
+bool block_pays(size_t windows, SmoothKind kind, int pre, int post, bool mixed) {
+    if (kind == SMOOTH_SMALL) return pre <= 2 && post <= 2;
+    const int passes = (pre + 1) / 2 + (post + 1) / 2 + (pre > 2 && pre % 2 == 0 ? 1 : 0);
+    const int waves = !mixed && windows > kBlockMaxWindows64 / 2 ? 2 : 1;
+    return 2 * passes * waves <= 2 * (pre + post) + 1;
+}
 
 inline hipStream_t as_stream(mf3d_stream s) { return reinterpret_cast<hipStream_t>(s); }
 
@@ -206,7 +219,7 @@ struct mf3d_workspace {
     bool fold_rz = true;
     // fused passes of large levels and window passes of small ones (MF3D_TUNE_FUSE):
     // 1 wherever the sizes allow, 0 never, -1 where they are faster (fused32_pays,
-    // fused64_pays, kBlockMaxWindows)
+    // fused64_pays, block_pays)
     int fuse = -1;
     size_t bytes = 0;
     std::vector<void*> owned;
@@ -721,7 +734,9 @@ int mg_setup(mf3d_workspace* ws, hipStream_t s, const mf3d_grid& g, const mf3d_b
         Level& L = ws->lv[l];
         L.block = ws->fuse != 0 && !defer_coarse && l + 1 < ws->lv.size() && ws->pre > 0 &&
                   ws->post > 0 && !L.fused && (!mixed || l > 0) &&
-                  kern::block_windows(L.g) <= (mixed ? kBlockMaxWindows32 : kBlockMaxWindows64);
+                  kern::block_windows(L.g) <= (mixed ? kBlockMaxWindows32 : kBlockMaxWindows64) &&
+                  (ws->fuse == 1 || block_pays(kern::block_windows(L.g), (SmoothKind)L.plan.kind,
+                                               ws->pre, ws->post, mixed));
         L.fused64 = ws->fuse != 0 && !mixed && !L.block && !defer_coarse &&
                     L.order64 == ORDER_SPLIT && ws->lv[l + 1].order64 == ORDER_SPLIT &&
                     ws->pre == 2 && ws->post == 2 && kern::fused64_ok(L.g) &&

@@ -67,6 +67,28 @@ def test_fp64_window_passes_match_half_sweeps(ctx, shape, levels, mix, counts):
     assert rel_l2(z[1], z[0]) < 1e-11
 
 
+@pytest.mark.parametrize("coef", list(ph.CoefFormat))
+@pytest.mark.parametrize("counts", [(2, 2), (1, 1), (3, 2), (4, 3)])
+@pytest.mark.parametrize("mix", ["darcy_x", "periodic_x_dirichlet_z", "all_periodic"])
+@pytest.mark.parametrize("shape,levels", [((80, 48, 32), 4), ((136, 16, 8), 3), ((104, 56, 40), 4)])
+def test_fp32_window_passes_every_face_format(ctx, shape, levels, mix, counts, coef):
+    """Every face format, smoothing counts for which the windows are slower included
+    (forced; with (2, 2) a forced level may take the fused passes: the default then)."""
+    fuse = -1 if counts == (2, 2) else 1
+    z = [_apply(ctx, shape, levels, mix, counts, F32, f, coef) for f in (0, fuse)]
+    assert torch.isfinite(z[1]).all()
+    assert torch.equal(z[0], z[1])
+
+
+@pytest.mark.parametrize("counts", [(1, 1), (3, 3), (4, 5)])
+@pytest.mark.parametrize("shape,levels", [((64, 64, 64), 4), ((48, 32, 16), 3)])
+def test_fp64_window_passes_forced(ctx, shape, levels, counts):
+    z = [_apply(ctx, shape, levels, "darcy_x", counts, ph.PrecondPrecision.FP64, f).cpu().numpy()
+         for f in (0, 1)]
+    assert np.isfinite(z[1]).all()
+    assert rel_l2(z[1], z[0]) < 1e-11  # (test_fp64_window_passes_match_half_sweeps)
+
+
 @pytest.mark.parametrize("graph", [0, 1])
 @pytest.mark.parametrize("fold_r", [0, 1])
 @pytest.mark.parametrize("shape", [(32, 32, 32), (40, 56, 24)])

@@ -84,3 +84,17 @@ def test_fp32_levels_in_fused_passes(shape, levels, fused):
     """Two fused passes for each level whose tiles are full, counted from the finest."""
     log, = host_runs.run(VCYCLE + f"show(vcycle({shape}, {levels}, True))")
     assert _count(log, "fused_kernel") == 2 * fused
+
+
+# V-cycle levels: 64^3 two waves of FP64 windows, 32^3 one, 16^3 and below one workgroup
+@pytest.mark.parametrize("mixed,counts,passes", [
+    (False, (2, 2), 2 + 2 + 2), (False, (1, 1), 0 + 2 + 2), (False, (2, 1), 0 + 2 + 2),
+    (False, (3, 3), 0 + 4 + 0), (False, (4, 4), 0 + 4 + 0), (False, (1, 3), 0 + 3 + 0),
+    # FP32: not the finest level
+    (True, (2, 2), 0 + 2 + 2), (True, (1, 1), 0 + 2 + 2), (True, (4, 4), 0 + 4 + 0)])
+def test_small_levels_in_window_passes(mixed, counts, passes):
+    """Window passes where they are fewer waves than half the launches they replace."""
+    log, = host_runs.run(VCYCLE + f"show(vcycle((64, 64, 64), 4, {mixed}, {counts}))")
+    assert _count(log, "block_kernel") == passes
+    log, = host_runs.run(VCYCLE + f"show(vcycle((64, 64, 64), 4, {mixed}, {counts}, fuse=0))")
+    assert _count(log, "block_kernel") == 0
