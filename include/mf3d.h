@@ -275,7 +275,9 @@ int mf3d_workspace_solve_counts(const mf3d_workspace* ws, long* op_applications,
 /* Extension: num_iters GSRB iterations on level `level` of the current
  * hierarchy, in place on the workspace's own correction and right-hand side
  * of that level (level 0: the preconditioner's input/output buffers), in the
- * set-up's precision. For timing and testing the smoother in situ. */
+ * set-up's precision. For timing and testing the smoother in situ (a level that
+ * MF3D_TUNE_FUSE's FP32 passes smooth holds its right-hand side in their order:
+ * set 0 to test there). */
 int mf3d_mg_smooth(mf3d_workspace* ws, mf3d_stream stream, int level, int num_iters);
 
 /* Number of levels of the current hierarchy (0 before set-up). */

@@ -88,9 +88,9 @@ struct Level {
     bool fused64 = false;   // FP64 smoothing in fused passes (fused64.hip), the same way
     double* x2 = nullptr;
     float* x32s = nullptr;
-    bool fused = false;     // FP32 smoothing in fused passes, which use
-    float* xb = nullptr;    // the black values between pre- and post-smoothing,
-    float* b2 = nullptr;    // the right-hand side as (red, black) pairs
+    bool fused = false;     // FP32 smoothing in fused passes, which take b32 as (red,
+                            // black) pairs of a place and use
+    float* xb = nullptr;    // the black values between pre- and post-smoothing
     void* rec = nullptr;    // and face records
     FaceSet f64;            // FP64 faces (operator on level 0, FP64 V-cycle)
     FaceSet flo;            // low-precision faces of the FP32 V-cycle
@@ -222,16 +222,50 @@ struct mf3d_workspace {
     // fused64_pays, block_pays)
     int fuse = -1;
     size_t bytes = 0;
-    std::vector<void*> owned;
+    std::vector<std::pair<void*, size_t>> owned;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
 
+    // The buffers of fused and window passes only make a solve faster: a level
+    // whose buffers do not fit keeps its half-sweeps, and they give way to any
+    // other buffer of the workspace.
+    bool try_bytes(void** p, size_t nbytes) {
+        if (*p) return true;
+        void* q = nullptr;
+        if (hipMalloc(&q, nbytes) != hipSuccess) {
+            (void)hipGetLastError();  // (reported by the next launch otherwise)
+            return false;
+        }
+        owned.emplace_back(q, nbytes);
+        bytes += nbytes;
+        *p = q;
+        return true;
+    }
+    void give_back(void* q) {
+        for (size_t i = 0; q && i < owned.size(); ++i) {
+            if (owned[i].first != q) continue;
+            (void)hipFree(q);  // (waits for the work that uses it)
+            bytes -= owned[i].second;
+            owned.erase(owned.begin() + i);
+            return;
+        }
+    }
+    void drop_passes(Level& L) {
+        for (void* q : {(void*)L.x2, (void*)L.x32s, (void*)L.xb, L.rec}) give_back(q);
+        L.x2 = nullptr, L.x32s = L.xb = nullptr, L.rec = nullptr;
+        L.block = L.fused = L.fused64 = false;
+    }
     int alloc_bytes(void** p, size_t nbytes) {
         void* q = nullptr;
         if (nbytes == 0) nbytes = 8;
         hipError_t e = hipMalloc(&q, nbytes);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            for (Level& L : lv) drop_passes(L);
+            e = hipMalloc(&q, nbytes);
+        }
         if (e != hipSuccess)
             return fail(MF3D_ERR_ALLOC, std::string("hipMalloc: ") + hipGetErrorString(e));
-        owned.push_back(q);
+        owned.emplace_back(q, nbytes);
         bytes += nbytes;
         *p = q;
         return MF3D_OK;
@@ -260,7 +294,7 @@ struct mf3d_workspace {
     }
     void release() {
         drain_coarse();
-        for (void* q : owned) (void)hipFree(q);
+        for (auto& q : owned) (void)hipFree(q.first);
         owned.clear();
         bytes = 0;
         lv.clear();
@@ -714,8 +748,8 @@ int mg_setup(mf3d_workspace* ws, hipStream_t s, const mf3d_grid& g, const mf3d_b
         if (!L.b32) MF3D_TRY(ws->alloc(&L.b32, L.n));
     }
     // fused smoothing passes: V(2,2) on colour-split levels with a colour-split
-    // coarse level, from the finest one down without a gap (a fused level's b is
-    // in b2, which the r update or the finer level's fused restriction writes)
+    // coarse level, from the finest one down without a gap (a fused level's b is in
+    // pairs, which the r update or the finer level's fused restriction writes)
     for (size_t l = 0; l < ws->lv.size(); ++l) {
         Level& L = ws->lv[l];
         L.fused = mixed && ws->fuse != 0 && !defer_coarse && L.order == ORDER_SPLIT &&
@@ -723,10 +757,10 @@ int mg_setup(mf3d_workspace* ws, hipStream_t s, const mf3d_grid& g, const mf3d_b
                   kern::fused32_ok(L.g, L.flo.type) && (l == 0 || ws->lv[l - 1].fused) &&
                   (ws->fuse == 1 || kern::fused32_pays(L.g));
         if (!L.fused) continue;
-        if (!L.xb) MF3D_TRY(ws->alloc(&L.xb, L.n / 2));
-        if (!L.b2) MF3D_TRY(ws->alloc(&L.b2, L.n));
-        if (!L.rec) MF3D_TRY(ws->alloc_bytes(&L.rec, kern::fused32_face_bytes(L.g)));
-        MF3D_TRY(kern::fused32_pack(s, L.g, ws->bct, L.flo, L.rec));
+        if (ws->try_bytes((void**)&L.xb, L.n / 2 * sizeof(float)) &&
+            ws->try_bytes(&L.rec, kern::fused32_face_bytes(L.g)))
+            MF3D_TRY(kern::fused32_pack(s, L.g, ws->bct, L.flo, L.rec));
+        else ws->drop_passes(L);
     }
     // window passes on small levels (the batched solve has its own launches, whose
     // (r, z) grouping the FP32 finest level shares)
@@ -742,8 +776,9 @@ int mg_setup(mf3d_workspace* ws, hipStream_t s, const mf3d_grid& g, const mf3d_b
                     ws->pre == 2 && ws->post == 2 && kern::fused64_ok(L.g) &&
                     (ws->fuse == 1 || kern::fused64_pays(L.g));
         if (!L.block && !L.fused64) continue;
-        if (mixed && !L.x32s) MF3D_TRY(ws->alloc(&L.x32s, L.n));
-        if (!mixed && !L.x2) MF3D_TRY(ws->alloc(&L.x2, L.n));
+        if (!(mixed ? ws->try_bytes((void**)&L.x32s, L.n * sizeof(float))
+                    : ws->try_bytes((void**)&L.x2, L.n * sizeof(double))))
+            ws->drop_passes(L);
     }
     // the FP64 operator's h = 1 / (2 K): built together with the 16-bit faces
     // when level 0 is the colour-split level of the FP32 V-cycle (decided
@@ -846,11 +881,11 @@ int vcycle(mf3d_workspace* ws, hipStream_t s, size_t l, T* x, const T* b, bool z
     Level& C = ws->lv[l + 1];
     const int fo = V::order(L), co = V::order(C);
     if constexpr (std::is_same<T, float>::value) {
-        if (L.fused) {  // zero start; b is in b2
+        if (L.fused) {  // zero start
             MF3D_TRY(kern::fused32_pre(s, L.g, ws->bct, ws->pin, cs * dx2, 1.0 / (cs * dx2), L.xb,
-                                       L.b2, F.type, L.rec, C.fused ? C.b2 : V::b(C), C.fused));
+                                       b, F.type, L.rec, V::b(C), C.fused));
             MF3D_TRY(vcycle<T>(ws, s, l + 1, V::x(C), V::b(C), true));
-            return kern::fused32_post(s, L.g, ws->bct, ws->pin, cs * dx2, L.xb, x, L.b2, F.type,
+            return kern::fused32_post(s, L.g, ws->bct, ws->pin, cs * dx2, L.xb, x, b, F.type,
                                       L.rec, V::x(C), rz);
         }
     }
@@ -1048,7 +1083,7 @@ int precondition(mf3d_workspace* ws, hipStream_t s, const double* r, double* z,
     if (ru && !fold) return fail(MF3D_ERR_UNSUPPORTED, "the r update needs the folded r sweep");
     // fused passes take b as it is; the r update makes it (or the conversion)
     const bool sweep_r = fold && !L0.fused;
-    if (L0.fused) MF3D_TRY(kern::r_to_b(s, L0.g, r, ru, L0.b2));
+    if (L0.fused) MF3D_TRY(kern::r_to_b(s, L0.g, r, ru, L0.b32));
     else if (!sweep_r) MF3D_TRY(kern::to_f32(s, r, L0.b32, L0.g, L0.order));
     // the last finest half-sweep forms (r, z): z in x32, post-smoothing on level 0
     const bool rz_fold = !z && rz_partials && ws->fold_rz && ws->post > 0 && fold;

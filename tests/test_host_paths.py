@@ -98,3 +98,49 @@ def test_small_levels_in_window_passes(mixed, counts, passes):
     assert _count(log, "block_kernel") == passes
     log, = host_runs.run(VCYCLE + f"show(vcycle((64, 64, 64), 4, {mixed}, {counts}, fuse=0))")
     assert _count(log, "block_kernel") == 0
+
+
+SOLVE = """
+def solve(shape, levels, mixed, fuse, h=1 << 43):
+    g, bc = core.Grid3D(*shape).c(), core.BCSpec.darcy_x().c()
+    cfg, res = _lib.mf3d_head_solve_config(), _lib.mf3d_head_solve_result()
+    lib.mf3d_default_config(ref(cfg))
+    cfg.mg_levels, cfg.precond_precision, cfg.coef_format = levels, int(mixed), 1
+    ws, n = C.c_void_p(), g.nx * g.ny * g.nz
+    assert lib.mf3d_workspace_create(ref(ws)) == 0
+    assert lib.mf3d_workspace_set_tuning(ws, 17, fuse) == 0
+    stub.clear()
+    st = lib.mf3d_solve_head(ws, None, ref(g), ref(bc), ref(cfg), C.c_void_p(1 << 43),
+                             C.c_void_p(h), n, ref(res))
+    log, used, said = stub.log(), stub.in_use(), lib.mf3d_workspace_bytes(ws)
+    lib.mf3d_workspace_destroy(ws)
+    assert stub.in_use() == 0 and used == said
+    return st, used, log
+"""
+
+
+@pytest.mark.parametrize("head", [1 << 43, (1 << 43) + 8])  # the second is solved in a copy
+@pytest.mark.parametrize("shape,levels,mixed", [((256, 256, 256), 5, True),
+                                                ((256, 256, 256), 5, False),
+                                                ((64, 64, 64), 4, False),
+                                                ((128, 128, 128), 5, True)])
+def test_memory_for_half_sweeps_is_enough(shape, levels, mixed, head):
+    """The fused and window passes' buffers give way: a solve that fits without them
+    fits, on half-sweeps, and with room for some of them takes those."""
+    off, on, tight, less, some = host_runs.run(SOLVE + f"""
+args = {shape}, {levels}, {mixed}
+off, on = solve(*args, 0, {head}), solve(*args, -1, {head})
+show(off); show(on)
+stub.limit(off[1])
+show(solve(*args, -1, {head}))
+stub.limit(off[1] - 1)
+show(solve(*args, -1, {head}))
+stub.limit((off[1] + on[1]) // 2)
+show(solve(*args, -1, {head}))
+""")
+    passes = lambda log: _count(log, "block_kernel") + _count(log, "fused")  # noqa: E731
+    assert off[0] == on[0] == tight[0] == some[0] == 0 and less[0] == 5  # MF3D_ERR_ALLOC
+    assert passes(on[2]) > passes(off[2]) == 0
+    assert off[1] < on[1] <= 1.15 * off[1]
+    assert tight[1] == off[1] and passes(tight[2]) == 0
+    assert off[1] <= some[1] <= (off[1] + on[1]) // 2
