@@ -258,7 +258,8 @@ enum {
     MF3D_TUNE_FUSE = 17                 /* two GSRB iterations of a large colour-split level in
                                            one pass: 1 wherever the sizes allow, 0 never (nor
                                            in windows of a small one), -1 (default): on the
-                                           levels where it is faster */
+                                           levels where it is faster. The heads of mixed
+                                           solves do not depend on it */
 };
 int mf3d_workspace_set_tuning(mf3d_workspace* ws, int key, long value);
 

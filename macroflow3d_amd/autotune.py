@@ -4,8 +4,8 @@ Its choices change where and when the work runs, not what is computed:
 
 * ``sweep_block``: threads per workgroup of the colour-split red-black sweeps
   of the mixed V-cycle (64, 128, 256, 512): a runtime launch parameter; each
-  cell's arithmetic and every partial sum are the same for each size, so the
-  head is bitwise unchanged;
+  cell's arithmetic is the same for each size, the (r, r) and (r, z) partials
+  that the sweeps form are regrouped;
 * ``graph``: replaying one captured PCG iteration or launching its kernels
   one by one (single mixed-precision solves and batches): bitwise unchanged;
 * ``op_tile``: the finest-level FP64 operator on plane tiles staged in LDS or

@@ -145,6 +145,14 @@ __global__ void __launch_bounds__(kBlock)
     x[o] = gs_value(f, v, b[o], bs, pin && o == 0);
 }
 
+// acc + the (r, z) terms of two neighbouring cells of a row. Every way of forming
+// (r, z) of the FP32 V-cycle adds the 8 cells of a thread in their natural order, by
+// fma, and the 2048 of a workgroup in one tree: single solves, on whatever kernels,
+// and batched ones agree bit for bit.
+__device__ __forceinline__ double rz_pair(double2 r, double z0, double z1, double acc) {
+    return fma(r.y, z1, fma(r.x, z0, acc));
+}
+
 // neighbours (x+, x-, y+, y-, z+, z-) of cell (i,j,k) from the opposite
 // colour's array O; r0 = (j + ny k) * nx/2 is the cell's row offset
 template <typename T>
@@ -587,12 +595,7 @@ __device__ __forceinline__ void split4_body(const Dims& d, const BcTypes& bc, in
     if (RZ) {  // own cells at natural 2e + p, the other colour at 2e + 1 - p
         double acc = 0.0;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const double2 v2 = rzr[e];
-            const double ro = p ? v2.y : v2.x, rt = p ? v2.x : v2.y;
-            acc += ro * (double)res[e];
-            acc += rt * (double)oc[e];
-        }
+        for (int e = 0; e < 4; ++e) acc = rz_pair(rzr[e], p ? oc[e] : res[e], p ? res[e] : oc[e], acc);
         const double sb = block_sum_dyn(valid ? acc : 0.0);
         if (threadIdx.x == 0) rz->partials[blk] = sb;
     }
@@ -1551,11 +1554,7 @@ __device__ __forceinline__ void split8_body(const Dims& d, const float* __restri
         if (DOT) {
             const double2* rp = reinterpret_cast<const double2*>(r + e0);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const double2 rv = rp[e];
-                prod += rv.x * z[2 * e];
-                prod += rv.y * z[2 * e + 1];
-            }
+            for (int e = 0; e < 4; ++e) prod = rz_pair(rp[e], z[2 * e], z[2 * e + 1], prod);
         }
     }
     if (DOT) {  // the block's 2048 consecutive cells: partials[reduce_blocks(n)]

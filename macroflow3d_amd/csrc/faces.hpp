@@ -99,19 +99,16 @@ bool fused32_pays(const mf3d_grid& g);  // faster than the half-sweeps there
 size_t fused32_face_bytes(const mf3d_grid& g);
 int fused32_pack(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, const FaceSet& F,
                  void* faces);
-// (r, z) partials of fused32_post
-unsigned fused32_partials(const mf3d_grid& g);
 // two GSRB iterations from zero: xb = the black values, bcoarse = restriction of
 // the residual's red cells. b (and bcoarse with pairs): (red, black) per place;
 // bcoarse without pairs: colour-split
 int fused32_pre(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, double bs,
                 double rs, float* xb, const float* b, CoefType t, const void* faces,
                 float* bcoarse, bool pairs);
-// x (colour-split) = two GSRB iterations from xb + the prolonged xc
-// (colour-split); rz (nullable): the (r, x) partials too
+// x (colour-split) = two GSRB iterations from xb + the prolonged xc (colour-split)
 int fused32_post(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, double bs,
                  const float* xb, float* x, const float* b, CoefType t, const void* faces,
-                 const float* xc, const RzDot* rz);
+                 const float* xc);
 // b = (float) r in pairs; ru: the PCG residual update first, with the (r, r)
 // partials (one per 2048 cells)
 int r_to_b(hipStream_t s, const mf3d_grid& g, const double* r, const RUpd* ru, float* b);

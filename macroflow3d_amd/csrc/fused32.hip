@@ -2,7 +2,7 @@
 //
 // Two red-black Gauss-Seidel iterations (four half-sweeps, gsrb_3d.cu:29-366)
 // and what follows or precedes them in the V-cycle (v_cycle.cu:36-74: residual
-// and restriction, prolongation, PCG's (r, z)) in ONE pass over the level.
+// and restriction, or prolongation) in ONE pass over the level.
 //
 // Bound: the half-sweeps one by one stream the level's faces four times (12
 // bytes a cell each, 48 together, and 12.5 more for the residual), and on
@@ -39,8 +39,8 @@
 // pairs per place for the same reason.
 //
 // MI355X, bf16 faces, this pass against the half-sweeps (and residual) it replaces:
-//   512^3 pre + restriction 690 us (1240), post + (r, z) 808 us (1394);
-//   256^3 100 us (123), 116 us (148). The (r, z) costs 29 us at 256^3, r's HBM time.
+//   512^3 pre + restriction 702 us (1240), post 746 us (1286);
+//   256^3 99 us (123), 86 us (124).
 // About two thirds of the vector issue slots are used; at 512^3 the misses of the
 // tiles' rims (1.4 times the bytes) take 4.8 TB/s.
 
@@ -62,7 +62,7 @@ constexpr int kPadLds = kTX + 1;               // neighbours of the tile's rim r
 constexpr int kSlots = kThreads + 2 * kPadLds;
 
 enum { START_ZERO = 0, START_PROLONG = 1 };
-enum { END_NONE = 0, END_RESTRICT = 1, END_RZ = 2 };
+enum { END_NONE = 0, END_RESTRICT = 1 };
 
 struct FGeo {
     int nx, ny, nz, h;
@@ -119,7 +119,6 @@ struct Fused {
     struct Lds {
         float x[STAGES + 1][2][kSlots];  // [s]: values half-sweep s left (0: black on arrival)
         F fx[2][kSlots + kTY], fy[2][kSlots];  // fx: then the column beyond the tile
-        double part[16];
     };
 
     struct In {  // one plane on its way
@@ -127,7 +126,6 @@ struct Fused {
         unsigned e;       // faces beyond the tile (END_RESTRICT)
         float2 b;
         float xb, par;
-        double2 r;        // END_RZ: r of the pair, STAGES planes below
     };
 
     static __device__ __forceinline__ void run(Lds& L, const FGeo& G, const BcTypes& bc, int pin,
@@ -136,10 +134,8 @@ struct Fused {
                                                const float2* __restrict__ b,
                                                const Rec* __restrict__ faces,
                                                const float* __restrict__ xc,
-                                               float* __restrict__ bcoarse,
-                                               const double* __restrict__ r64,
-                                               double* __restrict__ partials, int bx, int by,
-                                               int bz, long blk) {
+                                               float* __restrict__ bcoarse, int bx, int by,
+                                               int bz) {
         const int tid = (int)threadIdx.x;
         const int tx = tid & (kTX - 1), ty = tid / kTX;
         const int h = G.h, ny = G.ny, nz = G.nz;
@@ -155,11 +151,6 @@ struct Fused {
         const bool store = tx >= kHX && tx < kTX - kHX && ty >= kHY && ty < kTY - kHY && m < h &&
                            j < ny;
         const unsigned pl0 = (unsigned)mc + (unsigned)h * (unsigned)jc;
-        // END_RZ: only stored places need r; the rim repeats the nearest one's (a
-        // rim of its own would add half again to r's traffic)
-        const unsigned plr =
-            (unsigned)min(bx * kIX - kHX + min(max(tx, kHX), kTX - kHX - 1), h - 1) +
-            (unsigned)h * (unsigned)min(by * kIY - kHY + min(max(ty, kHY), kTY - kHY - 1), ny - 1);
         const long half = G.half, hn = (long)h * ny;
         const long HC = half >> 3;  // one colour of the coarse level
         const unsigned hc = (unsigned)h >> 1, nyc = (unsigned)ny >> 1;
@@ -195,7 +186,6 @@ struct Fused {
             lx[q] = ly[q] = lz[q] = lyn[q] = F{0u};
             lxn[q] = br[q] = bb[q] = xr[q] = xb[q] = 0.0f;
         }
-        double acc = 0.0;
         float even = 0.0f;  // END_RESTRICT: the pair of rows' residuals in the even plane
 
         In in[AHEAD];
@@ -212,8 +202,6 @@ struct Fused {
                 n.par = ldo<float>(xc + (long)hc * nyc * K,
                                    4u * ((c ? (unsigned)HC : 0u) + ((unsigned)mc >> 1) + hc * J));
             }
-            if (END == END_RZ)
-                n.r = ldo<double2>(r64 + 2 * hn * min(max(k - STAGES, 0), nz - 1), 16u * plr);
         };
 
         const int kbeg = k0 - WARM, kend = k1 - 1 + LAST;
@@ -242,11 +230,6 @@ struct Fused {
             if (END == END_RESTRICT) {
                 ext = nxt.e;
                 asm volatile("" : "+v"(ext));
-            }
-            double2 rq{0.0, 0.0};
-            if (END == END_RZ) {
-                rq = nxt.r;
-                asm volatile("" : "+v"(rq.x), "+v"(rq.y));
             }
             asm volatile("" : "+v"(lx[U].w), "+v"(ly[U].w), "+v"(lz[U].w));
             asm volatile("" : "+v"(br[U]), "+v"(bb[U]), "+v"(xb[U]));
@@ -343,10 +326,6 @@ struct Fused {
                     } else {
                         sto(xout + hn * q, 4u * pl0, xb[a]);
                     }
-                    if (END == END_RZ) {  // cell i = 2m is red when j + k - 4 is even (p = 1)
-                        acc += rq.x * (double)(p ? xr[a] : xb[a]);
-                        acc += rq.y * (double)(p ? xb[a] : xr[a]);
-                    }
                 }
             }
             if (END == END_RESTRICT) {
@@ -398,17 +377,6 @@ struct Fused {
                 step(std::integral_constant<int, 7>{}, k + 7);
             }
         }
-        if (END == END_RZ) {
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-            if ((tid & 63) == 0) L.part[tid >> 6] = acc;
-            __syncthreads();
-            if (tid == 0) {
-                double s = 0.0;
-                for (int w = 0; w < kThreads / 64; ++w) s += L.part[w];
-                partials[blk] = s;
-            }
-        }
     }
 };
 
@@ -417,15 +385,13 @@ __global__ void __launch_bounds__(kThreads)
     fused_kernel(FGeo G, BcTypes bc, int pin, float bs, float rs, const float* __restrict__ xin,
                  float* __restrict__ xout, const float2* __restrict__ b,
                  const Rec* __restrict__ faces, const float* __restrict__ xc,
-                 float* __restrict__ bcoarse, const double* __restrict__ r64,
-                 double* __restrict__ partials) {
+                 float* __restrict__ bcoarse) {
     __shared__ typename Fused<TC, START, END>::Lds L;
     const long blk = xcd_block((long)G.tx * G.ty * G.chunks);
     if (blk < 0) return;  // whole workgroup
     const int t = (int)(blk % ((long)G.tx * G.ty)), bz = (int)(blk / ((long)G.tx * G.ty));
     const int by = t / G.tx, bx = t - by * G.tx;
-    Fused<TC, START, END>::run(L, G, bc, pin, bs, rs, xin, xout, b, faces, xc, bcoarse, r64,
-                               partials, bx, by, bz, blk);
+    Fused<TC, START, END>::run(L, G, bc, pin, bs, rs, xin, xout, b, faces, xc, bcoarse, bx, by, bz);
 }
 
 // face records of a level from its half-sweep arrays
@@ -540,12 +506,11 @@ FGeo fgeo_of(const mf3d_grid& g) {
 template <typename TC, int START, int END>
 int launch(hipStream_t s, const FGeo& G, const BcTypes& bc, bool pin, double bs, double rs,
            const float* xin, float* xout, const float* b, const void* faces, const float* xc,
-           float* bcoarse, const RzDot* rz) {
+           float* bcoarse) {
     const long nb = (long)G.tx * G.ty * G.chunks;
     fused_kernel<TC, START, END><<<xcd_round((size_t)nb), kThreads, 0, s>>>(
         G, bc, pin ? 1 : 0, (float)bs, (float)rs, xin, xout, reinterpret_cast<const float2*>(b),
-        static_cast<const Rec*>(faces), xc, bcoarse, rz ? rz->r : nullptr,
-        rz ? rz->partials : nullptr);
+        static_cast<const Rec*>(faces), xc, bcoarse);
     MF3D_HIP_TRY(hipGetLastError());
     return MF3D_OK;
 }
@@ -609,11 +574,6 @@ int fused32_pack(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, const Fac
     return MF3D_OK;
 }
 
-unsigned fused32_partials(const mf3d_grid& g) {
-    const FGeo G = fgeo_of(g);
-    return (unsigned)(G.tx * G.ty * G.chunks);
-}
-
 int fused32_pre(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, double bs,
                 double rs, float* xb, const float* b, CoefType t, const void* faces,
                 float* bcoarse, bool pairs) {
@@ -621,26 +581,22 @@ int fused32_pre(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, 
     FGeo G = fgeo_of(g);
     G.bcp = pairs ? 1 : 0;
     if (t == COEF_BF16)
-        return launch<__hip_bfloat16, START_ZERO, END_RESTRICT>(
-            s, G, bc, pin, bs, rs, nullptr, xb, b, faces, nullptr, bcoarse, nullptr);
+        return launch<__hip_bfloat16, START_ZERO, END_RESTRICT>(s, G, bc, pin, bs, rs, nullptr, xb,
+                                                                b, faces, nullptr, bcoarse);
     return launch<__half, START_ZERO, END_RESTRICT>(s, G, bc, pin, bs, rs, nullptr, xb, b, faces,
-                                                    nullptr, bcoarse, nullptr);
+                                                    nullptr, bcoarse);
 }
 
 int fused32_post(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, double bs,
                  const float* xb, float* x, const float* b, CoefType t, const void* faces,
-                 const float* xc, const RzDot* rz) {
+                 const float* xc) {
     MF3D_TRY(check(g, t));
     const FGeo G = fgeo_of(g);
     if (t == COEF_BF16)
-        return rz ? launch<__hip_bfloat16, START_PROLONG, END_RZ>(s, G, bc, pin, bs, 0.0, xb, x, b,
-                                                                  faces, xc, nullptr, rz)
-                  : launch<__hip_bfloat16, START_PROLONG, END_NONE>(s, G, bc, pin, bs, 0.0, xb, x,
-                                                                    b, faces, xc, nullptr, rz);
-    return rz ? launch<__half, START_PROLONG, END_RZ>(s, G, bc, pin, bs, 0.0, xb, x, b, faces, xc,
-                                                      nullptr, rz)
-              : launch<__half, START_PROLONG, END_NONE>(s, G, bc, pin, bs, 0.0, xb, x, b, faces,
-                                                        xc, nullptr, rz);
+        return launch<__hip_bfloat16, START_PROLONG, END_NONE>(s, G, bc, pin, bs, 0.0, xb, x, b,
+                                                               faces, xc, nullptr);
+    return launch<__half, START_PROLONG, END_NONE>(s, G, bc, pin, bs, 0.0, xb, x, b, faces, xc,
+                                                   nullptr);
 }
 
 int r_to_b(hipStream_t s, const mf3d_grid& g, const double* r, const RUpd* ru, float* b) {

@@ -886,7 +886,7 @@ int vcycle(mf3d_workspace* ws, hipStream_t s, size_t l, T* x, const T* b, bool z
                                        b, F.type, L.rec, V::b(C), C.fused));
             MF3D_TRY(vcycle<T>(ws, s, l + 1, V::x(C), V::b(C), true));
             return kern::fused32_post(s, L.g, ws->bct, ws->pin, cs * dx2, L.xb, x, b, F.type,
-                                      L.rec, V::x(C), rz);
+                                      L.rec, V::x(C));
         }
     }
     MF3D_TRY(kern::smooth_faces(s, L.g, ws->bct, ws->pin, cs * dx2, x, b, F, ws->pre,
@@ -1085,13 +1085,15 @@ int precondition(mf3d_workspace* ws, hipStream_t s, const double* r, double* z,
     const bool sweep_r = fold && !L0.fused;
     if (L0.fused) MF3D_TRY(kern::r_to_b(s, L0.g, r, ru, L0.b32));
     else if (!sweep_r) MF3D_TRY(kern::to_f32(s, r, L0.b32, L0.g, L0.order));
-    // the last finest half-sweep forms (r, z): z in x32, post-smoothing on level 0
-    const bool rz_fold = !z && rz_partials && ws->fold_rz && ws->post > 0 && fold;
+    // the last finest half-sweep forms (r, z): z in x32, post-smoothing on level 0. (A
+    // fused pass could form it per tile, for 1 to 3 % of a solve, but then a batched
+    // realisation's beta and head would differ from its single solve's in the last bits.)
+    const bool rz_fold = !z && rz_partials && ws->fold_rz && ws->post > 0 && sweep_r;
     const RzDot rzd{r, rz_partials};
     MF3D_TRY(vcycle<float>(ws, s, 0, L0.x32, L0.b32, true, sweep_r ? r : nullptr, false,
                            sweep_r ? ru : nullptr, rz_fold ? &rzd : nullptr));
     if (rz_fold) {
-        if (np_rz) *np_rz = L0.fused ? kern::fused32_partials(L0.g) : sweep_partials(ws);
+        if (np_rz) *np_rz = sweep_partials(ws);
         return MF3D_OK;
     }
     if (!z) return rz_partials ? kern::rz_split8(s, L0.x32, L0.g, r, rz_partials) : MF3D_OK;

@@ -195,10 +195,11 @@ class FlowWorkspace:
         folded PCG steps, plane-tile operator and its chunk depth, the FP64
         sweeps' workgroup target, graph replay, fused smoothing passes);
         applied at the next set-up
-        or solve. None changes the result beyond rounding; the sweep block
-        size of the mixed V-cycle and the graph replay leave it bit-identical,
-        the operator tile and chunk depth regroup the (p, Ap) partials, the
-        FP64 sweeps' block size and workgroup target the (r, z) partials."""
+        or solve. None changes the result beyond rounding; the graph replay
+        and, for mixed solves, the fused passes leave it bit-identical, the
+        operator tile and chunk depth regroup the (p, Ap) partials, the
+        sweeps' block size and the FP64 sweeps' workgroup target the (r, z)
+        partials."""
         _lib.call("mf3d_workspace_set_tuning", self._h, int(key), int(value))
 
     def solve_counts(self) -> tuple[int, int]:

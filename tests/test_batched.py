@@ -85,3 +85,30 @@ def test_batched_second_call_reuses_workspaces(ctx):
     for w in wss:
         w.close()
 
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shapes,levels", [([(32, 32, 32), (96, 96, 96), (64, 32, 48)], 4),
+                                           ([(256, 256, 128)], 6)])
+def test_batched_heads_equal_single_ones(ctx, shapes, levels):
+    """The head and the iteration count of a realisation are its single solve's, bit
+    for bit, whatever kernels the single solve's levels take (256x256x128: fused passes
+    by default)."""
+    reals = _realisations(ctx, shapes, 700)
+    bc, cfg = BCSpec.darcy_x(), ph.HeadSolveConfig.mixed(1e-10, levels)
+    hs = [ctx.zeros(g.num_cells()) for g, _ in reals]
+    wss = [ph.FlowWorkspace() for _ in reals]
+    res = ph.solve_head_batched(hs, [K for _, K in reals], [g for g, _ in reals], bc, cfg, ctx, wss)
+    for fuse in (-1, 0, 1):
+        for fold_rz in (1, 0):
+            ws1 = ph.FlowWorkspace()
+            ws1.set_tuning(ws1.TUNE_FUSE, fuse)
+            ws1.set_tuning(ws1.TUNE_FOLD_RZ, fold_rz)
+            for (g, K), h, r in zip(reals, hs, res):
+                h1 = ctx.zeros(g.num_cells())
+                r1 = ph.solve_head(h1, K, g, bc, cfg, ctx, ws1)
+                assert r.num_iterations == r1.num_iterations
+                assert torch.equal(h, h1), (g, fuse, fold_rz)
+            ws1.close()
+    for w in wss:
+        w.close()
