@@ -14,6 +14,7 @@
 //   Neumann face: 0; periodic face: harmonic mean across the wrap.
 
 #include <algorithm>
+#include <type_traits>
 
 #include "kernels.hpp"
 #include "reduce.hpp"
@@ -133,41 +134,60 @@ __global__ void __launch_bounds__(kBlock)
 // ---- velocity diagnostics (velocity_diagnostics.cu:46-177) -------------------
 // Everything but the divergence is differences of cell-centred means (u: of the
 // cell's two x faces, and so on), so a cell needs its own six faces and its
-// neighbours' means. A workgroup owns 64 x 16 columns (a wave a row; rows 0 and 15
-// only supply means: 64 x 14 cells a tile) and marches kz planes up: each thread
-// forms its column's means from five loads a plane, two planes ahead of their use,
-// keeps them for three planes (z differences) and shares plane k's through LDS (two
-// buffers, one barrier a plane).
+// neighbours' means. A workgroup owns 64 columns by 4, 8 or 16 rows (a wave a row; the
+// first and last row only supply means unless the tile holds every row) and marches
+// kz planes up: each thread forms its column's means from five loads a plane, two
+// planes ahead of their use, keeps them for three planes (z differences) and shares
+// plane k's through LDS (two buffers, one barrier a plane).
 // Bound: HBM, the three padded components read once and the three cell fields
-// written once, 48 bytes a cell. 250x190x130: with 17 loads a cell and plane, each
-// plane's waited for at once, 105 us (2.8 TB/s); now 77 us (3.9 TB/s), 94 with
-// ordinary stores, which push the velocities out of the Infinity Cache.
-constexpr int kDiagX = 64, kDiagRows = 16, kDiagY = kDiagRows - 2;
-constexpr int kDiagBlock = kDiagX * kDiagRows;
+// written once, 48 bytes a cell. 250x190x130, with the statistics' second stage: with 17
+// loads a cell and plane, each plane's waited for at once, 112 us; now 62 (the kernel
+// 55, 5.4 TB/s). With ordinary stores, which push the velocities out of the Infinity
+// Cache, 84.
+constexpr int kDiagX = 64;
 constexpr int kDiagQ = 9;  // per-workgroup partials: (min, max, sum) x 3 fields
 
-// the number of z-chunks that makes the fewest steps with one workgroup a CU
 struct Tiles {
     int tx, ty, kz;
+    int rows;
+    int halo;  // rows that only supply means, at either end: none where a tile needs none
     long nblocks;
+    long steps;
 };
-Tiles tiles_of(int nx, int ny, int nz) {
-    Tiles t{(nx + kDiagX - 1) / kDiagX, (ny + kDiagY - 1) / kDiagY, 0, 0};
-    long best = -1;
-    for (int c = 1; c <= nz; ++c) {
-        const int kz = (nz + c - 1) / c, chunks = (nz + kz - 1) / kz;
-        const long nb = (long)t.tx * t.ty * chunks;
-        const long steps = (nb + 255) / 256 * (kz + 2);  // two planes before the first step
-        if (best < 0 || steps < best) best = steps, t.kz = kz, t.nblocks = nb;
+// Tiles of `rows` rows and as many z-chunks as make the fewest steps with 16 waves a
+// CU: one, two, ... rounds of workgroups, (planes of a chunk and two before the first
+// step) each.
+Tiles tiles_of_rows(int nx, int ny, int nz, int rows, bool curl) {
+    Tiles best{};
+    const int halo = curl && ny > rows ? 1 : 0, own = rows - 2 * halo;
+    const int tx = (nx + kDiagX - 1) / kDiagX, ty = (ny + own - 1) / own;
+    const long tiles = (long)tx * ty, flight = 256 * 16 / rows;
+    for (long r = (tiles + flight - 1) / flight, c = 0; c < 32; ++r, ++c) {
+        const int most = (int)std::min((long)nz, r * flight / tiles), kz = (nz + most - 1) / most;
+        const long nb = tiles * ((nz + kz - 1) / kz);
+        const long steps = (nb + flight - 1) / flight * (kz + 2);
+        if (c == 0 || steps < best.steps) best = Tiles{tx, ty, kz, rows, halo, nb, steps};
+        if (kz == 1) break;
     }
-    return t;
+    return best;
+}
+// 8 rows, 6 of them stored, with two workgroups a CU; 16 where that saves over a sixth of
+// the steps (it waits longer at its barriers and ends a launch in larger pieces); 4
+// where they hold every row. With 16 always, us: 32^3 9.8 for 8.1, 512x512x16 57.9
+// for 49.5, 250x190x130 66.5 for 62.3; with 8 always: 256^3 226 for 215, 1568x84x220 375
+// for 335, 1000x14x600 88 for 76. 1024x1x1024 in 4, 8, 16: 26, 41, 72.
+// Without the curl (a dimension below 3) nothing is shared between rows: 4.
+Tiles tiles_of(int nx, int ny, int nz, bool curl) {
+    if (ny <= 4 || !curl) return tiles_of_rows(nx, ny, nz, 4, curl);
+    const Tiles t8 = tiles_of_rows(nx, ny, nz, 8, curl), t16 = tiles_of_rows(nx, ny, nz, 16, curl);
+    return 6 * t16.steps < 5 * t8.steps ? t16 : t8;
 }
 
 struct DiagDims {
     int nx, ny, nz;
     Tiles t;
     double ix, iy, iz;
-    int curl;      // all dimensions >= 3
+    bool curl;     // all dimensions >= 3
 };
 
 // padded_idx (src/physics/flow/padded_layout.cuh:30-33)
@@ -189,54 +209,75 @@ struct MinMaxSum {
     }
 };
 
-// min, max and sum over the workgroup (BS threads), valid in thread 0;
-// wv: LDS of 3 * BS / 64 doubles
-template <int BS>
-__device__ inline void block_mms(MinMaxSum& a, double* wv) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        a.lo = fmin(a.lo, __shfl_xor(a.lo, off, 64));
-        a.hi = fmax(a.hi, __shfl_xor(a.hi, off, 64));
-        a.sum += __shfl_xor(a.sum, off, 64);
-    }
-    constexpr int W = BS / 64;
+// one of min (0), max (1), sum (2)
+__device__ __forceinline__ double mms_op(int kind, double a, double b) {
+    return kind == 0 ? fmin(a, b) : kind == 1 ? fmax(a, b) : a + b;
+}
+// the value of the lane N places on in the row of 16 (rotated), by DPP
+template <int N>
+__device__ __forceinline__ double row_ror(double v) {
+    const int2 u = __builtin_bit_cast(int2, v);
+    return __builtin_bit_cast(
+        double, int2{__builtin_amdgcn_update_dpp(0, u.x, 0x120 + N, 0xf, 0xf, false),
+                     __builtin_amdgcn_update_dpp(0, u.y, 0x120 + N, 0xf, 0xf, false)});
+}
+__device__ __forceinline__ double row_mms(int kind, double v) {
+    v = mms_op(kind, v, row_ror<8>(v));
+    v = mms_op(kind, v, row_ror<4>(v));
+    v = mms_op(kind, v, row_ror<2>(v));
+    return mms_op(kind, v, row_ror<1>(v));
+}
+// min, max and sum of F fields over the workgroup of BS threads: out(q, v) for q = 3
+// field + (0 min, 1 max, 2 sum), each from one thread. Rows of 16 lanes reduce by
+// DPP, their values meet in LDS and the waves share the q's. (As wave-wide shuffles
+// and a serial end, three fields of 1024 threads took about 6 us a workgroup, LDS
+// bandwidth, as long as a thin tile's march.)
+template <int BS, int F, typename Out>
+__device__ __forceinline__ void block_mms(const MinMaxSum (&a)[F], Out&& out) {
+    constexpr int E = BS / 16, W = BS / 64;
+    static_assert(E <= 64, "a lane per row");
+    __shared__ double wv[3 * F][E];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    __syncthreads();  // wv may still be read by a previous call
-    if (lane == 0) {
-        wv[w] = a.lo;
-        wv[W + w] = a.hi;
-        wv[2 * W + w] = a.sum;
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        const double v[3] = {row_mms(0, a[f].lo), row_mms(1, a[f].hi), row_mms(2, a[f].sum)};
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+            if (!(lane & 15)) wv[3 * f + q][threadIdx.x >> 4] = v[q];
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int q = 1; q < W; ++q) {
-            a.lo = fmin(a.lo, wv[q]);
-            a.hi = fmax(a.hi, wv[W + q]);
-        }
-        double s = wv[2 * W];
-        for (int q = 1; q < W; ++q) s += wv[2 * W + q];
-        a.sum = s;
+    for (int q = w; q < 3 * F; q += W) {
+        const int kind = q % 3;
+        double v = kind == 0 ? __builtin_huge_val() : kind == 1 ? -__builtin_huge_val() : 0.0;
+        if (lane < E) v = wv[q][lane];
+        v = row_mms(kind, v);
+        v = mms_op(kind, v, __shfl_xor(v, 16, 64));
+        v = mms_op(kind, v, __shfl_xor(v, 32, 64));
+        if (lane == 0) out(q, v);
     }
 }
 
-__global__ void __launch_bounds__(kDiagBlock)
+template <int ROWS, bool CURL>
+__global__ void __launch_bounds__(kDiagX* ROWS, 4)
     diag_kernel(DiagDims d, const double* __restrict__ U, const double* __restrict__ V,
                 const double* __restrict__ W, double* __restrict__ dv, double* __restrict__ om,
                 double* __restrict__ he, double* __restrict__ partials) {
     constexpr int kRow = kDiagX + 2;
-    __shared__ double mu[2][kDiagRows][kRow], mv[2][kDiagRows][kRow], mw[2][kDiagRows][kRow];
+    constexpr int S = CURL ? ROWS : 1;
+    __shared__ double mu[2][S][kRow], mv[2][S][kRow], mw[2][S][kRow];
     const long blk = xcd_block(d.t.nblocks);
     if (blk < 0) return;  // padding block: uniform exit before the barriers
     const long tiles = (long)d.t.tx * d.t.ty;
     const int tile = (int)(blk % tiles), chunk = (int)(blk / tiles);
     const int lane = (int)(threadIdx.x & 63), row = (int)(threadIdx.x >> 6);
-    const int i = tile % d.t.tx * kDiagX + lane, j = tile / d.t.tx * kDiagY - 1 + row;
+    const int i = tile % d.t.tx * kDiagX + lane, j = tile / d.t.tx * (ROWS - 2 * d.t.halo) - d.t.halo + row;
     const int k0 = chunk * d.t.kz, k1 = min(k0 + d.t.kz, d.nz);
-    const bool active = i < d.nx && j >= 0 && j < d.ny && row > 0 && row < kDiagRows - 1;
+    const bool active = i < d.nx && j >= 0 && j < d.ny && row >= d.t.halo &&
+                        row < ROWS - d.t.halo;
     // every load stays inside the padded arrays: columns clamped to the grid, planes
-    // to [0, nz] (a clamped column's means are not used)
+    // to [0, nz) (a clamped column's means are not used)
     const int ic = min(i, d.nx - 1), jc = min(max(j, 0), d.ny - 1);
-    const bool colin = d.curl && i >= 1 && i <= d.nx - 2 && j >= 1 && j <= d.ny - 2;
+    const bool colin = CURL && i >= 1 && i <= d.nx - 2 && j >= 1 && j <= d.ny - 2;
     const double hx = 0.5 * d.ix, hy = 0.5 * d.iy, hz = 0.5 * d.iz;
     // the columns beyond the tile: the left one for lanes 0..31, the right one for the
     // others, every lane loading so that all loads are in flight together
@@ -247,41 +288,47 @@ __global__ void __launch_bounds__(kDiagBlock)
     const long o = pad_idx(d, ic, jc, 0), oe = pad_idx(d, ie, jc, 0);
     const int yp = d.nx + 1;
 
+    // the planes that are needed (others repeat the nearest one, unused): those either
+    // side of the chunk for the curl's z differences only
+    const int klo = CURL ? max(k0 - 1, 0) : k0, khi = CURL ? min(k1, d.nz - 1) : k1 - 1;
+
     struct Plane {  // plane k as loaded; w: of plane k + 1
         double ua, ub, va, vb, w, ea, eb, ew;
     };
     auto load = [&](int k) {
-        const long q = sp * min(max(k, 0), d.nz), qw = sp * min(max(k + 1, 0), d.nz);
-        return Plane{U[q + o], U[q + o + 1], V[q + o],       V[q + o + yp],
-                     W[qw + o], V[q + oe],    V[q + oe + yp], W[qw + oe]};
+        k = min(max(k, klo), khi);
+        const long q = sp * k, qw = sp * (k + 1);
+        Plane p{U[q + o], U[q + o + 1], V[q + o], V[q + o + yp], W[qw + o]};
+        if (CURL) p.ea = V[q + oe], p.eb = V[q + oe + yp], p.ew = W[qw + oe];
+        return p;
     };
     double w0 = W[sp * k0 + o], ew0 = W[sp * k0 + oe];
     Plane below = load(k0 - 1), cur = load(k0), nxt = load(k0 + 1);
     double u0 = 0.5 * (below.ua + below.ub), v0 = 0.5 * (below.va + below.vb);
 
-    MinMaxSum sd, so, sh;
-    sd.init();
-    so.init();
-    sh.init();
+    MinMaxSum a[3];
+    for (MinMaxSum& f : a) f.init();
     for (int k = k0; k < k1; ++k) {
-        const Plane ahead = load(k + 2);  // (the chunk's last ones unused)
+        const Plane ahead = load(k + 2);
         const int buf = k & 1;
         const double uc = 0.5 * (cur.ua + cur.ub), vc = 0.5 * (cur.va + cur.vb),
                      wc = 0.5 * (w0 + cur.w);
         const double u2 = 0.5 * (nxt.ua + nxt.ub), v2 = 0.5 * (nxt.va + nxt.vb);
-        mu[buf][row][lane + 1] = uc;
-        mv[buf][row][lane + 1] = vc;
-        mw[buf][row][lane + 1] = wc;
-        if (edge) {
-            mv[buf][row][eslot] = 0.5 * (cur.ea + cur.eb);
-            mw[buf][row][eslot] = 0.5 * (ew0 + cur.ew);
+        if (CURL) {
+            mu[buf][row][lane + 1] = uc;
+            mv[buf][row][lane + 1] = vc;
+            mw[buf][row][lane + 1] = wc;
+            if (edge) {
+                mv[buf][row][eslot] = 0.5 * (cur.ea + cur.eb);
+                mw[buf][row][eslot] = 0.5 * (ew0 + cur.ew);
+            }
+            lds_barrier();
         }
-        lds_barrier();
         if (active) {
             const double divv = (cur.ub - cur.ua) * d.ix + (cur.vb - cur.va) * d.iy +
                                 (cur.w - w0) * d.iz;
             double omv = 0.0, hev = 0.0;
-            if (colin && k >= 1 && k <= d.nz - 2) {
+            if (CURL && colin && k >= 1 && k <= d.nz - 2) {
                 const double wx = (mw[buf][row + 1][lane + 1] - mw[buf][row - 1][lane + 1]) * hy -
                                   (v2 - v0) * hz;
                 const double wy = (u2 - u0) * hz -
@@ -296,27 +343,16 @@ __global__ void __launch_bounds__(kDiagBlock)
             __builtin_nontemporal_store(omv, om + c);
             __builtin_nontemporal_store(hev, he + c);
             if (partials) {
-                sd.add(divv);
-                so.add(omv);
-                sh.add(hev);
+                a[0].add(divv);
+                a[1].add(omv);
+                a[2].add(hev);
             }
         }
         u0 = uc, v0 = vc, w0 = cur.w, ew0 = cur.ew;
         cur = nxt, nxt = ahead;
     }
     if (!partials) return;  // uniform across the grid
-    __shared__ double wv[3 * kDiagBlock / 64];
-    block_mms<kDiagBlock>(sd, wv);
-    block_mms<kDiagBlock>(so, wv);
-    block_mms<kDiagBlock>(sh, wv);
-    if (threadIdx.x == 0) {
-        const MinMaxSum* f[3] = {&sd, &so, &sh};
-        for (int q = 0; q < 3; ++q) {
-            partials[(3 * q + 0) * d.t.nblocks + blk] = f[q]->lo;
-            partials[(3 * q + 1) * d.t.nblocks + blk] = f[q]->hi;
-            partials[(3 * q + 2) * d.t.nblocks + blk] = f[q]->sum;
-        }
-    }
+    block_mms<kDiagX * ROWS>(a, [&](int q, double v) { partials[q * d.t.nblocks + blk] = v; });
 }
 
 // compute_field_stats first stage (stochastic.cu:369-414): min, max and sum of
@@ -329,18 +365,12 @@ __global__ void __launch_bounds__(kBlock)
     double v[kPer];
 #pragma unroll
     for (int u = 0; u < kPer; ++u) v[u] = x[min(base + (long)u * kBlock, n - 1)];
-    MinMaxSum a;
-    a.init();
+    MinMaxSum a[1];
+    a[0].init();
 #pragma unroll
     for (int u = 0; u < kPer; ++u)
-        if (base + (long)u * kBlock < n) a.add(v[u]);
-    __shared__ double wv[3 * kBlock / 64];
-    block_mms<kBlock>(a, wv);
-    if (threadIdx.x == 0) {
-        partials[blockIdx.x] = a.lo;
-        partials[gridDim.x + blockIdx.x] = a.hi;
-        partials[2 * (long)gridDim.x + blockIdx.x] = a.sum;
-    }
+        if (base + (long)u * kBlock < n) a[0].add(v[u]);
+    block_mms<kBlock>(a, [&](int q, double v) { partials[q * (long)gridDim.x + blockIdx.x] = v; });
 }
 
 // second stage, a workgroup per field with its (min, max, sum) partials of np blocks;
@@ -348,24 +378,18 @@ __global__ void __launch_bounds__(kBlock)
 __global__ void __launch_bounds__(kBlock)
     stats_final_kernel(const double* __restrict__ partials, long np, double n,
                        double* __restrict__ out) {
-    __shared__ double wv[3 * kBlock / 64];
     const int q = (int)blockIdx.x;
     const double* lo = partials + (3 * q + 0) * np;
     const double* hi = partials + (3 * q + 1) * np;
     const double* sm = partials + (3 * q + 2) * np;
-    MinMaxSum a;
-    a.init();
+    MinMaxSum a[1];
+    a[0].init();
     for (long b = threadIdx.x; b < np; b += kBlock) {
-        a.lo = fmin(a.lo, lo[b]);
-        a.hi = fmax(a.hi, hi[b]);
-        a.sum += sm[b];
+        a[0].lo = fmin(a[0].lo, lo[b]);
+        a[0].hi = fmax(a[0].hi, hi[b]);
+        a[0].sum += sm[b];
     }
-    block_mms<kBlock>(a, wv);
-    if (threadIdx.x == 0) {
-        out[3 * q + 0] = a.lo;
-        out[3 * q + 1] = a.hi;
-        out[3 * q + 2] = a.sum / n;
-    }
+    block_mms<kBlock>(a, [&](int e, double v) { out[3 * q + e] = e == 2 ? v / n : v; });
 }
 
 DiagDims diag_dims(const mf3d_grid& g) {
@@ -373,11 +397,11 @@ DiagDims diag_dims(const mf3d_grid& g) {
     d.nx = g.nx;
     d.ny = g.ny;
     d.nz = g.nz;
-    d.t = tiles_of(g.nx, g.ny, g.nz);
+    d.curl = g.nx >= 3 && g.ny >= 3 && g.nz >= 3;
+    d.t = tiles_of(g.nx, g.ny, g.nz, d.curl);
     d.ix = 1.0 / g.dx;
     d.iy = 1.0 / g.dy;
     d.iz = 1.0 / g.dz;
-    d.curl = g.nx >= 3 && g.ny >= 3 && g.nz >= 3;
     return d;
 }
 
@@ -391,8 +415,17 @@ int velocity_diagnostics(hipStream_t s, const mf3d_grid& g, const double* U, con
                          const double* W, double* div, double* omag, double* hel,
                          double* partials, double* stats) {
     const DiagDims d = diag_dims(g);
-    diag_kernel<<<xcd_round((size_t)d.t.nblocks), kDiagBlock, 0, s>>>(d, U, V, W, div, omag, hel,
-                                                                     stats ? partials : nullptr);
+    const unsigned nb = xcd_round((size_t)d.t.nblocks);
+    double* const part = stats ? partials : nullptr;
+    auto launch = [&](auto rows) {
+        constexpr int R = decltype(rows)::value;
+        diag_kernel<R, true><<<nb, kDiagX * R, 0, s>>>(d, U, V, W, div, omag, hel, part);
+    };
+    if (!d.curl)
+        diag_kernel<4, false><<<nb, kDiagX * 4, 0, s>>>(d, U, V, W, div, omag, hel, part);
+    else if (d.t.rows == 4) launch(std::integral_constant<int, 4>{});
+    else if (d.t.rows == 8) launch(std::integral_constant<int, 8>{});
+    else launch(std::integral_constant<int, 16>{});
     MF3D_HIP_TRY(hipGetLastError());
     if (stats) {
         stats_final_kernel<<<3, kBlock, 0, s>>>(partials, d.t.nblocks, (double)cells(g), stats);
