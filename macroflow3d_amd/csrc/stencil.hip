@@ -1,13 +1,15 @@
 // Cell-centred 7-point variable-K stencil kernels (FP64), gfx950.
 //
-// One thread per cell (or per own-colour cell for the red-black smoother),
+// Smoother, residual and operator straight from K march cell pairs up in z,
 // all boundary types handled in the same launch: the reference spends 27
 // launches per colour on interior/face/edge/vertex kernels
 // (src/multigrid/smoothers/gsrb_3d.cu:392-575); here a colour is one launch.
-// These kernels serve every level and every boundary mix of the
-// reference-semantics entry points (mf3d_gsrb_smooth_3d, ...).
+// With the transfers, coarsening, right-hand side and guess (a thread per cell)
+// they serve every size and boundary mix of the reference-semantics entry
+// points (mf3d_gsrb_smooth_3d, ...). Then the coarsest direct solve.
 
 #include <algorithm>
+#include <type_traits>
 
 #include "hface.hpp"
 #include "kernels.hpp"
@@ -56,8 +58,11 @@ __device__ __forceinline__ double kface(const Side& s, double ia, double ib, dou
 struct ColumnGeo {
     int nx, ny, nz;
     int np;     // pairs per row: ceil(nx / 2)
-    int tiles;  // workgroups per plane
-    int kz;     // planes per workgroup
+    int tiles;  // workgroups per plane (FLAT: unused)
+    int kz;     // planes per thread
+    int chunks;
+    int slabs;  // a row holds a multiple of 8 workgroups: in launch order each XCD then
+                // owns slabs along x, with all their y and z neighbours
     long nblocks;
 };
 
@@ -87,18 +92,24 @@ __device__ __forceinline__ Pair ldpair(const double* __restrict__ p, long o, int
 // times x_C at cell 0). COL_APPLY: out = A x (varcoeff_laplacian.cu:38-239; the
 // pin's diagonal counts in-domain neighbours only, :110-119, :232-234).
 enum { COL_GSRB = 0, COL_RES = 1, COL_APPLY = 2 };
-template <int KIND, bool VEC>
+// FLAT: a workgroup takes columns of several chunks, for planes that would leave most
+// of its threads without one.
+template <int KIND, bool VEC, bool FLAT>
 __global__ void __launch_bounds__(kBlock)
     column_kernel(ColumnGeo G, double dx2, double inv_dx2, BcTypes bc, int pin, const double* x,
                   const double* b, const double* __restrict__ K, double* out, int colour) {
-    const long blk = xcd_block(G.nblocks);
-    if (blk < 0) return;
-    const int chunk = (int)(blk / G.tiles);
-    const long tp = (blk - (long)chunk * G.tiles) * kBlock + threadIdx.x;
-    if (tp >= (long)G.np * G.ny) return;
+    const long blk = G.slabs ? blockIdx.x : xcd_block(G.nblocks);
+    if (blk < 0 || blk >= G.nblocks) return;
     const int nx = G.nx, ny = G.ny, nz = G.nz;
-    const int j = (int)(tp / G.np);
-    const int i = 2 * (int)(tp - (long)j * G.np);
+    // (a grid has at most 4e9 cells: 32-bit divisions)
+    const unsigned plane = (unsigned)G.np * (unsigned)G.ny;
+    const unsigned t = (unsigned)blk * kBlock + threadIdx.x;
+    const int chunk = (int)(FLAT ? t / plane : (unsigned)blk / (unsigned)G.tiles);
+    const unsigned tp = t - (FLAT ? (unsigned)chunk * plane
+                                  : (unsigned)chunk * (unsigned)G.tiles * kBlock);
+    if (FLAT ? chunk >= G.chunks : tp >= plane) return;
+    const int j = (int)(tp / (unsigned)G.np);
+    const int i = 2 * (int)(tp - (unsigned)j * (unsigned)G.np);
     const bool two = i + 1 < nx;  // the pair's second cell exists
     const int d1 = two ? 1 : 0;
     const long sz = (long)nx * ny;
@@ -112,9 +123,13 @@ __global__ void __launch_bounds__(kBlock)
     const Side D0 = side(k0 > 0, -sz, bc.t[4], (long)(nz - 1) * sz);
     Pair Kc = ldpair<VEC>(K, o, d1), xc = ldpair<VEC>(x, o, d1);
     Pair Kd = ldpair<VEC>(K, o + D0.off, d1), xd = ldpair<VEC>(x, o + D0.off, d1);
-    Pair ic, id;
+    Pair ic{}, id{};
+    // the first plane's reciprocals, once its loads are on their way
+    auto first = [&](int k) {
+        if (k != k0) return;
 #pragma unroll
-    for (int e = 0; e < 2; ++e) ic.v[e] = recip(Kc.v[e]), id.v[e] = recip(Kd.v[e]);
+        for (int e = 0; e < 2; ++e) ic.v[e] = recip(Kc.v[e]), id.v[e] = recip(Kd.v[e]);
+    };
     for (int k = k0; k < k1; ++k, o += sz) {
         const Side U = side(k < nz - 1, sz, bc.t[5], -(long)(nz - 1) * sz);
         const Side D = k == k0 ? D0 : In;
@@ -136,6 +151,7 @@ __global__ void __launch_bounds__(kBlock)
             const long op = oe + Xp.off;
             const double Kp1 = two ? 0.0 : K[op], xp1 = two ? 0.0 : x[op];
             const double bv = b[oe];
+            first(k);
 #pragma unroll
             for (int q = 0; q < 2; ++q) iu.v[q] = recip(Ku.v[q]);
             const double io = recip(Ko);
@@ -164,6 +180,7 @@ __global__ void __launch_bounds__(kBlock)
             const double Ke = K[o + d1 + E.off], xe = x[o + d1 + E.off];
             Pair bv{};
             if (KIND == COL_RES) bv = ldpair<VEC>(b, o, d1);
+            first(k);
 #pragma unroll
             for (int q = 0; q < 2; ++q) iu.v[q] = recip(Ku.v[q]);
             const double iw = recip(Kw), ie = recip(Ke);
@@ -850,31 +867,48 @@ __global__ void __launch_bounds__(kFactorThreads)
 namespace kern {
 
 namespace {
-// Planes per workgroup: long columns reuse the marched planes and short ones
+// Planes per thread: long columns reuse the marched planes and short ones
 // fill the chip; up to 16 planes while 2048 workgroups (8 waves a SIMD pair)
-// remain.
+// remain. GSRB iterations, us: 2x2x65536 8.0 flat (142 with a chunk a workgroup),
+// 4x4x4096 6.5 (16.8); slabs for 8192x8x8 10.8 (14.6), 4096x256x16 244 (271), but
+// 4096x4x512 119 (107): few rows leave an XCD narrow pieces of many chunks.
+constexpr int kFlatColumns = 1024;
+bool column_flat(const mf3d_grid& g) { return (long)((g.nx + 1) / 2) * g.ny < kFlatColumns; }
 ColumnGeo column_geo(const mf3d_grid& g) {
     ColumnGeo G;
     G.nx = g.nx, G.ny = g.ny, G.nz = g.nz;
     G.np = (g.nx + 1) / 2;
-    G.tiles = (int)(((long)G.np * g.ny + kBlock - 1) / kBlock);
-    G.kz = (int)std::max(1L, std::min(16L, (long)G.tiles * g.nz / 2048));
-    G.nblocks = (long)G.tiles * ((g.nz + G.kz - 1) / G.kz);
+    const long plane = (long)G.np * g.ny;
+    G.tiles = (int)((plane + kBlock - 1) / kBlock);
+    const long fill = column_flat(g) ? plane * g.nz / kBlock : (long)G.tiles * g.nz;
+    G.kz = (int)std::max(1L, std::min(16L, fill / 2048));
+    G.chunks = (g.nz + G.kz - 1) / G.kz;
+    G.slabs = G.np % (8 * kBlock) == 0 && (g.ny >= 8 || G.kz == 1);
+    G.nblocks = column_flat(g) ? (plane * G.chunks + kBlock - 1) / kBlock : (long)G.tiles * G.chunks;
     return G;
 }
 template <int KIND>
-int launch_column(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, bool pin, const double* x,
+int launch_column(hipStream_t s, mf3d_grid g, BcTypes bc, bool pin, const double* x,
                   const double* b, const double* K, double* out, int colour) {
+    // a one-cell x axis moves to z (the same cells in the same order, one spacing for
+    // all axes), so that pairs are pairs: 1x1024x1024 operator 13.0 us otherwise
+    for (int q = 0; q < 2 && g.nx == 1; ++q) {
+        std::rotate(bc.t, bc.t + 2, bc.t + 6);
+        g.nx = g.ny, g.ny = g.nz, g.nz = 1;
+    }
     const ColumnGeo G = column_geo(g);
     const double dx2 = g.dx * g.dx;
     auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
-    const unsigned nb = xcd_round((size_t)G.nblocks);
-    if (!(g.nx & 1) && al(x) && al(K) && al(out) && (KIND != COL_RES || al(b)))
-        column_kernel<KIND, true><<<nb, kBlock, 0, s>>>(G, dx2, 1.0 / dx2, bc, pin, x, b, K, out,
-                                                        colour);
-    else
-        column_kernel<KIND, false><<<nb, kBlock, 0, s>>>(G, dx2, 1.0 / dx2, bc, pin, x, b, K, out,
-                                                         colour);
+    const bool vec = !(g.nx & 1) && al(x) && al(K) && al(out) && (KIND != COL_RES || al(b));
+    auto launch = [&](auto v, auto f) {
+        column_kernel<KIND, decltype(v)::value, decltype(f)::value>
+            <<<xcd_round((size_t)G.nblocks), kBlock, 0, s>>>(G, dx2, 1.0 / dx2, bc, pin, x, b, K,
+                                                             out, colour);
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    if (column_flat(g)) vec ? launch(yes, yes) : launch(no, yes);
+    else vec ? launch(yes, no) : launch(no, no);
     MF3D_HIP_TRY(hipGetLastError());
     return MF3D_OK;
 }

@@ -122,3 +122,33 @@ def test_cells_of_zero_conductivity_close_their_faces(ctx):
     assert rel_err(host(r), ro) < TOL
     nm.VarCoeffLaplacian(g, dev(K, ctx), bc).apply(ctx, dev(x, ctx), r)
     assert rel_err(host(r), yo) < TOL
+
+
+# planes of few columns (several chunks a workgroup), either side of the 1024 columns from
+# which a workgroup stays in one chunk; 4x4x140000: two planes a thread
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("mix", ["darcy_x", "periodic_yz", "all_neumann"])
+@pytest.mark.parametrize("shape", [(1, 1, 5000), (2, 2, 3000), (3, 4, 700), (1, 64, 64),
+                                   (511, 4, 6), (510, 4, 6), (511, 3, 10), (4, 4, 140000)])
+def test_narrow_columns_match_oracle(ctx, shape, mix, off):
+    test_column_kernels_match_oracle(ctx, shape, mix, off)
+
+
+def test_smoother_meets_cells_of_zero_conductivity(ctx):
+    """Such a cell has no diagonal: its value and, through 0 times that, its neighbours'
+    are what IEEE division and multiplication make them; all others are untouched."""
+    g, og = grid_pair(10, 6, 4)
+    bc, obc = bc_pair("darcy_x")
+    n = g.num_cells()
+    rng = np.random.default_rng(13)
+    K, x, b = random_K(n, 14), rng.standard_normal(n), rng.standard_normal(n)
+    K[[0, 33, 34, 44, n - 1]] = 0.0
+    b[33] = 0.0
+    with np.errstate(all="ignore"):
+        ref = O.gsrb_smooth_3d(og, obc, False, x, b, K, 1)
+    xd = dev(x, ctx)
+    mg.gsrb_smooth_3d(ctx, g, xd, dev(b, ctx), dev(K, ctx), 1, bc)
+    got, ok = host(xd), np.isfinite(ref)
+    assert 0 < (~ok).sum() < n // 4
+    assert np.array_equal(got[~ok], ref[~ok], equal_nan=True)
+    assert rel_err(got[ok], ref[ok]) < TOL
