@@ -230,7 +230,7 @@ struct Planar {
     long plane;    // one channel
     int gpr;       // 8-voxel groups per row
     long groups;   // over all rows of the grid
-    int ny;
+    int nx, ny;
 };
 Planar planar_of(const mf3d_grid& g) {
     Planar P;
@@ -240,7 +240,7 @@ Planar planar_of(const mf3d_grid& g) {
     P.plane = P.slab * (g.nz + 2) + 2 * kPlanarLead;
     P.gpr = n8;
     P.groups = (long)n8 * g.ny * g.nz;
-    P.ny = g.ny;
+    P.nx = g.nx, P.ny = g.ny;
     return P;
 }
 
@@ -331,8 +331,19 @@ __device__ __forceinline__ void wgrad_body(const WLayer& L, int tap, int slice) 
     // The tap's shift along x is made in registers from an aligned load and the
     // 4 bytes next to it: 16-byte loads at odd element offsets took 68 us
     // for the launch instead of 51.
+    // Products that are not part of the sum are 0 x 0 (the other factor may be infinite):
+    // X is zeroed past the end, and where dx = -1 would bring a row's last value
+    // beside the zero after its dY (the row's last group, element nx & 7, if it has one).
+    const int tail = dx < 0 ? (L.P.nx & 7) : 0;
+    uint4 keep{~0u, ~0u, ~0u, ~0u};
+    if (tail) {  // uniform
+        const unsigned half = tail & 1 ? 0x0000ffffu : 0xffff0000u;
+        const int w = tail >> 1;
+        keep = uint4{w == 0 ? half : ~0u, w == 1 ? half : ~0u, w == 2 ? half : ~0u,
+                     w == 3 ? half : ~0u};
+    }
     auto load = [&](bool mine, bf16x8 (&a)[CT], bf16x8 (&b)[IT]) {
-        const bool ok = mine && q < groups;
+        const bool ok = mine && q < groups, last = x8 == L.P.gpr - 1;
         const long oo = ok ? o : L.P.slab + L.P.row;
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
@@ -351,8 +362,9 @@ __device__ __forceinline__ void wgrad_body(const WLayer& L, int tap, int slice) 
                 const unsigned n = *reinterpret_cast<const unsigned*>(p - 2);
                 d = uint4{__builtin_amdgcn_alignbit(d.x, n, 16), __builtin_amdgcn_alignbit(d.y, d.x, 16),
                           __builtin_amdgcn_alignbit(d.z, d.y, 16), __builtin_amdgcn_alignbit(d.w, d.z, 16)};
+                if (tail && last) d.x &= keep.x, d.y &= keep.y, d.z &= keep.z, d.w &= keep.w;
             }
-            b[i] = __builtin_bit_cast(bf16x8, d);
+            b[i] = ok ? __builtin_bit_cast(bf16x8, d) : zero8;
         }
         q += 4, x8 += 4, o += 32;
         while (x8 >= L.P.gpr) {  // rows end with 8 zeros; the next z skips the border rows

@@ -54,3 +54,33 @@ def test_convolution_gradients_over_launch_shapes(ctx, shape, cin, cout):
               dY.data_ptr(), gw.data_ptr(), gb.data_ptr())
     assert _rel(host(gw), rw) < 1e-4
     assert _rel(host(gb), rb) < 1e-4
+
+
+@pytest.mark.parametrize("shape", [(9, 3, 2), (14, 4, 3), (8, 2, 2), (5, 1, 1), (24, 20, 3)])
+def test_weight_gradient_of_infinite_inputs(ctx, shape):
+    """An infinite input reaches the taps whose sums hold it, as an infinity, and no
+    other: products outside the sums (rows' ends, past the last voxel) are 0 x 0."""
+    nx, ny, nz = shape
+    rng = np.random.default_rng(nx)
+    x = CO.bf16(rng.standard_normal((nz, ny, nx, 16)))
+    dy = CO.bf16(0.5 + rng.random((nz, ny, nx, 16)))  # positive: inf, never inf - inf
+    x[0, 0, 0, 1] = x[-1, -1, -1, 2] = x[0, 0, -1, 3] = np.inf
+    ref = np.zeros((16, 27, 16))
+    for tap in range(27):
+        d = (tap // 9 - 1, tap // 3 % 3 - 1, tap % 3 - 1)  # z, y, x
+        src = tuple(slice(max(0, s), n + min(0, s)) for s, n in zip(d, (nz, ny, nx)))
+        dst = tuple(slice(max(0, -s), n + min(0, -s)) for s, n in zip(d, (nz, ny, nx)))
+        a, b = dy[dst].reshape(-1, 16), x[src].reshape(-1, 16)
+        for c in range(16):
+            ref[:, tap, c] = (a * b[:, c:c + 1]).sum(0)
+    dev = lambda t: torch.as_tensor(np.ascontiguousarray(t), dtype=torch.float32).to(torch.bfloat16).to(ctx.device)  # noqa: E731
+    X, dY = dev(x), dev(dy)
+    g = Grid3D(nx, ny, nz).c()
+    gw = torch.empty((16, 27, 16), dtype=torch.float32, device=ctx.device)
+    gb = torch.empty(16, dtype=torch.float32, device=ctx.device)
+    _lib.call("mf3d_conv3d_backward_weights", ctx.handle, C.byref(g), 16, 16, X.data_ptr(),
+              dY.data_ptr(), gw.data_ptr(), gb.data_ptr())
+    got, fin = gw.cpu().numpy().astype(np.float64), np.isfinite(ref)
+    assert (~fin).any() and np.array_equal(np.isposinf(got), np.isposinf(ref))
+    assert not np.isnan(got).any()
+    assert np.abs(got[fin] - ref[fin]).max() < 1e-4 * np.abs(ref[fin]).max()
