@@ -97,8 +97,7 @@ bool fused32_ok(const mf3d_grid& g, CoefType t);
 bool fused32_pays(const mf3d_grid& g);  // faster than the half-sweeps there
 // the level's face records, made from its half-sweep faces
 size_t fused32_face_bytes(const mf3d_grid& g);
-int fused32_pack(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, const FaceSet& F,
-                 void* faces);
+int fused32_pack(hipStream_t s, const mf3d_grid& g, const FaceSet& F, void* faces);
 // two GSRB iterations from zero: xb = the black values, bcoarse = restriction of
 // the residual's red cells. b (and bcoarse with pairs): (red, black) per place;
 // bcoarse without pairs: colour-split

@@ -65,7 +65,7 @@ enum { START_ZERO = 0, START_PROLONG = 1 };
 enum { END_NONE = 0, END_RESTRICT = 1 };
 
 struct FGeo {
-    int nx, ny, nz, h;
+    int h, ny, nz;
     long half;
     int tx, ty;      // tiles
     int kz, chunks;  // planes per chunk (even)
@@ -397,7 +397,7 @@ __global__ void __launch_bounds__(kThreads)
 // face records of a level from its half-sweep arrays
 template <typename TC>
 __global__ void __launch_bounds__(256)
-    pack_faces_kernel(Dims d, BcTypes bc, SFaces<TC> F, Rec* __restrict__ out) {
+    pack_faces_kernel(Dims d, SFaces<TC> F, Rec* __restrict__ out) {
     const int h = d.nx >> 1;
     const long total = (long)(h + 1) * (d.ny + 1) * (d.nz + 1);
     const long t = (long)blockIdx.x * 256 + threadIdx.x;
@@ -486,7 +486,7 @@ long steps_of(int tiles, int chunks, int kz) {
 
 FGeo fgeo_of(const mf3d_grid& g) {
     FGeo G;
-    G.nx = g.nx, G.ny = g.ny, G.nz = g.nz;
+    G.ny = g.ny, G.nz = g.nz;
     G.bcp = 0;
     G.h = g.nx / 2;
     G.half = (long)G.h * g.ny * g.nz;
@@ -552,8 +552,7 @@ size_t fused32_face_bytes(const mf3d_grid& g) {
     return sizeof(Rec) * (size_t)(g.nx / 2 + 1) * (g.ny + 1) * (g.nz + 1);
 }
 
-int fused32_pack(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, const FaceSet& F,
-                 void* faces) {
+int fused32_pack(hipStream_t s, const mf3d_grid& g, const FaceSet& F, void* faces) {
     MF3D_TRY(check(g, F.type));
     if (!F.split) return fail(MF3D_ERR_UNSUPPORTED, "face records come from colour-split faces");
     const unsigned nb = (unsigned)((fused32_face_bytes(g) / sizeof(Rec) + 255) / 256);
@@ -562,12 +561,12 @@ int fused32_pack(hipStream_t s, const mf3d_grid& g, const BcTypes& bc, const Fac
     if (F.type == COEF_BF16) {
         typedef __hip_bfloat16 T;
         pack_faces_kernel<T><<<nb, 256, 0, s>>>(
-            d, bc, SFaces<T>{(const T*)F.fx, (const T*)F.fy, (const T*)F.fz, (const T*)F.ux,
+            d, SFaces<T>{(const T*)F.fx, (const T*)F.fy, (const T*)F.fz, (const T*)F.ux,
                              (const T*)F.uy, (const T*)F.uz}, o);
     } else {
         typedef __half T;
         pack_faces_kernel<T><<<nb, 256, 0, s>>>(
-            d, bc, SFaces<T>{(const T*)F.fx, (const T*)F.fy, (const T*)F.fz, (const T*)F.ux,
+            d, SFaces<T>{(const T*)F.fx, (const T*)F.fy, (const T*)F.fz, (const T*)F.ux,
                              (const T*)F.uy, (const T*)F.uz}, o);
     }
     MF3D_HIP_TRY(hipGetLastError());

@@ -7,8 +7,8 @@
 //
 // Bound: one by one the half-sweeps stream 20 bytes a cell each (the other
 // colour's x, b, h of both colours, the own x) at 4.9 TB/s, four of them and the
-// residual 100 bytes. Fused, x, b and h cross HBM once: 24 bytes a cell for
-// pre-smoothing + restriction, 32 for prolongation + post-smoothing. What bounds
+// residual 100 bytes. Fused, x, b and h cross HBM once: 21 bytes a cell for
+// pre-smoothing + restriction, 29 for prolongation + post-smoothing. What bounds
 // the pass instead is vector instructions: about 75 FP64 ones a cell, half of them
 // for the faces (1 / (h_a + h_b)) and the diagonals' reciprocals.
 //
@@ -38,7 +38,7 @@
 // (438 as half-sweeps, with the r update), prolongation + post-smoothing + (r, z) 237
 // (327). 45 % of the vector issue slots are used; the rest waits on LDS and the
 // chains of the quotients with two waves a SIMD. (One iteration a pass, 1024 threads,
-// would stream 32 bytes a cell for the two half-sweeps' 40.)
+// would stream 28 bytes a cell for the two half-sweeps' 40.)
 
 #include <algorithm>
 #include <type_traits>
@@ -215,7 +215,7 @@ struct Fused64 {
             hr[U] = !inside ? ghost : ki ? nxt.hr : zghost;
             hb[U] = !inside ? ghost : ki ? nxt.hb : zghost;
             double he = ein ? nxt.he : eghost;
-                double br1 = nxt.br, bb1 = nxt.bb;
+            double br1 = nxt.br, bb1 = nxt.bb;
             if (PARK) pk = pk == kPark - 1 ? 0 : pk + 1;  // plane k - 1
             else br[sl(1)] = br1, bb[sl(1)] = bb1;
             xr[U] = xb[U] = 0.0;

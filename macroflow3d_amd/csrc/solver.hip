@@ -759,7 +759,7 @@ int mg_setup(mf3d_workspace* ws, hipStream_t s, const mf3d_grid& g, const mf3d_b
         if (!L.fused) continue;
         if (ws->try_bytes((void**)&L.xb, L.n / 2 * sizeof(float)) &&
             ws->try_bytes(&L.rec, kern::fused32_face_bytes(L.g)))
-            MF3D_TRY(kern::fused32_pack(s, L.g, ws->bct, L.flo, L.rec));
+            MF3D_TRY(kern::fused32_pack(s, L.g, L.flo, L.rec));
         else ws->drop_passes(L);
     }
     // window passes on small levels (the batched solve has its own launches, whose

@@ -80,6 +80,20 @@ Geo geo_of(const mf3d_grid& g) {
     return G;
 }
 
+// (sum f x_nb - b bs) / sum f, summed x+, x-, y+, y-, z+, z- (gsrb_3d.cu:53-69)
+__device__ __forceinline__ double gs64(const double (&f)[6], const double (&v)[6], double b,
+                                       double bs, bool pin0) {
+    double result = v[0] * f[0];
+    result += v[1] * f[1];
+    result += v[2] * f[2];
+    result += v[3] * f[3];
+    result += v[4] * f[4];
+    result += v[5] * f[5];
+    double aC = f[0] + f[1] + f[2] + f[3] + f[4] + f[5];
+    if (pin0) aC *= 2.0;
+    return (result - b * bs) / aC;
+}
+
 // Other-colour values at the x neighbours of the thread's two cells, from the
 // other colour's pair a = (places base, base + 1) of row r0 (array O):
 // xp[e] / xm[e] at x+ / x- of cell e; the places outside the pair come from

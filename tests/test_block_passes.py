@@ -59,8 +59,8 @@ def test_fp32_window_passes_equal_half_sweeps(ctx, shape, levels, mix, counts):
 @pytest.mark.parametrize("mix", list(BC_MIXES))
 @pytest.mark.parametrize("shape,levels", SHAPES)
 def test_fp64_window_passes_match_half_sweeps(ctx, shape, levels, mix, counts):
-    """FP64 differs by the order of the x terms and the quotients' last bit: some
-    1e-16 a cell and half-sweep, times the coarsest system's condition (< 1e4)."""
+    """FP64 differs by the order of the x terms: some 1e-16 a cell and half-sweep,
+    times the coarsest system's condition (< 1e4)."""
     z = [_apply(ctx, shape, levels, mix, counts, ph.PrecondPrecision.FP64, fuse).cpu().numpy()
          for fuse in (0, -1)]
     assert np.isfinite(z[1]).all()

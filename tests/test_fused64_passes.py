@@ -23,8 +23,8 @@ SHAPES = [((80, 72, 56), 4), ((136, 104, 24), 4), ((160, 104, 16), 4), ((48, 40,
 @pytest.mark.parametrize("mix", list(BC_MIXES))
 @pytest.mark.parametrize("shape,levels", SHAPES)
 def test_fused64_vcycle_matches_half_sweeps(ctx, shape, levels, mix):
-    """The same sums up to the order of the x terms and the quotients' last bit:
-    some 1e-16 a cell and half-sweep, times the coarsest system's condition (< 1e4)."""
+    """The same sums up to the order of the x terms: some 1e-16 a cell and half-sweep,
+    times the coarsest system's condition (< 1e4)."""
     g = Grid3D(*shape)
     bc, _ = bc_pair(mix)
     n = g.num_cells()
@@ -44,6 +44,14 @@ def test_fused64_vcycle_matches_half_sweeps(ctx, shape, levels, mix):
         ws.close()
     assert np.isfinite(z[1]).all()
     assert rel_l2(z[1], z[0]) < 1e-11
+
+
+@pytest.mark.parametrize("mix", list(BC_MIXES))
+@pytest.mark.parametrize("shape,levels", [((16, 64, 512), 4), ((40, 16, 640), 4), ((96, 16, 352), 4)])
+def test_fused64_vcycle_narrower_than_a_tile(ctx, shape, levels, mix):
+    """Domains of fewer places or rows than a tile: on periodic sides it wraps onto
+    itself."""
+    test_fused64_vcycle_matches_half_sweeps(ctx, shape, levels, mix)
 
 
 @pytest.mark.parametrize("graph", [0, 1])

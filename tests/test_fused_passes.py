@@ -46,12 +46,22 @@ def test_fused_vcycle_equals_half_sweeps(ctx, shape, levels, mix, coef):
     assert torch.equal(z[0], z[1])
 
 
+@pytest.mark.parametrize("mix", list(BC_MIXES))
+@pytest.mark.parametrize("shape,levels", [((96, 16, 128), 3), ((16, 64, 128), 3), ((8, 96, 256), 3),
+                                          ((24, 8, 320), 3)])
+def test_fused_vcycle_narrower_than_a_tile(ctx, shape, levels, mix):
+    """Domains of fewer rows or places than a tile: on periodic sides it wraps onto
+    itself."""
+    test_fused_vcycle_equals_half_sweeps(ctx, shape, levels, mix, ph.CoefFormat.BF16)
+
+
 @pytest.mark.parametrize("graph", [0, 1])
 @pytest.mark.parametrize("fold_r", [0, 1])
 @pytest.mark.parametrize("shape", [(64, 64, 64), (128, 96, 48)])
 def test_fused_solve_matches_half_sweeps(ctx, shape, fold_r, graph):
-    """The solve around them: r update, (r, z) partials grouped by tile instead
-    of by sweep workgroup, so heads equal to rounding and equal iterations."""
+    """The solve around them, with the r update folded into the half-sweeps' first one
+    or before the passes: (r, r) grouped differently, which decides only when to
+    stop (test_batched.py holds the heads to equality)."""
     g = Grid3D(*shape)
     bc, _ = bc_pair("darcy_x")
     K = torch.exp(lognormal_lnK(*shape, 2.0, 5.0, 41, device=ctx.device)[0])
