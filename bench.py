@@ -11,10 +11,12 @@ stay FP64). The plain FP64 MG-PCG is timed on the same field as the
 denominator, and the mixed head/velocity are compared with it.
 
 Also measured here:
-  * roofline of the dominant kernel (the finest level's GSRB colour sweep of
-    the headline V-cycle): algorithmic bytes per launch / average launch time
-    from HIP events on the solve stream; HBM traffic per launch from the
-    rocprofv3 FETCH_SIZE/WRITE_SIZE summaries committed under profiles/;
+  * roofline of the dominant kernel (the headline V-cycle's smoothing of the
+    finest level: its two fused passes, or one colour's half-sweep where a
+    level does not take them): algorithmic bytes per launch / average launch
+    time from HIP events on the solve stream; HBM traffic per launch from the
+    rocprofv3 FETCH_SIZE/WRITE_SIZE summaries committed under profiles/. The
+    half-sweep, which such a level falls back to, is timed beside it;
   * CPU baseline: the CPU FP64 oracle (OpenMP) solving the same 256^3 K to
     1e-10 (set-up + solve, median of 3); the GPU FP64 head and velocity
     checksums against that same-algorithm solve, and both GPU heads against
@@ -133,14 +135,20 @@ def summarize_trace(d: str, tail: int = 0) -> int:
     # the finest-level half-sweeps' last launches at each grid are the timed
     # smoother repetitions (2 per mg_smooth iteration), the launches bench.py's
     # HIP events cover; the averages above also hold the in-solve launches.
-    # Mixed V-cycle: colour_split4_kernel<., 0, false>; FP64: sweep64_kernel<0, ...>
+    # Mixed V-cycle: colour_split4_kernel<., 0, false>; FP64: march64_kernel<0, ...>
     # (the FP64 march kernel launches the same grid on every level it runs
     # on, so its rows above mix levels; its last launches are the finest
-    # level's timed repetitions)
+    # level's timed repetitions). The fused passes likewise: each kind's last
+    # launches, one of each per repetition.
     sweeps = [(k, v) for k, v in acc.items()
               if ("colour_split4_kernel<" in k[0] and ", 0, false>" in k[0]) or
               "march64_kernel<0, false, false>" in k[0]]
     if tail > 0:
+        for (name, grid), (_, _, launches) in acc.items():
+            if "::fused_kernel<" in name or "::fused64_kernel<" in name:
+                last = [d for _, d in sorted(launches)[-tail // 2:]]
+                print(f"{sum(last) / len(last) / 1e3:10.2f} us avg\tcalls={len(last)}\tgrid={grid}"
+                      f"\tlast {len(last)} launches (timed passes)\t{name[:80]}")
         for kind in ("colour_split4_kernel<", "march64_kernel<"):
             own = [kv for kv in sweeps if kind in kv[0][0]]
             # the two largest grids: the finest levels of the 256^3 and 512^3 runs
@@ -229,15 +237,17 @@ def cpu_baseline(args, K_host, gpu):
             parity, ref_sums)
 
 
-def committed_traffic(n: int, coef: str):
-    """HBM bytes per launch of the dominant kernel from the committed PMC summary:
-    the line `traffic_bytes_per_launch n=<n> coef=<coef>: <bytes>`."""
+def committed_traffic(n: int, coef: str, kernel: str):
+    """HBM bytes per launch of a smoothing kernel (fused: the two passes' mean;
+    half_sweep) from the committed PMC summary, its line
+    `traffic_bytes_per_launch n=<n> coef=<coef> kernel=<kernel>: <bytes>`."""
     try:
         with open(TRAFFIC_FILE) as f:
             for line in f:
-                m = re.match(r"\s*traffic_bytes_per_launch n=(\d+) coef=(\w+):\s*([0-9.eE+]+)", line)
-                if m and int(m.group(1)) == n and m.group(2) == coef:
-                    return float(m.group(3))
+                m = re.match(r"\s*traffic_bytes_per_launch n=(\d+) coef=(\w+) kernel=(\w+):"
+                             r"\s*([0-9.eE+]+)", line)
+                if m and (int(m.group(1)), m.group(2), m.group(3)) == (n, coef, kernel):
+                    return float(m.group(4))
     except OSError:
         pass
     return None
@@ -260,10 +270,61 @@ def time_smoother(ctx, ws, reps):
     return e0.elapsed_time(e1) / (2 * reps)
 
 
+def time_passes(ctx, ws, reps):
+    """Average duration (ms) of one of the finest level's two fused passes
+    (mf3d_mg_passes), or None where it is smoothed in half-sweeps."""
+    import torch
+
+    from macroflow3d_amd import _lib
+    from macroflow3d_amd import multigrid as mg
+    try:
+        mg.level_passes(ctx, ws, 0, 1)
+    except _lib.MF3DError as e:
+        if e.status != 7:  # MF3D_ERR_UNSUPPORTED
+            raise
+        return None
+    e0 = torch.cuda.Event(enable_timing=True)
+    e1 = torch.cuda.Event(enable_timing=True)
+    e0.record(ctx.stream)
+    mg.level_passes(ctx, ws, 0, reps)
+    e1.record(ctx.stream)
+    e1.synchronize()
+    return e0.elapsed_time(e1) / (2 * reps)
+
+
+# algorithmic bytes a cell of one launch. Half-sweep: 3 faces (mixed) or h of both
+# colours (FP64), the other colour's x, the own b, the own x out. Fused passes, the mean
+# of the two: pre-smoothing + restriction (faces or h, b, the black x and a coarse b an
+# eighth of the level out), prolongation + post-smoothing (faces or h, b, the black x
+# and the coarse x in, x out).
+HALF_SWEEP_BYTES = {"bf16": 12.0, "fp16": 12.0, "fp32": 18.0, "fp64": 20.0}
+PASS_BYTES = {"bf16": (12.5 + 16.5) / 2, "fp16": (12.5 + 16.5) / 2,
+              "fp64": (8 + 8 + 4 + 1 + 8 + 8 + 4 + 1 + 8) / 2}
+
+
+def kernel_line(name, t_ms, bytes_per_launch):
+    gbs = bytes_per_launch / (t_ms * 1e-3) / 1e9
+    return {"kernel": name, "avg_launch_us": round(t_ms * 1e3, 2),
+            "algorithmic_bytes_per_launch": bytes_per_launch, "achieved_GBs": round(gbs, 1),
+            "frac": round(gbs / HBM_PEAK_GBS, 4)}
+
+
+def smoother_lines(ctx, ws, reps, coef, n):
+    """(the finest level's kernel in a solve, its half-sweep): the same line twice
+    where it is smoothed in half-sweeps."""
+    names = (("fused64_kernel (FP64 finest level, mean of its two passes)",
+              "march64_kernel<0> (FP64 colour-split half-sweep)") if coef == "fp64" else
+             (f"fused_kernel<{coef}> (finest level, mean of its two passes)",
+              f"colour_split4_kernel<{coef}> (finest level, one colour)"))
+    half = kernel_line(names[1], time_smoother(ctx, ws, reps), HALF_SWEEP_BYTES[coef] * n)
+    t = time_passes(ctx, ws, reps)
+    return (kernel_line(names[0], t, PASS_BYTES[coef] * n) if t is not None else half), half
+
+
 def sweep_only(args):
     """One hierarchy (FP64 or mixed) on the workload's K, then --smoother-reps
-    timed red-black iterations of its finest level: the only launches of the
-    dominant half-sweep kernel in the run, for kernel traces and counters."""
+    timed red-black iterations and fused passes of its finest level: the only
+    launches of the smoothing kernels in the run, for kernel traces and counters."""
     import torch
 
     from macroflow3d_amd import multigrid as mg
@@ -286,26 +347,13 @@ def sweep_only(args):
     del ca, cb
     ws = ph.FlowWorkspace()
     mg.mg_setup(ctx, ws, g, BCSpec.darcy_x(), cfg, K)
-    t = time_smoother(ctx, ws, args.smoother_reps)
-    ws.close()
     N = g.num_cells()
-    bpc = 20.0 if args.sweep_only == "fp64" else 12.0
-    gbs = bpc * N / (t * 1e-3) / 1e9
-    print(json.dumps({"sweep": args.sweep_only, "cells": N, "avg_launch_us": round(t * 1e3, 2),
-                      "algorithmic_bytes_per_launch": bpc * N, "achieved_GBs": round(gbs, 1),
-                      "frac": round(gbs / HBM_PEAK_GBS, 4)}), flush=True)
+    used, half = smoother_lines(ctx, ws, args.smoother_reps,
+                                "fp64" if args.sweep_only == "fp64" else "bf16", N)
+    ws.close()
+    print(json.dumps({"sweep": args.sweep_only, "cells": N, "in_solve": used,
+                      "half_sweep": half}), flush=True)
     return 0
-
-
-def fp64_smoother_line(t_ms, n):
-    """The FP64 V-cycle's finest half-sweep (colour-split, faces from
-    h = 1/(2K)): 20 B/cell algorithmic (h 8, other-colour x 4, own b 4, own x
-    out 4)."""
-    alg = 20.0 * n
-    gbs = alg / (t_ms * 1e-3) / 1e9
-    return {"kernel": "march64_kernel<0> (FP64 colour-split half-sweep)",
-            "avg_launch_us": round(t_ms * 1e3, 2), "algorithmic_bytes_per_launch": alg,
-            "achieved_GBs": round(gbs, 1), "frac": round(gbs / HBM_PEAK_GBS, 4)}
 
 
 def main():
@@ -391,11 +439,12 @@ def main():
         r64, ms64 = timed(cfg64, args.fp64_steps, 1, h64, v64, ws64)
     else:
         r64, ms64 = step(cfg64, h64, v64, ws64, False), float("nan")
-    t64 = time_smoother(ctx, ws64, args.smoother_reps)
+    fp64_smoother, fp64_half = smoother_lines(ctx, ws64, args.smoother_reps, "fp64", N)
     ws64.close()
     log(args, f"fp64: {r64.num_iterations} iterations, rel true residual "
-              f"{r64.true_residual / r64.bnorm:.3e}, {ms64:.2f} ms per solve; half-sweep "
-              f"{t64 * 1e3:.1f} us")
+              f"{r64.true_residual / r64.bnorm:.3e}, {ms64:.2f} ms per solve; finest level "
+              f"{fp64_smoother['avg_launch_us']} us a launch, half-sweep "
+              f"{fp64_half['avg_launch_us']} us")
 
     # mixed precision from the linear head
     ws = ph.FlowWorkspace()
@@ -438,23 +487,14 @@ def main():
               f"mean |curl| {diagnostics['vorticity_mag_mean']:.4e}")
     del pv, diag
 
-    # dominant kernel: finest-level colour sweep of the headline V-cycle,
-    # timed in place on the workspace's own level-0 buffers
-    mg.smooth_level(ctx, ws, 0, 1)
-    e0 = torch.cuda.Event(enable_timing=True)
-    e1 = torch.cuda.Event(enable_timing=True)
-    e0.record(ctx.stream)
-    mg.smooth_level(ctx, ws, 0, args.smoother_reps)
-    e1.record(ctx.stream)
-    e1.synchronize()
-    t_launch_ms = e0.elapsed_time(e1) / (2 * args.smoother_reps)
-    # one colour (half-sweep) of the mixed V-cycle: 3 faces x 2 B + opposite-
-    # colour x 2 B + own-colour x write 2 B + own-colour b 2 B per cell
-    alg_bytes = {"bf16": 12.0, "fp16": 12.0, "fp32": 18.0}[args.coef] * N
-    achieved = alg_bytes / (t_launch_ms * 1e-3) / 1e9
-    log(args, f"smoother: {t_launch_ms * 1e3:.1f} us per colour sweep, {achieved:.0f} GB/s "
-              f"algorithmic")
-    traffic = committed_traffic(n, args.coef)
+    # dominant kernel: the headline V-cycle's smoothing of the finest level,
+    # timed on the workspace's own level-0 buffers
+    used, half = smoother_lines(ctx, ws, args.smoother_reps, args.coef, N)
+    fused = used is not half
+    log(args, f"smoother: {used['kernel']} {used['avg_launch_us']} us, {used['achieved_GBs']} GB/s "
+              f"algorithmic; half-sweep {half['avg_launch_us']} us, {half['achieved_GBs']} GB/s")
+    traffic = committed_traffic(n, args.coef, "fused" if fused else "half_sweep")
+    half["traffic"] = committed_traffic(n, args.coef, "half_sweep")
 
     out = {
         "metric": METRIC,
@@ -492,18 +532,21 @@ def main():
         "head_rel_l2_vs_fp64": head_err,
         "velocity_rel_l2_vs_fp64": vel_err,
         "velocity_diagnostics": diagnostics,
-        "fp64_smoother": fp64_smoother_line(t64, N),
+        "fp64_smoother": fp64_smoother,
+        "fp64_half_sweep": fp64_half,
         "roofline": {
-            "kernel": f"colour_split4_kernel<{args.coef}> (finest level, one colour)",
-            "bound": "hbm",
-            "achieved": round(achieved, 1),
+            "kernel": used["kernel"],
+            # (a pass moves about a quarter of the bytes of the half-sweeps it holds)
+            "bound": "vector instructions" if fused else "hbm",
+            "achieved": used["achieved_GBs"],
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4),
+            "frac": used["frac"],
             "traffic": traffic,
-            "algorithmic_bytes_per_launch": alg_bytes,
-            "avg_launch_us": round(t_launch_ms * 1e3, 2),
+            "algorithmic_bytes_per_launch": used["algorithmic_bytes_per_launch"],
+            "avg_launch_us": used["avg_launch_us"],
         },
+        "half_sweep": half,
     }
     ws.close()
     if not args.no_cpu:
@@ -568,16 +611,12 @@ def bench_512(args, ctx, coef):
             ph.compute_velocity_from_head(v, h, K, g, bc, ctx)
         torch.cuda.synchronize()
         ms = (time.perf_counter() - t) * 1e3 / reps
-        ts = time_smoother(ctx, ws, args.smoother_reps)
-        if name == "fp64":
-            out["fp64_smoother_512"] = fp64_smoother_line(ts, g.num_cells())
-        else:  # 12 B/cell: BF16 faces 6, other-colour x 2, own b 2, own x out 2
-            gbs = 12.0 * g.num_cells() / (ts * 1e-3) / 1e9
-            out["smoother_512"] = {"kernel": "colour_split4_kernel<bf16> (finest level, one colour)",
-                                   "avg_launch_us": round(ts * 1e3, 2),
-                                   "achieved_GBs": round(gbs, 1),
-                                   "frac": round(gbs / HBM_PEAK_GBS, 4)}
-        log(args, f"512^3 {name} half-sweep {ts * 1e3:.1f} us")
+        used, half = smoother_lines(ctx, ws, args.smoother_reps,
+                                    "fp64" if name == "fp64" else args.coef, g.num_cells())
+        pre = "fp64_" if name == "fp64" else ""
+        out[pre + "smoother_512"], out[pre + "half_sweep_512"] = used, half
+        log(args, f"512^3 {name} finest level: {used['avg_launch_us']} us a launch, half-sweep "
+                  f"{half['avg_launch_us']} us")
         ws.close()
         out[f"{name}_ms_512"] = round(ms, 3)
         out[f"{name}_iterations_512"] = res.num_iterations

@@ -281,6 +281,12 @@ int mf3d_workspace_solve_counts(const mf3d_workspace* ws, long* op_applications,
  * set 0 to test there). */
 int mf3d_mg_smooth(mf3d_workspace* ws, mf3d_stream stream, int level, int num_iters);
 
+/* Extension: the two fused passes of one V-cycle on level `level` (pre-smoothing with
+ * the restriction, prolongation with post-smoothing), reps times, on the
+ * workspace's own buffers: what solves on this hierarchy launch there, for timing. A
+ * level that is not smoothed in fused passes: MF3D_ERR_UNSUPPORTED. */
+int mf3d_mg_passes(mf3d_workspace* ws, mf3d_stream stream, int level, int reps);
+
 /* Number of levels of the current hierarchy (0 before set-up). */
 int mf3d_mg_num_levels(const mf3d_workspace* ws);
 

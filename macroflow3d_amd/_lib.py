@@ -90,6 +90,7 @@ SIGNATURES = {
     "mf3d_workspace_solve_counts": (_i, [_vp, _vp, _vp]),
     "mf3d_workspace_reserve": (_i, [_vp, _g, _i]),
     "mf3d_mg_smooth": (_i, [_vp, _vp, _i, _i]),
+    "mf3d_mg_passes": (_i, [_vp, _vp, _i, _i]),
     "mf3d_mg_precondition": (_i, [_vp, _vp, _vp, _vp, _sz]),
     "mf3d_varcoeff_apply": (_i, [_vp, _g, _b, _i, _vp, _vp, _vp, _sz]),
     "mf3d_dot": (_i, [_vp, _vp, _vp, _vp, _sz, _vp]),

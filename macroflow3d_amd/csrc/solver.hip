@@ -2315,6 +2315,39 @@ int mf3d_mg_smooth(mf3d_workspace* ws, mf3d_stream stream, int level, int num_it
                               (const double*)nullptr, L.plan);
 }
 
+int mf3d_mg_passes(mf3d_workspace* ws, mf3d_stream stream, int level, int reps) {
+    MF3D_CHECK_PTR(ws);
+    if (!ws->ready || !ws->K0)
+        return fail(MF3D_ERR_INVALID_ARGUMENT, "mf3d_mg_setup has not been called");
+    if (level < 0 || level >= (int)ws->lv.size())
+        return fail(MF3D_ERR_INVALID_ARGUMENT, "level out of range");
+    if (reps < 0) return fail(MF3D_ERR_INVALID_ARGUMENT, "reps < 0");
+    Level& L = ws->lv[level];
+    if (!L.fused && !L.fused64)
+        return fail(MF3D_ERR_UNSUPPORTED, "the level is not smoothed in fused passes");
+    clear_stale_error();
+    hipStream_t s = as_stream(stream);
+    Level& C = ws->lv[level + 1];
+    const double dx2 = L.g.dx * L.g.dx, bs = L.cs * dx2;
+    for (int q = 0; q < reps; ++q) {
+        if (L.fused) {
+            MF3D_TRY(kern::fused32_pre(s, L.g, ws->bct, ws->pin, bs, 1.0 / bs, L.xb, L.b32,
+                                       L.flo.type, L.rec, C.b32, C.fused));
+            MF3D_TRY(kern::fused32_post(s, L.g, ws->bct, ws->pin, bs, L.xb, L.x32, L.b32,
+                                        L.flo.type, L.rec, C.x32));
+            continue;
+        }
+        kern::BlockPass<double> p{};
+        p.iters = 2, p.bs = dx2, p.rs = 1.0 / dx2, p.b = L.b, p.corder = C.order64;
+        p.xout = L.x2, p.bcoarse = C.b;
+        MF3D_TRY(kern::fused64_pass(s, L.g, ws->bct, ws->pin, L.hs, p));
+        p.xin = L.x2, p.xout = L.x, p.bcoarse = nullptr, p.xc = C.x;
+        if (level == 0) p.z = ws->z, p.partials = ws->partials;
+        MF3D_TRY(kern::fused64_pass(s, L.g, ws->bct, ws->pin, L.hs, p));
+    }
+    return MF3D_OK;
+}
+
 int mf3d_mg_num_levels(const mf3d_workspace* ws) {
     return ws && ws->ready ? (int)ws->lv.size() : 0;
 }

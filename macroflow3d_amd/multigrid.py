@@ -105,3 +105,9 @@ def smooth_level(ctx: HipContext, workspace, level: int, num_iters: int) -> None
     """num_iters GSRB iterations on one level of the workspace's hierarchy, in
     place on that level's own buffers (timing and in-situ tests)."""
     _lib.call("mf3d_mg_smooth", workspace.handle, ctx.handle, int(level), int(num_iters))
+
+
+def level_passes(ctx: HipContext, workspace, level: int, reps: int) -> None:
+    """The fused passes of reps V-cycles on one level, on the workspace's own
+    buffers (timing); raises if the level is not smoothed in fused passes."""
+    _lib.call("mf3d_mg_passes", workspace.handle, ctx.handle, int(level), int(reps))

@@ -144,3 +144,21 @@ show(solve(*args, -1, {head}))
     assert off[1] < on[1] <= 1.15 * off[1]
     assert tight[1] == off[1] and passes(tight[2]) == 0
     assert off[1] <= some[1] <= (off[1] + on[1]) // 2
+
+
+@pytest.mark.parametrize("mixed,level,kernels", [
+    (True, 0, ["fused_kernel", "fused_kernel"]), (True, 1, None),
+    (False, 0, ["fused64_kernel", "fused64_kernel"]), (False, 4, None)])
+def test_fused_passes_of_one_level(mixed, level, kernels):
+    """mf3d_mg_passes launches what a V-cycle launches on that level, or refuses."""
+    code = VCYCLE.replace("    lib.mf3d_workspace_destroy(ws)", f"""    vc = stub.log()
+    stub.clear()
+    show([lib.mf3d_mg_passes(ws, None, {level}, 1), stub.log(), vc])
+    lib.mf3d_workspace_destroy(ws)""")
+    (st, log, vc), = host_runs.run(code + f"vcycle((256, 256, 256), 5, {mixed})")
+    if kernels is None:
+        assert st == 7 and log == []  # MF3D_ERR_UNSUPPORTED
+        return
+    assert st == 0 and len(log) == 2 and all(k in n for k, n in zip(kernels, log))
+    # (without PCG's partial sums the FP64 result stays in natural order too)
+    assert log[0] in vc and log[1] in vc
