@@ -7,8 +7,11 @@ The code sees ``stub`` (limit, in_use, fail, log, clear), ``lib`` (the C ABI), `
 ``run`` returns."""
 from __future__ import annotations
 
+import atexit
+import functools
 import json
 import os
+import shutil
 import subprocess
 import sys
 import tempfile
@@ -34,14 +37,21 @@ def show(value): print("=" + json.dumps(value), flush=True)
 """
 
 
-def run(code: str, lib_root: str = ROOT) -> list:
+@functools.lru_cache(maxsize=1)
+def _stub() -> str:
+    """The stub library, built once a process."""
+    tmp = tempfile.mkdtemp()
+    atexit.register(shutil.rmtree, tmp, ignore_errors=True)
+    so = os.path.join(tmp, "hip_stub.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC",
+                    os.path.join(HERE, "cpp", "hip_stub.cpp"), "-o", so], check=True)
+    return so
+
+
+def run(code: str) -> list:
     """The values that ``code`` showed, in order; raises if it failed."""
-    with tempfile.TemporaryDirectory() as tmp:
-        so = os.path.join(tmp, "hip_stub.so")
-        subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC",
-                        os.path.join(HERE, "cpp", "hip_stub.cpp"), "-o", so], check=True)
-        r = subprocess.run([sys.executable, "-c", PRELUDE + code, so], cwd=lib_root,
-                           capture_output=True, text=True, timeout=120)
+    r = subprocess.run([sys.executable, "-c", PRELUDE + code, _stub()], cwd=ROOT,
+                       capture_output=True, text=True, timeout=120)
     if r.returncode != 0:
         raise RuntimeError(f"exit {r.returncode}\n{r.stdout}\n{r.stderr}")
     return [json.loads(line[1:]) for line in r.stdout.splitlines() if line.startswith("=")]
